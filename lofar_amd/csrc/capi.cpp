@@ -378,21 +378,25 @@ int take(DeviceCtx& c, Arena* ar, Buffer& b, size_t bytes, char** out)
     return LOFAR_OK;
 }
 
-// exp(+2*pi*i*m/N), m < N, from long double arithmetic, rounded once
-int twiddles(DeviceCtx& c, int n, int precision, void** out)
+// exp(+2*pi*i*m/N), m < N, from long double arithmetic, rounded once; mixed: in the order
+// of the mixed-radix transforms' stages
+int twiddles(DeviceCtx& c, int n, int precision, void** out, bool mixed = false)
 {
-    const long long key = (long long)n * 4 + precision;
+    const long long key = (long long)n * 4 + (mixed ? 2 : 0) + precision;
     auto it = c.twiddles.find(key);
     if (it != c.twiddles.end()) {
         *out = it->second;
         return LOFAR_OK;
     }
     std::vector<double> tw(2 * (size_t)n);
+    std::vector<int> order(n);
+    for (int i = 0; i < n; i++) order[i] = i;
+    if (mixed && !mixed_twiddle_order(n, order.data())) return fail(LOFAR_ESIZE);
     const long double two_pi = 6.283185307179586476925286766559005768L;
-    for (int m = 0; m < n; m++) {
-        const long double a = two_pi * (long double)m / (long double)n;
-        tw[2 * m] = (double)cosl(a);
-        tw[2 * m + 1] = (double)sinl(a);
+    for (int i = 0; i < n; i++) {
+        const long double a = two_pi * (long double)order[i] / (long double)n;
+        tw[2 * i] = (double)cosl(a);
+        tw[2 * i + 1] = (double)sinl(a);
     }
     void* d = nullptr;
     size_t bytes = (size_t)n * (precision == LOFAR_FP64 ? 16 : 8);
@@ -411,14 +415,15 @@ int twiddles(DeviceCtx& c, int n, int precision, void** out)
 
 // Twiddles of the allocation-free entry point: a slice of the static workspace
 // filled on the device (no allocation and no host copy).
-int twiddles_for(DeviceCtx& c, Arena* ar, int n, int precision, hipStream_t st, void** out)
+int twiddles_for(DeviceCtx& c, Arena* ar, int n, int precision, hipStream_t st, void** out,
+                 bool mixed = false)
 {
-    if (!ar || !ar->base) return twiddles(c, n, precision, out);
+    if (!ar || !ar->base) return twiddles(c, n, precision, out, mixed);
     Buffer unused;
     char* p = nullptr;
     int r = take(c, ar, unused, (size_t)n * (precision == LOFAR_FP64 ? 16 : 8), &p);
     if (r) return r;
-    HIPCHK(fill_twiddles(precision, n, p, st));
+    HIPCHK(mixed ? fill_mixed_twiddles(precision, n, p, st) : fill_twiddles(precision, n, p, st));
     *out = p;
     return LOFAR_OK;
 }
@@ -465,9 +470,9 @@ int fft_generic_planes(DeviceCtx& c, Arena* ar, int precision, int sign, const v
                        bool rows_first = false)
 {
     void *twx, *twy;
-    int r = twiddles_for(c, ar, nx, precision, st, &twx);
+    int r = twiddles_for(c, ar, nx, precision, st, &twx, true);
     if (r) return r;
-    r = twiddles_for(c, ar, ny, precision, st, &twy);
+    r = twiddles_for(c, ar, ny, precision, st, &twy, true);
     if (r) return r;
     auto cols = [&](const void* src) {
         return precision == LOFAR_FP64

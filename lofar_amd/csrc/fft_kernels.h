@@ -482,9 +482,12 @@ PhaseParams phase_params(int nw, int xtot, int ytot, double resolution, double w
 hipError_t fill_twiddles(int precision, int n, void* tw, hipStream_t st);
 
 // Mixed-radix line transforms for sides that are not powers of two (prime factors at most
-// 13, side at most 8192): line l of `lines` starts at (l / per) * plane + (l % per) *
-// lstride, its elements estride apart; out may alias in.  fft_size_ok: a side either the
-// power-of-two kernels or these take.
+// 13, side at most 8192; fft_mixed.hip): line l of `lines` starts at (l / per) * plane + (l %
+// per) * lstride, its elements estride apart (1: rows); out may alias in.  tw: the length's
+// table in the order of mixed_twiddle_order (n entries), or filled by fill_mixed_twiddles.
+// fft_size_ok: a side either the power-of-two kernels or these take.
+bool mixed_twiddle_order(int n, int* order);
+hipError_t fill_mixed_twiddles(int precision, int n, void* tw, hipStream_t st);
 bool fft_size_ok(int n);
 template <typename Real>
 hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int n, long long lines,
