@@ -31,14 +31,16 @@
 
 namespace lofar {
 
-constexpr int kScanBlock = 4096;  // elements per block of the local scan (256 threads x 16)
 constexpr int kMaxFine = 256;     // sst <= 16
 constexpr int kUnroll = 4;        // samples or records per thread per round
 
-__global__ __launch_bounds__(256) void k_fill_u32(unsigned* p, long long n, unsigned v)
+// n words of p and m words of q
+__global__ __launch_bounds__(256) void k_fill_u32(unsigned* p, long long n, unsigned* q,
+                                                  long long m, unsigned v)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+    else if (i - n < m) q[i - n] = v;
 }
 
 // Tiles [tu_a, tu_b] x [tv_a, tv_b] of a non-empty window.
@@ -116,72 +118,90 @@ __global__ __launch_bounds__(256) void k_l1_count(int mode, long long n, const d
 }
 
 // ---------------------------------------------------------------------------
-// exclusive scan (counts -> offsets; the total to two places)
+// scans over the super-tiles
 
-__global__ __launch_bounds__(256) void k_scan_local(const unsigned* in, long long* out,
-                                                    long long* partials, long long n)
+// Exclusive scan of one value per thread over the workgroup; the sum to total.
+// Ends with every wave past the barrier that publishes the wave sums.
+template <int NT, typename T>
+__device__ __forceinline__ T block_exscan(T v, T* wsum, T& total)
 {
-    __shared__ long long sh[256];
-    const int tid = threadIdx.x;
-    const long long base = (long long)blockIdx.x * kScanBlock + tid * 16;
-    long long v[16];
-    long long sum = 0;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    T x = v;
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        v[e] = (base + e < n) ? (long long)in[base + e] : 0;
-        sum += v[e];
+    for (int d = 1; d < 64; d <<= 1) {
+        const T y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
     }
-    sh[tid] = sum;
+    if (lane == 63) wsum[wid] = x;
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        const long long x = tid >= off ? sh[tid - off] : 0;
-        __syncthreads();
-        sh[tid] += x;
-        __syncthreads();
+    T pre = 0, tot = 0;
+#pragma unroll NT <= 512 ? NT / 64 : 1
+    for (int w = 0; w < NT / 64; w++) {
+        const T s = wsum[w];
+        pre += w < wid ? s : (T)0;
+        tot += s;
     }
-    long long run = sh[tid] - sum;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-        if (base + e < n) out[base + e] = run;
-        run += v[e];
-    }
-    if (tid == 255) partials[blockIdx.x] = sh[255];
+    total = tot;
+    return pre + x - v;
 }
 
-// single workgroup: exclusive scan of the block partials; writes the grand total
-__global__ __launch_bounds__(1024) void k_scan_partials(long long* partials, long long nblk,
-                                                        long long* total_a, long long* total_b)
+// One workgroup: record, entry and level-2 block offsets of every super-tile, the block
+// table, and the call's status (entry total, validation flag, then seq, which the host waits
+// for) straight into host memory.  Nine scan launches and a copy took 45 us of a small
+// image's 220; this takes about 5 up to 8192 super-tiles.
+__global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned* count1,
+                                                  const unsigned* count1e, long long* off1,
+                                                  long long* eoff1, long long bs, long long* boff,
+                                                  L2Block* blk, const int* err,
+                                                  volatile long long* status, long long seq)
 {
-    __shared__ long long sh[1024];
-    const int tid = threadIdx.x;
-    long long carry = 0;
-    for (long long c0 = 0; c0 < nblk; c0 += 1024) {
-        const long long idx = c0 + tid;
-        const long long x = idx < nblk ? partials[idx] : 0;
-        sh[tid] = x;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            const long long y = tid >= off ? sh[tid - off] : 0;
-            __syncthreads();
-            sh[tid] += y;
-            __syncthreads();
+    __shared__ long long ws[3][1024 / 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    long long crec = 0, cent = 0, cblk = 0;
+    for (long long c0 = 0; c0 < nk1; c0 += 1024) {
+        const long long k = c0 + tid;
+        const long long r = k < nk1 ? (long long)count1[k] : 0;
+        const long long e = k < nk1 ? (long long)count1e[k] : 0;
+        const long long nb = (r + bs - 1) / bs;
+        long long tr, te, tb;
+        const long long rec = crec + block_exscan<1024>(r, ws[0], tr);
+        const long long ent = cent + block_exscan<1024>(e, ws[1], te);
+        const long long b0 = cblk + block_exscan<1024>(nb, ws[2], tb);
+        if (k < nk1) {
+            off1[k] = rec;
+            eoff1[k] = ent;
         }
-        if (idx < nblk) partials[idx] = carry + sh[tid] - x;
-        const long long chunk = sh[1023];
-        __syncthreads();
-        carry += chunk;
+        if (boff) {
+            if (k < nk1) boff[k] = b0;
+            // block descriptors: the wave writes each of its lanes' segments together
+            for (unsigned long long m = __ballot(nb > 0); m; m &= m - 1) {
+                const int src = __ffsll(m) - 1;
+                const long long sk = __shfl(k, src), sr = __shfl(rec, src), sn = __shfl(r, src);
+                const long long sb = __shfl(b0, src), snb = __shfl(nb, src);
+                for (long long j = lane; j < snb; j += 64) {
+                    L2Block d;
+                    d.k1 = sk;
+                    d.beg = sr + j * bs;
+                    d.end = sr + min(sn, (j + 1) * bs);
+                    d.pad = 0;
+                    blk[sb + j] = d;
+                }
+            }
+        }
+        crec += tr;
+        cent += te;
+        cblk += tb;
+        __syncthreads();  // the wave sums are read: free for the next round
     }
     if (tid == 0) {
-        *total_a = carry;
-        *total_b = carry;
+        off1[nk1] = crec;
+        eoff1[nk1] = cent;
+        if (boff) boff[nk1] = cblk;
+        status[0] = cent;
+        status[1] = *err;
+        __threadfence_system();
+        status[2] = seq;
     }
-}
-
-__global__ __launch_bounds__(256) void k_scan_add(long long* out, const long long* partials,
-                                                  long long n)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += partials[i / kScanBlock];
 }
 
 // ---------------------------------------------------------------------------
@@ -285,31 +305,6 @@ struct L1Stage {
     static constexpr int U = 4;
     static_assert(CAP * (sizeof(Rec) + 2) + kStageMaxBins * 16 + 64 <= 81920, "LDS");
 };
-
-// Exclusive scan of one value per thread over the workgroup; the sum to total.
-// Ends with every wave past the barrier that publishes the wave sums.
-template <int NT>
-__device__ __forceinline__ unsigned block_exscan(unsigned v, unsigned* wsum, unsigned& total)
-{
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    unsigned x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const unsigned y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-    }
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    unsigned pre = 0u, tot = 0u;
-#pragma unroll
-    for (int w = 0; w < NT / 64; w++) {
-        const unsigned s = wsum[w];
-        pre += w < wid ? s : 0u;
-        tot += s;
-    }
-    total = tot;
-    return pre + x - v;
-}
 
 // Per-round bin bookkeeping of a staged scatter.  gnext (thread tid's register, bin
 // tid): global slot of the bin's next record.  After open(): dst[k] + p is the
@@ -564,33 +559,6 @@ __device__ __forceinline__ bool record_tiles(const Rec& r, const Geometry& g, co
     }
 }
 
-// blocks per segment
-__global__ __launch_bounds__(256) void k_l2_nblocks(long long nk1, const long long* off1,
-                                                    long long bs, unsigned* nblk)
-{
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nk1) nblk[k] = (unsigned)((off1[k + 1] - off1[k] + bs - 1) / bs);
-}
-
-// block descriptors: segment, first record, end record
-__global__ __launch_bounds__(256) void k_l2_blocks(long long nk1, const long long* off1,
-                                                   long long bs, const long long* boff,
-                                                   L2Block* blk)
-{
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nk1) return;
-    const long long beg = off1[k], end = off1[k + 1];
-    long long j = boff[k];
-    for (long long r = beg; r < end; r += bs, j++) {
-        L2Block d;
-        d.k1 = k;
-        d.beg = r;
-        d.end = min(end, r + bs);
-        d.pad = 0;
-        blk[j] = d;
-    }
-}
-
 template <int OUT, typename Rec>
 __global__ __launch_bounds__(256) void k_l2_count(Geometry g, TileMap tm, const long long* nblocks,
                                                   const L2Block* blk, const Rec* rec,
@@ -624,43 +592,43 @@ __global__ __launch_bounds__(256) void k_l2_count(Geometry g, TileMap tm, const 
     for (int f = tid; f < nf; f += 256) cnt2[b * nf + f] = cnt[f];
 }
 
-// one workgroup per segment: per fine tile, running sums over the segment's
+// one workgroup per segment, one fine tile per thread: running sums over the segment's
 // blocks (replacing the counts by block bases relative to the segment's first
-// entry), then the exclusive scan over fine tiles gives the bucket offsets
-__global__ __launch_bounds__(256) void k_l2_scan(TileMap tm, const long long* eoff1,
-                                                 const long long* boff, unsigned* cnt2,
-                                                 long long* offsets)
+// entry), then the exclusive scan over fine tiles gives the bucket offsets.  The blocks'
+// counts are read 8 at a time: they come back to back instead of one latency each.
+__global__ __launch_bounds__(kMaxFine) void k_l2_scan(TileMap tm, const long long* eoff1,
+                                                      const long long* boff, unsigned* cnt2,
+                                                      long long* offsets)
 {
-    __shared__ unsigned tot[kMaxFine];
-    const int tid = threadIdx.x;
+    __shared__ unsigned ws[kMaxFine / 64];
+    constexpr int G = 8;
+    const int f = threadIdx.x;
     const int nf = tm.sst * tm.sst;
     const long long k1 = blockIdx.x;
     const long long b0 = boff[k1], b1 = boff[k1 + 1];
-    for (int f = tid; f < nf; f += 256) {
-        unsigned run = 0;
-        for (long long j = b0; j < b1; j++) {
-            const unsigned c = cnt2[j * nf + f];
-            cnt2[j * nf + f] = run;
-            run += c;
+    const bool on = f < nf;
+    unsigned tot = 0;
+    for (long long j = b0; j < b1; j += G) {
+        unsigned c[G];
+#pragma unroll
+        for (int i = 0; i < G; i++) c[i] = on && j + i < b1 ? cnt2[(j + i) * nf + f] : 0u;
+#pragma unroll
+        for (int i = 0; i < G; i++) tot += c[i];
+    }
+    unsigned all;
+    unsigned run = block_exscan<kMaxFine>(tot, ws, all);
+    if (on) offsets[k1 * nf + f] = eoff1[k1] + run;
+    for (long long j = b0; j < b1; j += G) {
+        unsigned c[G];
+#pragma unroll
+        for (int i = 0; i < G; i++) c[i] = on && j + i < b1 ? cnt2[(j + i) * nf + f] : 0u;
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            if (on && j + i < b1) cnt2[(j + i) * nf + f] = run;
+            run += c[i];
         }
-        tot[f] = run;
     }
-    __syncthreads();
-    if (tid == 0) {
-        unsigned run = 0;
-        for (int f = 0; f < nf; f++) {
-            const unsigned c = tot[f];
-            tot[f] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    const long long beg = eoff1[k1];
-    for (int f = tid; f < nf; f += 256) {
-        offsets[k1 * nf + f] = beg + tot[f];
-        for (long long j = b0; j < b1; j++) cnt2[j * nf + f] += tot[f];
-    }
-    if (k1 == 0 && tid == 0) offsets[tm.nk1 * nf] = eoff1[tm.nk1];
+    if (k1 == 0 && f == 0) offsets[tm.nk1 * nf] = eoff1[tm.nk1];
 }
 
 // The entry of record x (window s) for fine tile (fv, fu) of super-tile (sv, su).
@@ -799,30 +767,20 @@ __global__ __launch_bounds__(kStageThreads) void k_l2_scatter_staged(
 
 static inline unsigned blocks_for(long long n, int t) { return (unsigned)((n + t - 1) / t); }
 
-static void scan(const unsigned* in, long long* out, long long n, long long* partials,
-                 long long* total_b, hipStream_t st)
-{
-    const long long nblk = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nblk), dim3(256), 0, st, in, out, partials, n);
-    hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(1024), 0, st, partials, nblk, out + n,
-                       total_b);
-    hipLaunchKernelGGL(k_scan_add, dim3(blocks_for(n, 256)), dim3(256), 0, st, out, partials, n);
-}
-
 hipError_t fill_u32(unsigned* p, long long n, unsigned v, hipStream_t st)
 {
-    if (n > 0) hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n, 256)), dim3(256), 0, st, p, n, v);
+    if (n > 0)
+        hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n, 256)), dim3(256), 0, st, p, n,
+                           (unsigned*)nullptr, 0LL, v);
     return hipGetLastError();
 }
 
 hipError_t bucket_count(int mode, long long n, const double* uu, const double* vv, const double* ww,
-                        const Geometry& g, const Buckets& b, hipStream_t st)
+                        const Geometry& g, const Buckets& b, unsigned* zero2, long long nzero2,
+                        hipStream_t st)
 {
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(b.map.nk1, 256)), dim3(256), 0, st, b.count1,
-                       b.map.nk1, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(b.map.nk1, 256)), dim3(256), 0, st, b.count1e,
-                       b.map.nk1, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, (unsigned*)b.err, 1LL, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(b.nzero + nzero2, 256)), dim3(256), 0, st,
+                       (unsigned*)b.zero, b.nzero, zero2, nzero2, 0u);
     if (n > 0 && b.global_l1)
         hipLaunchKernelGGL(k_l1_count<true>, dim3((unsigned)b.nwg), dim3(256), 0, st, mode, n, uu,
                            vv, ww, g, b.map, b.chunk, b.count1, b.count1e, b.base1, b.err);
@@ -833,10 +791,10 @@ hipError_t bucket_count(int mode, long long n, const double* uu, const double* v
     return hipGetLastError();
 }
 
-hipError_t bucket_scan(const Buckets& b, hipStream_t st)
+hipError_t bucket_scan(const Buckets& b, long long seq, hipStream_t st)
 {
-    scan(b.count1, b.off1, b.map.nk1, b.partials, b.total_rec, st);
-    scan(b.count1e, b.eoff1, b.map.nk1, b.partials, b.total, st);
+    hipLaunchKernelGGL(k_l1_scan, dim3(1), dim3(1024), 0, st, b.map.nk1, b.count1, b.count1e,
+                       b.off1, b.eoff1, b.l2_block, b.l2_boff, b.l2_blk, b.err, b.status, seq);
     return hipGetLastError();
 }
 
@@ -845,16 +803,11 @@ static hipError_t level2(const Geometry& g, const Buckets& b, const Rec* rec, Ou
                          hipStream_t st)
 {
     const long long nk1 = b.map.nk1;
-    hipLaunchKernelGGL(k_l2_nblocks, dim3(blocks_for(nk1, 256)), dim3(256), 0, st, nk1, b.off1,
-                       b.l2_block, b.l2_nblk);
-    scan(b.l2_nblk, b.l2_boff, nk1, b.partials, b.l2_boff + nk1, st);
-    hipLaunchKernelGGL(k_l2_blocks, dim3(blocks_for(nk1, 256)), dim3(256), 0, st, nk1, b.off1,
-                       b.l2_block, b.l2_boff, b.l2_blk);
     const unsigned grid = (unsigned)b.l2_max_blocks;
     const long long* nblocks = b.l2_boff + nk1;
     hipLaunchKernelGGL((k_l2_count<OUT, Rec>), dim3(grid), dim3(256), 0, st, g, b.map, nblocks,
                        b.l2_blk, rec, b.l2_cnt);
-    hipLaunchKernelGGL(k_l2_scan, dim3((unsigned)nk1), dim3(256), 0, st, b.map, b.eoff1, b.l2_boff,
+    hipLaunchKernelGGL(k_l2_scan, dim3((unsigned)nk1), dim3(kMaxFine), 0, st, b.map, b.eoff1, b.l2_boff,
                        b.l2_cnt, b.offsets);
     if (b.stage & kStageL2)
         hipLaunchKernelGGL((k_l2_scatter_staged<OUT, Rec, Out>), dim3(grid), dim3(kStageThreads),

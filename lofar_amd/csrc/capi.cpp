@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <condition_variable>
 #include <cstdlib>
@@ -166,7 +167,8 @@ struct DeviceCtx {
     char* stage_buf[kStage] = {};
     hipEvent_t stage_done[kStage] = {};
     Buffer occ;                     // per-tile occupancy of the fused imaging path
-    long long* status_host = nullptr;  // pinned: [total, err]
+    volatile long long* status_host = nullptr;  // pinned: [total, err, call number]
+    long long status_seq = 0;       // call number of the last bucket count
     char* scratch = nullptr;        // this device's copy of `scratch` (allocation-free calls)
     hipError_t scratch_err = hipSuccess;
     std::map<long long, void*> twiddles;
@@ -221,9 +223,10 @@ int get_ctx(DeviceCtx** out)
             return LOFAR_EHIP;
         if (hipEventCreateWithFlags(&c.last_done, hipEventDisableTiming) != hipSuccess)
             return LOFAR_EHIP;
-        if (hipHostMalloc((void**)&c.status_host, 2 * sizeof(long long), hipHostMallocDefault) !=
+        if (hipHostMalloc((void**)&c.status_host, 4 * sizeof(long long), hipHostMallocDefault) !=
             hipSuccess)
             return LOFAR_EHIP;
+        for (int i = 0; i < 4; i++) c.status_host[i] = 0;
         // this device's copy of the allocation-free workspace (device `dev` is current)
         void* sp = nullptr;
         c.scratch_err = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch));
@@ -534,6 +537,7 @@ struct BucketCfg {
     int sst;
     long long chunk, block;
     int stage;
+    bool forced;
 };
 
 BucketCfg bucket_cfg()
@@ -543,11 +547,12 @@ BucketCfg bucket_cfg()
         if (const char* e = getenv("LOFAR_BUCKET_STAGE")) stage = atoi(e) & (kStageL1 | kStageL2);
         int a = (stage & kStageL1) ? 16 : 8;
         long long b = 16384, l2 = 8192;
-        if (const char* e = getenv("LOFAR_BUCKET_CFG")) sscanf(e, "%d,%lld,%lld", &a, &b, &l2);
+        const char* over = getenv("LOFAR_BUCKET_CFG");
+        if (over) sscanf(over, "%d,%lld,%lld", &a, &b, &l2);
         if (a < 1 || a > 16 || (a & (a - 1))) a = 16;
         if (b < 256) b = 256;
         if (l2 < 256) l2 = 256;
-        return BucketCfg{a, b, l2, stage};
+        return BucketCfg{a, b, l2, stage, over != nullptr};
     }();
     return cfg;
 }
@@ -566,24 +571,20 @@ int tile_order_log(const TileMap& m)
     return want;
 }
 
-// Level-2 block table and fine counts, placed after the records once the entry
-// total is known: returns the bytes needed; with base set, assigns the pointers.
+// Level-2 fine counts, placed after the records once the entry total is known: returns the
+// bytes needed; with base set, assigns the pointer.
 size_t level2_layout(Buckets& b, long long total, char* base)
 {
     b.l2_max_blocks = (total + b.l2_block - 1) / b.l2_block + b.map.nk1;
     const size_t nf = (size_t)b.map.sst * b.map.sst;
-    const size_t blk_bytes = align256((size_t)b.l2_max_blocks * sizeof(L2Block));
-    const size_t cnt_bytes = align256((size_t)b.l2_max_blocks * nf * sizeof(unsigned));
-    if (base) {
-        b.l2_blk = (L2Block*)base;
-        b.l2_cnt = (unsigned*)(base + blk_bytes);
-    }
-    return blk_bytes + cnt_bytes;
+    if (base) b.l2_cnt = (unsigned*)base;
+    return align256((size_t)b.l2_max_blocks * nf * sizeof(unsigned));
 }
 
 // Two-level counting sort of the samples into (w, tile) buckets: sizes the
-// workspace, counts per super-tile, scans, and reads back the entry total and
-// the validation flag (the only host synchronisation of a call).  The level-1
+// workspace, counts per super-tile (clearing nzero2 words of zero2 on the way), scans, and
+// waits for the entry total and the validation flag (the only host synchronisation of a
+// call).  The level-1
 // histograms of nw*ceil(ntv/sst)*ceil(ntu/sst) super-tiles (records and
 // entries) live in LDS up to kMaxSuperTiles (64 KiB), in global memory beyond.
 constexpr long long kMaxSuperTiles = 8192;
@@ -603,12 +604,22 @@ long long l1_lds_max()
 
 int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double* vv,
                   const double* ww, const Geometry& g, hipStream_t st, Buckets& b,
-                  long long& total, Arena* ar = nullptr)
+                  long long& total, Arena* ar = nullptr, unsigned* zero2 = nullptr,
+                  long long nzero2 = 0)
 {
     const BucketCfg cfg = bucket_cfg();
     int sst = cfg.sst;
-    const long long chunk = cfg.chunk;
+    // Few samples are spread over the chip: level-1 chunks and level-2 blocks shrink so that
+    // there are about two workgroups per CU (1M samples took 64 workgroups and 140 us for
+    // count and scatter at the full chunk).  The allocation-free call keeps the full sizes:
+    // the smaller ones need more tables, and what fitted its array has to fit.
+    long long chunk = cfg.chunk;
     b.l2_block = cfg.block;
+    if ((!ar || !ar->base) && !cfg.forced) {
+        const long long want = std::max(512LL, ((long long)n + 262143) / 262144 * 512);
+        chunk = std::min(chunk, want);
+        b.l2_block = std::min(b.l2_block, std::max(1024LL, want));
+    }
     const int span = g.ntu > g.ntv ? g.ntu : g.ntv;
     while (sst > 1 && sst / 2 >= span) sst /= 2;  // no super-tile wider than the grid
     auto super_tiles = [&](int s) {
@@ -631,43 +642,54 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     b.nwg = n > 0 ? (n + chunk - 1) / chunk : 1;
     if (b.nwg > 4096) b.nwg = 4096;
     b.chunk = n > 0 ? (n + b.nwg - 1) / b.nwg : 1;
-    const long long nblk = (m.nk1 + 4095) / 4096;
-    const size_t off_status = 0;
-    const size_t off_totrec = align256(off_status + 2 * sizeof(long long));
-    const size_t off_count1 = align256(off_totrec + sizeof(long long));
-    const size_t off_off1 = align256(off_count1 + (size_t)m.nk1 * sizeof(unsigned));
-    const size_t off_count1e = align256(off_off1 + (size_t)(m.nk1 + 1) * sizeof(long long));
-    const size_t off_eoff1 = align256(off_count1e + (size_t)m.nk1 * sizeof(unsigned));
+    const size_t off_err = 0;
+    const size_t off_count1 = align256(off_err + sizeof(long long));
+    const size_t off_count1e = align256(off_count1 + (size_t)m.nk1 * sizeof(unsigned));
+    const size_t off_off1 = align256(off_count1e + (size_t)m.nk1 * sizeof(unsigned));
+    const size_t off_eoff1 = align256(off_off1 + (size_t)(m.nk1 + 1) * sizeof(long long));
     const size_t off_base1 = align256(off_eoff1 + (size_t)(m.nk1 + 1) * sizeof(long long));
     const size_t nbase1 = b.global_l1 ? (size_t)m.nk1 : (size_t)(b.nwg * m.nk1);
     const size_t off_offsets = align256(off_base1 + nbase1 * sizeof(unsigned));
-    const size_t off_partials =
-        align256(off_offsets + (size_t)(m.nbuckets() + 1) * sizeof(long long));
-    const size_t off_l2nblk = align256(off_partials + (size_t)(nblk + 1) * sizeof(long long));
-    const size_t off_l2boff = align256(off_l2nblk + (size_t)m.nk1 * sizeof(unsigned));
-    const size_t bytes = align256(off_l2boff + (size_t)(m.nk1 + 1) * sizeof(long long));
+    const size_t off_l2boff = align256(off_offsets + (size_t)(m.nbuckets() + 1) * sizeof(long long));
+    const size_t off_l2blk = align256(off_l2boff + (size_t)(m.nk1 + 1) * sizeof(long long));
+    // a window (at most 17 cells) touches at most 4 super-tiles
+    const size_t max_blk = (size_t)((4LL * n + b.l2_block - 1) / b.l2_block + m.nk1);
+    const size_t bytes = align256(off_l2blk + max_blk * sizeof(L2Block));
     char* base = nullptr;
     int r = take(c, ar, c.meta, bytes, &base);
     if (r) return r;
-    b.total = (long long*)(base + off_status);
-    b.err = (int*)(base + off_status + sizeof(long long));
-    b.total_rec = (long long*)(base + off_totrec);
+    b.err = (int*)(base + off_err);
+    b.zero = base + off_err;
+    b.nzero = (long long)(off_off1 - off_err) / 4;
     b.count1 = (unsigned*)(base + off_count1);
     b.off1 = (long long*)(base + off_off1);
     b.count1e = (unsigned*)(base + off_count1e);
     b.eoff1 = (long long*)(base + off_eoff1);
     b.base1 = (unsigned*)(base + off_base1);
     b.offsets = (long long*)(base + off_offsets);
-    b.partials = (long long*)(base + off_partials);
-    b.l2_nblk = (unsigned*)(base + off_l2nblk);
     b.l2_boff = (long long*)(base + off_l2boff);
-    HIPCHK(stage(c, kStCount, st, [&] { return bucket_count(mode, n, uu, vv, ww, g, b, st); }));
-    HIPCHK(stage(c, kStScan, st, [&] { return bucket_scan(b, st); }));
-    HIPCHK(hipMemcpyAsync(c.status_host, b.total, 2 * sizeof(long long), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    const int err = (int)(c.status_host[1] & 0xffffffff);
-    if (err) return fail(LOFAR_ECOORD);
+    b.l2_blk = (L2Block*)(base + off_l2blk);
+    b.status = c.status_host;
+    const long long seq = ++c.status_seq;
+    HIPCHK(stage(c, kStCount, st,
+                 [&] { return bucket_count(mode, n, uu, vv, ww, g, b, zero2, nzero2, st); }));
+    HIPCHK(stage(c, kStScan, st, [&] { return bucket_scan(b, seq, st); }));
+    // The scan's last store is the call number: waiting for it costs less than a copy and a
+    // stream synchronisation, which takes over for work queued long ahead and for errors.
+    const auto t0 = std::chrono::steady_clock::now();
+    while (c.status_host[2] != seq &&
+           std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(2000))
+        for (int i = 0; i < 32 && c.status_host[2] != seq; i++) __builtin_ia32_pause();
+    if (c.status_host[2] != seq) HIPCHK(hipStreamSynchronize(st));
+    std::atomic_thread_fence(std::memory_order_acquire);
+    if (c.status_host[2] != seq) return fail(LOFAR_EHIP);
+    if (c.status_host[1]) return fail(LOFAR_ECOORD);
     total = c.status_host[0];
+    // the block table was sized for any sample positions: give back what these cannot use
+    if (ar && ar->base) {
+        const size_t used = (size_t)((total + b.l2_block - 1) / b.l2_block + m.nk1);
+        ar->used -= bytes - align256(off_l2blk + used * sizeof(L2Block));
+    }
     return LOFAR_OK;
 }
 
@@ -680,7 +702,7 @@ int validate_direct(DeviceCtx& c, Arena* ar, long n, const double* uu, const dou
     int r = take(c, ar, c.meta, 256, &p);
     if (r) return r;
     HIPCHK(validate_samples(n, uu, vv, ww, g, (int*)p, st));
-    HIPCHK(hipMemcpyAsync(&c.status_host[1], p, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync((void*)&c.status_host[1], p, sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     if ((int)(c.status_host[1] & 0xffffffff)) return fail(LOFAR_ECOORD);
     return LOFAR_OK;
@@ -692,7 +714,7 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
               const double* uu, const double* vv, const double* ww, const float* vr,
               const float* vi, const float* wt, double dx, double dw, int support, int nx, int ny,
               void* cube, hipStream_t st, unsigned long long* occ = nullptr, int sm_log = -1,
-              Arena* ar = nullptr, const lofar_plan_s* plan = nullptr)
+              Arena* ar = nullptr, const lofar_plan_s* plan = nullptr, long long nocc = 0)
 {
     int r = check_grid_args(precision, nw, n, F, P, dx, dw, support, nx, ny);
     if (r) return fail(r);
@@ -708,6 +730,7 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
         return LOFAR_OK;
     }
     if (plan) {
+        if (occ) HIPCHK(fill_u32((unsigned*)occ, 2 * nocc, 0u, st));
         Buckets b{};
         b.map = plan->gmap;
         b.offsets = plan->goff;
@@ -754,10 +777,11 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     }
     Buckets b;
     long long total = 0;
-    r = build_buckets(c, kBucketFootprint, n, uu, vv, ww, g, st, b, total, ar);
+    r = build_buckets(c, kBucketFootprint, n, uu, vv, ww, g, st, b, total, ar, (unsigned*)occ,
+                      occ ? 2 * nocc : 0);
     if (r) return r;
     // level-1 records (at most one per entry), the sorted entries, then the
-    // level-2 block table
+    // level-2 counts
     const size_t esz = precision == LOFAR_FP64 ? sizeof(Entry64) : sizeof(Entry32);
     const size_t rbytes = align256((size_t)total * sizeof(Entry64));
     const size_t ebytes = align256((size_t)total * esz);
@@ -1006,6 +1030,7 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
     // larger planes are written whole)
     int r = LOFAR_OK;
     unsigned long long* occ = nullptr;
+    long long nocc = 0;
     const long long plane_bytes = (long long)grid_size_x * grid_size_y *
                                   (precision == LOFAR_FP64 ? 16 : 8);
     // windows wider than the tile kernels take are gridded without buckets into a whole
@@ -1017,12 +1042,11 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
     if (plane_bytes < (1LL << 31) && !direct && !generic) {
         const long long ntv = (grid_size_y + kTile - 1) / kTile;
         const long long ntu = (grid_size_x + kTile - 1) / kTile;
-        const long long nocc = (long long)num_w_planes * ntu * ((ntv + 63) / 64);
+        nocc = (long long)num_w_planes * ntu * ((ntv + 63) / 64);
         char* op = nullptr;
         r = take(c, ar, c.occ, (size_t)nocc * 8 + 256, &op);
         if (r) return r;
-        occ = (unsigned long long*)op;
-        HIPCHK(fill_u32((unsigned*)occ, 2 * nocc, 0u, st));
+        occ = (unsigned long long*)op;  // cleared by grid_impl
     }
     // FP64: the scratch cube is laid out strip-major, in strips of 2^sm_log whole
     // columns (the 64-column tile width by default), so every tile flush is one
@@ -1039,7 +1063,7 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
                            : -1;
     r = grid_impl(c, precision, 0, num_w_planes, num_points, freq_per_chan, polarizations, uu, vv,
                   ww, vis_real, vis_img, weight, dx, dw, w_support, grid_size_x, grid_size_y, cube,
-                  st, occ, sm_log, ar, plan);
+                  st, occ, sm_log, ar, plan, nocc);
     if (r) return r;
     if (generic) {
         r = fft_generic_planes(c, ar, precision, 1, cube, cube, grid_size_x, grid_size_y,

@@ -204,16 +204,16 @@ struct Buckets {
     long long nent = 0;    // entries in all buckets, when the host knows it (else 0)
     const void* vis = nullptr;  // index entries: each sample's summed visibility (float2),
                                 // gathered by the gridder (grid_gathers)
-    long long* partials;   // scan partials
-    long long* total;      // host-visible total entry count (status[0])
-    long long* total_rec;  // total record count (device)
-    int* err;              // host-visible validation flag (status[1])
-    // level 2 (set once the entry total is known)
+    int* err;              // validation flag (device)
+    void* zero;            // err, count1, count1e: nzero words to clear before the count
+    long long nzero;
+    volatile long long* status;  // host memory: entry total, validation flag, call number
+    // level 2
     long long l2_block;       // records per level-2 block
-    long long l2_max_blocks;  // grid of the per-block kernels: ceil(total/l2_block) + nk1
-    unsigned* l2_nblk;        // [nk1] blocks per segment
     long long* l2_boff;       // [nk1+1] first block of each segment; [nk1] = block count
-    L2Block* l2_blk;          // [l2_max_blocks]
+    L2Block* l2_blk;          // block table
+    // set once the entry total is known
+    long long l2_max_blocks;  // grid of the per-block kernels: ceil(total/l2_block) + nk1
     unsigned* l2_cnt;         // [l2_max_blocks * sst^2] fine counts, then block bases
 };
 
@@ -223,10 +223,13 @@ enum { kBucketFootprint = 0, kBucketHome = 1 };
 enum { kStageL1 = 1, kStageL2 = 2 };
 constexpr long long kStageMaxBins = 512;
 
-// Level 1 (bucket.hip): count records and entries per super-tile, validate.
+// Level 1 (bucket.hip): count records and entries per super-tile, validate (nzero2 words of
+// zero2 are cleared on the way); then the offsets, the level-2 block table and the status
+// with call number seq.
 hipError_t bucket_count(int mode, long long n, const double* uu, const double* vv, const double* ww,
-                        const Geometry& g, const Buckets& b, hipStream_t st);
-hipError_t bucket_scan(const Buckets& b, hipStream_t st);
+                        const Geometry& g, const Buckets& b, unsigned* zero2, long long nzero2,
+                        hipStream_t st);
+hipError_t bucket_scan(const Buckets& b, long long seq, hipStream_t st);
 // Level 1 scatter into super-tile order (rec: one Entry64 per record), then level
 // 2 into (w, tile) order (entries: Entry64 for FP64, Entry32 for FP32C).
 // index_vis: the entries carry each sample's index in the real part's slot instead
