@@ -592,15 +592,44 @@ __global__ __launch_bounds__(256) void k_l2_count(Geometry g, TileMap tm, const 
     for (int f = tid; f < nf; f += 256) cnt2[b * nf + f] = cnt[f];
 }
 
+// Lists a dense tile and its pieces; the tile's place in the list is left in slots.
+__device__ __forceinline__ void list_heavy(const Heavy& h, long long bkt, long long beg,
+                                           long long n, int* slots, int* nslots)
+{
+    const int np = (int)((n + h.piece - 1) / h.piece);
+    const int t = atomicAdd(&h.count[0], 1), p0 = atomicAdd(&h.count[1], np);
+    HeavyTile d;
+    d.bkt = bkt;
+    d.beg = beg;
+    d.end = beg + n;
+    d.np = np;
+    d.pad = 0;
+    h.tile[t] = d;
+    for (int i = 0; i < np; i++) h.piece_of[p0 + i] = int2{t, i};
+    slots[atomicAdd(nslots, 1)] = t;
+}
+
+// Clears the states of the workgroup's listed tiles.
+template <int NT>
+__device__ __forceinline__ void clear_heavy(const Heavy& h, const int* slots, int nslots)
+{
+    if (!h.state) return;
+    constexpr int W = sizeof(HeavyState) / 4;
+    for (int i = threadIdx.x; i < nslots * W; i += NT)
+        ((unsigned*)&h.state[slots[i / W]])[i % W] = 0u;
+}
+
 // one workgroup per segment, one fine tile per thread: running sums over the segment's
 // blocks (replacing the counts by block bases relative to the segment's first
 // entry), then the exclusive scan over fine tiles gives the bucket offsets.  The blocks'
-// counts are read 8 at a time: they come back to back instead of one latency each.
+// counts are read 8 at a time: they come back to back instead of one latency each.  Dense
+// tiles are listed on the way (Heavy).
 __global__ __launch_bounds__(kMaxFine) void k_l2_scan(TileMap tm, const long long* eoff1,
                                                       const long long* boff, unsigned* cnt2,
-                                                      long long* offsets)
+                                                      long long* offsets, Heavy h)
 {
     __shared__ unsigned ws[kMaxFine / 64];
+    __shared__ int hslot[kMaxFine], hn;
     constexpr int G = 8;
     const int f = threadIdx.x;
     const int nf = tm.sst * tm.sst;
@@ -618,6 +647,11 @@ __global__ __launch_bounds__(kMaxFine) void k_l2_scan(TileMap tm, const long lon
     unsigned all;
     unsigned run = block_exscan<kMaxFine>(tot, ws, all);
     if (on) offsets[k1 * nf + f] = eoff1[k1] + run;
+    if (f == 0) hn = 0;
+    __syncthreads();
+    if (on && (long long)tot > h.min) list_heavy(h, k1 * nf + f, eoff1[k1] + run, tot, hslot, &hn);
+    __syncthreads();
+    clear_heavy<kMaxFine>(h, hslot, hn);
     for (long long j = b0; j < b1; j += G) {
         unsigned c[G];
 #pragma unroll
@@ -808,7 +842,7 @@ static hipError_t level2(const Geometry& g, const Buckets& b, const Rec* rec, Ou
     hipLaunchKernelGGL((k_l2_count<OUT, Rec>), dim3(grid), dim3(256), 0, st, g, b.map, nblocks,
                        b.l2_blk, rec, b.l2_cnt);
     hipLaunchKernelGGL(k_l2_scan, dim3((unsigned)nk1), dim3(kMaxFine), 0, st, b.map, b.eoff1, b.l2_boff,
-                       b.l2_cnt, b.offsets);
+                       b.l2_cnt, b.offsets, b.heavy);
     if (b.stage & kStageL2)
         hipLaunchKernelGGL((k_l2_scatter_staged<OUT, Rec, Out>), dim3(grid), dim3(kStageThreads),
                            0, st, g, b.map, b.eoff1, nblocks, b.l2_blk, b.l2_cnt, rec, ent);

@@ -41,6 +41,8 @@ struct lofar_plan_s {
     long long* hoff = nullptr;
     lofar::DEntry* hent = nullptr;
     unsigned long long* need = nullptr;  // tiles the degridding reads (powers of two)
+    // dense tiles of both sorts (tables in gmem and hmem)
+    lofar::Heavy gheavy, hheavy;
     float* wt = nullptr;
     double *uu = nullptr, *vv = nullptr, *ww = nullptr;
     char* gmem = nullptr;
@@ -605,7 +607,7 @@ long long l1_lds_max()
 int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double* vv,
                   const double* ww, const Geometry& g, hipStream_t st, Buckets& b,
                   long long& total, Arena* ar = nullptr, unsigned* zero2 = nullptr,
-                  long long nzero2 = 0)
+                  long long nzero2 = 0, int heavy_min = 0)
 {
     const BucketCfg cfg = bucket_cfg();
     int sst = cfg.sst;
@@ -643,7 +645,8 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     if (b.nwg > 4096) b.nwg = 4096;
     b.chunk = n > 0 ? (n + b.nwg - 1) / b.nwg : 1;
     const size_t off_err = 0;
-    const size_t off_count1 = align256(off_err + sizeof(long long));
+    const size_t off_hcount = off_err + sizeof(long long);
+    const size_t off_count1 = align256(off_hcount + 2 * sizeof(int));
     const size_t off_count1e = align256(off_count1 + (size_t)m.nk1 * sizeof(unsigned));
     const size_t off_off1 = align256(off_count1e + (size_t)m.nk1 * sizeof(unsigned));
     const size_t off_eoff1 = align256(off_off1 + (size_t)(m.nk1 + 1) * sizeof(long long));
@@ -654,7 +657,19 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     const size_t off_l2blk = align256(off_l2boff + (size_t)(m.nk1 + 1) * sizeof(long long));
     // a window (at most 17 cells) touches at most 4 super-tiles
     const size_t max_blk = (size_t)((4LL * n + b.l2_block - 1) / b.l2_block + m.nk1);
-    const size_t bytes = align256(off_l2blk + max_blk * sizeof(L2Block));
+    // Tables of the dense tiles (at most one entry per sample and touched tile).  The
+    // allocation-free call does without: what fitted its array has to fit.
+    Heavy& h = b.heavy;
+    h = Heavy();
+    const long long most = (mode == kBucketHome ? 1LL : 4LL) * n;
+    if (heavy_min > 0 && most > heavy_min && (!ar || !ar->base)) {
+        h.min = h.piece = heavy_min;
+        h.max_tiles = std::min(most / heavy_min, m.nbuckets());
+        h.max_pieces = most / heavy_min + h.max_tiles;
+    }
+    const size_t off_htile = align256(off_l2blk + max_blk * sizeof(L2Block));
+    const size_t off_hpiece = align256(off_htile + (size_t)h.max_tiles * sizeof(HeavyTile));
+    const size_t bytes = align256(off_hpiece + (size_t)h.max_pieces * sizeof(int2));
     char* base = nullptr;
     int r = take(c, ar, c.meta, bytes, &base);
     if (r) return r;
@@ -669,6 +684,9 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     b.offsets = (long long*)(base + off_offsets);
     b.l2_boff = (long long*)(base + off_l2boff);
     b.l2_blk = (L2Block*)(base + off_l2blk);
+    h.tile = (HeavyTile*)(base + off_htile);
+    h.piece_of = (int2*)(base + off_hpiece);
+    h.count = (int*)(base + off_hcount);
     b.status = c.status_host;
     const long long seq = ++c.status_seq;
     HIPCHK(stage(c, kStCount, st,
@@ -685,6 +703,10 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     if (c.status_host[2] != seq) return fail(LOFAR_EHIP);
     if (c.status_host[1]) return fail(LOFAR_ECOORD);
     total = c.status_host[0];
+    if (h.max_pieces > 0) {
+        h.max_tiles = std::min(total / h.min, h.max_tiles);
+        h.max_pieces = h.max_tiles > 0 ? total / h.piece + h.max_tiles : 0;
+    }
     // the block table was sized for any sample positions: give back what these cannot use
     if (ar && ar->base) {
         const size_t used = (size_t)((total + b.l2_block - 1) / b.l2_block + m.nk1);
@@ -692,6 +714,20 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     }
     return LOFAR_OK;
 }
+
+// Scratch bytes of the gridder's dense tiles (states, then sum words); with base set, assigns
+// the pointers.
+size_t heavy_layout(Heavy& h, char* base)
+{
+    const size_t state = align256((size_t)h.max_tiles * sizeof(HeavyState));
+    if (base) {
+        h.state = (HeavyState*)base;
+        h.acc = (unsigned long long*)(base + state);
+    }
+    return state + (size_t)h.max_tiles * 2 * kTile * kTile * sizeof(unsigned long long);
+}
+
+int heavy_min_of(int precision) { return precision == LOFAR_FP64 ? kHeavyFp64 : kHeavyFp32; }
 
 // Sample validation of the bucket-free path (the checks of the bucket count): read back
 // before anything is written, so that a bad sample leaves the outputs untouched.
@@ -735,12 +771,24 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
         b.map = plan->gmap;
         b.offsets = plan->goff;
         b.nent = plan->gtotal;
+        if (grid_splits(precision, accumulate)) b.heavy = plan->gheavy;
+        const size_t hbytes = b.heavy.max_tiles > 0 ? heavy_layout(b.heavy, nullptr) : 0;
+        auto dense = [&](char* base) -> int {
+            if (b.heavy.max_tiles <= 0) return LOFAR_OK;
+            heavy_layout(b.heavy, base);
+            HIPCHK(fill_u32((unsigned*)b.heavy.state,
+                            b.heavy.max_tiles * (long long)(sizeof(HeavyState) / 4), 0u, st));
+            return LOFAR_OK;
+        };
         if (grid_gathers(precision, accumulate)) {
             // the gridder gathers each entry's sample sum: no filled copy of the entries
             char* vb = nullptr;
-            r = take(c, ar, c.ents, align256(plan_vis_bytes(precision, n)) + 256, &vb);
+            const size_t vbytes = align256(plan_vis_bytes(precision, n));
+            r = take(c, ar, c.ents, vbytes + hbytes + 256, &vb);
             if (r) return r;
             b.vis = vb;
+            r = dense(vb + vbytes);
+            if (r) return r;
             HIPCHK(stage(c, kStScatter, st, [&] {
                 return plan_vis(precision, n, F, P, vr, vi, wt, vb, st);
             }));
@@ -751,8 +799,11 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
         }
         const size_t esz = precision == LOFAR_FP64 ? sizeof(Entry64) : sizeof(Entry32);
         const size_t ebytes = align256((size_t)plan->gtotal * esz);
+        const size_t vbytes = align256(plan_vis_bytes(precision, n));
         char* eb = nullptr;
-        r = take(c, ar, c.ents, ebytes + align256(plan_vis_bytes(precision, n)) + 256, &eb);
+        r = take(c, ar, c.ents, ebytes + vbytes + hbytes + 256, &eb);
+        if (r) return r;
+        r = dense(eb + ebytes + vbytes);
         if (r) return r;
         HIPCHK(stage(c, kStScatter, st, [&] {
             return plan_fill(precision, n, plan->gtotal, plan->gent, eb, F, P, vr, vi, wt,
@@ -778,7 +829,8 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     Buckets b;
     long long total = 0;
     r = build_buckets(c, kBucketFootprint, n, uu, vv, ww, g, st, b, total, ar, (unsigned*)occ,
-                      occ ? 2 * nocc : 0);
+                      occ ? 2 * nocc : 0,
+                      grid_splits(precision, accumulate) ? heavy_min_of(precision) : 0);
     if (r) return r;
     // level-1 records (at most one per entry), the sorted entries, then the
     // level-2 counts
@@ -786,12 +838,22 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     const size_t rbytes = align256((size_t)total * sizeof(Entry64));
     const size_t ebytes = align256((size_t)total * esz);
     const size_t l2 = level2_layout(b, total, nullptr);
+    // the dense tiles' states; their sums take the place of the records, which are no longer
+    // read when the gridder runs (32 bytes a record, at most 16 an entry of a dense tile)
+    const size_t hs = align256((size_t)b.heavy.max_tiles * sizeof(HeavyState));
     char* eb = nullptr;
-    r = take(c, ar, c.ents, rbytes + ebytes + l2 + 256, &eb);
+    r = take(c, ar, c.ents, rbytes + ebytes + l2 + hs + 256, &eb);
     if (r) return r;
     Entry64* rec = (Entry64*)eb;
     void* ents = eb + rbytes;
     level2_layout(b, total, eb + rbytes + ebytes);
+    static_assert(2 * kTile * kTile * 8 <= kHeavyFp64 * (int)sizeof(Entry64) &&
+                      kHeavyFp64 <= kHeavyFp32,
+                  "a dense tile's sums fit its records");
+    if (b.heavy.max_tiles > 0) {
+        b.heavy.state = (HeavyState*)(eb + rbytes + ebytes + l2);
+        b.heavy.acc = (unsigned long long*)eb;
+    }
     b.nent = total;
     HIPCHK(stage(c, kStScatter, st, [&] {
         return bucket_sort_grid(precision, n, F, P, uu, vv, ww, vr, vi, wt, g, b, rec, ents, st);
@@ -1188,7 +1250,8 @@ int lofar_degrid_cube_dev(int precision, int num_w_planes, long num_points, long
     }
     Buckets b;
     long long total = 0;
-    r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, cg.st, b, total);
+    r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, cg.st, b, total, nullptr, nullptr,
+                      0, kHeavyHome);
     if (r) return r;
     const size_t ebytes = align256((size_t)total * sizeof(DEntry));
     const size_t l2 = level2_layout(b, total, nullptr);
@@ -1318,7 +1381,8 @@ int lofar_degrid_dev(int precision, int num_w_planes, long num_points, long freq
     // the tiles it reads, the transforms storing only those, and the interpolation
     Buckets b;
     long long total = 0;
-    r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, st, b, total);
+    r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, st, b, total, nullptr, nullptr, 0,
+                      kHeavyHome);
     if (r) return r;
     const size_t ebytes = align256((size_t)total * sizeof(DEntry));
     const size_t l2 = level2_layout(b, total, nullptr);
@@ -1351,6 +1415,41 @@ int lofar_degrid_dev(int precision, int num_w_planes, long num_points, long freq
 
 // ---------------------------------------------------------------------------
 // plans: one sort of fixed samples, kept for repeated imaging and degridding
+
+// A plan's dense tiles: how many there are (after the sort that listed them), the bytes of
+// their tables, and the tables' copy into the plan's memory.
+static int plan_heavy_size(const Heavy& from, Heavy& to, hipStream_t st)
+{
+    to = Heavy();
+    if (from.max_pieces <= 0) return LOFAR_OK;
+    int count[2] = {0, 0};
+    HIPCHK(hipMemcpyAsync(count, from.count, sizeof(count), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (count[0] <= 0) return LOFAR_OK;
+    to.min = from.min;
+    to.piece = from.piece;
+    to.max_tiles = count[0];
+    to.max_pieces = count[1];
+    return LOFAR_OK;
+}
+static size_t plan_heavy_bytes(const Heavy& h)
+{
+    return 256 + align256((size_t)h.max_tiles * sizeof(HeavyTile)) +
+           align256((size_t)h.max_pieces * sizeof(int2));
+}
+static int plan_heavy_copy(const Heavy& from, Heavy& to, char* mem, hipStream_t st)
+{
+    if (to.max_tiles <= 0) return LOFAR_OK;
+    to.count = (int*)mem;
+    to.tile = (HeavyTile*)(mem + 256);
+    to.piece_of = (int2*)(mem + 256 + align256((size_t)to.max_tiles * sizeof(HeavyTile)));
+    HIPCHK(hipMemcpyAsync(to.count, from.count, 2 * sizeof(int), hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipMemcpyAsync(to.tile, from.tile, to.max_tiles * sizeof(HeavyTile),
+                          hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipMemcpyAsync(to.piece_of, from.piece_of, to.max_pieces * sizeof(int2),
+                          hipMemcpyDeviceToDevice, st));
+    return LOFAR_OK;
+}
 
 int lofar_plan_create(int precision, int num_w_planes, long num_points, long freq_per_chan,
                       long polarizations, const double* uu, const double* vv, const double* ww,
@@ -1423,7 +1522,8 @@ int lofar_plan_create(int precision, int num_w_planes, long num_points, long fre
         // gridding: the sort of lofar_grid_dev with sample indices for visibilities
         Buckets b;
         long long total = 0;
-        r = build_buckets(c, kBucketFootprint, num_points, uu, vv, ww, g, st, b, total);
+        r = build_buckets(c, kBucketFootprint, num_points, uu, vv, ww, g, st, b, total, nullptr,
+                          nullptr, 0, heavy_min_of(precision));
         if (r) return r;
         const size_t esz = precision == LOFAR_FP64 ? sizeof(Entry64) : sizeof(Entry32);
         const size_t rbytes = align256((size_t)total * sizeof(Entry64));
@@ -1438,7 +1538,11 @@ int lofar_plan_create(int precision, int num_w_planes, long num_points, long fre
                                 true));
         const long long nbg = b.map.nbuckets();
         const size_t obytes = align256((size_t)(nbg + 1) * sizeof(long long));
-        r = alloc(&p->gmem, obytes + ebytes);
+        r = plan_heavy_size(b.heavy, p->gheavy, st);
+        if (r) return r;
+        r = alloc(&p->gmem, obytes + ebytes + plan_heavy_bytes(p->gheavy));
+        if (r) return r;
+        r = plan_heavy_copy(b.heavy, p->gheavy, p->gmem + obytes + ebytes, st);
         if (r) return r;
         p->gmap = b.map;
         p->gtotal = total;
@@ -1453,7 +1557,8 @@ int lofar_plan_create(int precision, int num_w_planes, long num_points, long fre
         // degridding: the home sort of lofar_degrid_cube_dev
         Buckets hb;
         long long htotal = 0;
-        r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, st, hb, htotal);
+        r = build_buckets(c, kBucketHome, num_points, uu, vv, ww, g, st, hb, htotal, nullptr,
+                          nullptr, 0, kHeavyHome);
         if (r) return r;
         const size_t hbytes = align256((size_t)htotal * sizeof(DEntry));
         const size_t hl2 = level2_layout(hb, htotal, nullptr);
@@ -1467,7 +1572,11 @@ int lofar_plan_create(int precision, int num_w_planes, long num_points, long fre
         const size_t hobytes = align256((size_t)(nbh + 1) * sizeof(long long));
         const bool pow2 = pow2_ok(grid_size_x) && pow2_ok(grid_size_y);
         const size_t nbytes = pow2 ? align256((size_t)need_words(g) * 8) : 0;
-        r = alloc(&p->hmem, hobytes + hbytes + wbytes + nbytes);
+        r = plan_heavy_size(hb.heavy, p->hheavy, st);
+        if (r) return r;
+        r = alloc(&p->hmem, hobytes + hbytes + wbytes + nbytes + plan_heavy_bytes(p->hheavy));
+        if (r) return r;
+        r = plan_heavy_copy(hb.heavy, p->hheavy, p->hmem + hobytes + hbytes + wbytes + nbytes, st);
         if (r) return r;
         p->hmap = hb.map;
         p->htotal = htotal;
@@ -1533,6 +1642,7 @@ int lofar_plan_degrid(lofar_plan plan, double resolution, double wmin, double wm
     Buckets hb{};
     hb.map = plan->hmap;
     hb.offsets = plan->hoff;
+    hb.heavy = plan->hheavy;
     HIPCHK(stage(c, kStDegrid, cg.st, [&] {
         return degrid_tiles(plan->precision, g, hb, plan->hent, cube, plan->wt, plan->F, plan->P,
                             model_real, model_imag, cg.st);

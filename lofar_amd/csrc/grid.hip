@@ -602,6 +602,14 @@ __device__ __forceinline__ float half_value(unsigned long long word, double inv)
         return (float)__longlong_as_double((long long)word);
 }
 
+// The two sums of a packed word, times 2^-S
+__device__ __forceinline__ float2 packed_value(unsigned long long t, double inv)
+{
+    const int im = (int)(unsigned)t;
+    const long long re = (long long)(t - (unsigned long long)(long long)im) >> 32;
+    return float2{(float)((double)re * inv), (float)((double)im * inv)};
+}
+
 // Entry e; with vis (a plan's entries, whose real part's slot holds the sample index),
 // its visibility is the sample's summed visibility in vis.
 __device__ __forceinline__ Entry32 entry_at(const Entry32* entries, const float2* vis, long long e)
@@ -647,11 +655,248 @@ __device__ __forceinline__ void grid_halves(unsigned long long* acc, const Geome
     }
 }
 
+// ---------------------------------------------------------------------------
+// dense tiles (Heavy): their pieces' workgroups first collect the tile's largest component,
+// sum and finiteness (in the tile kernels' launch), then accumulate with the scale that
+// follows from them; the pieces' integer sums meet in the tile's sum words with global
+// atomics, and the last piece stores the tile.  The sums are those of one workgroup bit for
+// bit in FP32C mode; in FP64 mode the scale follows the entries touching the densest 4x4
+// block instead of all of the tile's, so the quantum is finer.  A core-dominated array's
+// 1.05M x 8 visibilities on 2048x2048x16: the FP64 gridder 1.45 -> 0.3 ms, the image 2.79
+// -> 1.04 ms; one workgroup had taken the core's tile.  The extra launch (two in FP32C
+// mode) costs 3 us where no tile is dense.
+
+struct Piece {
+    int tile, num;
+    HeavyTile t;
+    long long beg, end;  // entries
+    long long w;
+    int tv, tu;
+};
+__device__ __forceinline__ bool piece_at(const Geometry& g, const TileMap& tm, const Heavy& h,
+                                         long long id, Piece& p)
+{
+    if (id >= (long long)h.count[1]) return false;
+    const int2 x = h.piece_of[id];
+    p.tile = x.x;
+    p.num = x.y;
+    p.t = h.tile[x.x];
+    p.beg = p.t.beg + (long long)x.y * h.piece;
+    p.end = min(p.t.end, p.beg + h.piece);
+    return tm.decode(p.t.bkt, g, p.w, p.tv, p.tu);
+}
+
+// Counts an FP64 entry in the 4x4 blocks its clipped window touches.
+template <int WIN>
+__device__ __forceinline__ void count_blocks(unsigned* cnt, const Geometry& g, int u0, int v0,
+                                             const Entry64& en)
+{
+    const TileWin t = clip_window((int)en.pu, (int)en.pv, g, u0, v0);
+    for (int r = t.b0 / kBlk; r <= (t.b0 + t.nb) / kBlk; r++)
+        for (int c = t.a0 / kBlk; c <= (t.a0 + t.na) / kBlk; c++)
+            atomicAdd(&cnt[r * kNBlk + c], 1u);
+}
+
+// Statistics of one piece into its tile's state (FP64: the block counts too, through cnt in
+// LDS), and its share of clearing the tile's sum words.
+template <int WIN, int NT, bool FP64, typename Ent>
+__device__ __forceinline__ void heavy_stats(const Geometry& g, const TileMap& tm, const Heavy& h,
+                                            long long id, const Ent* entries, const float2* vis,
+                                            unsigned* cnt)
+{
+    Piece p;
+    if (!piece_at(g, tm, h, id, p)) return;
+    const int tid = threadIdx.x;
+    unsigned long long* words = h.acc + (long long)p.tile * 2 * kPlane;
+    const int c1 = (int)((long long)(p.num + 1) * 2 * kPlane / p.t.np);
+    for (int c = (int)((long long)p.num * 2 * kPlane / p.t.np) + tid; c < c1; c += NT)
+        words[c] = 0ull;
+    if constexpr (FP64) {
+        for (int b = tid; b < kNBlk * kNBlk; b += NT) cnt[b] = 0u;
+        __syncthreads();
+    }
+    double m = 0.0, sa = 0.0;
+    bool finite = true;
+    for (long long e = p.beg + tid; e < p.end; e += NT) {
+        Ent en;
+        if constexpr (FP64)
+            en = entries[e];
+        else
+            en = entry_at(entries, vis, e);
+        const double vr = fabs((double)en.vr), vi = fabs((double)en.vi);
+        finite = finite && isfinite(vr) && isfinite(vi);
+        m = fmax(m, fmax(vr, vi));
+        sa += vr + vi;
+        if constexpr (FP64) count_blocks<WIN>(cnt, g, p.tu * kTile, p.tv * kTile, en);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        m = fmax(m, __shfl_xor(m, off));
+        sa += __shfl_xor(sa, off);
+    }
+    const bool wave_finite = __all(finite);
+    HeavyState* st = &h.state[p.tile];
+    if ((tid & 63) == 0) {
+        atomicMax(&st->m, (unsigned long long)__double_as_longlong(m));  // m >= 0
+        atomicAdd(&st->sa, sa);
+        if (!wave_finite) atomicOr(&st->nonfinite, 1u);
+    }
+    if constexpr (FP64) {
+        __syncthreads();
+        for (int b = tid; b < kNBlk * kNBlk; b += NT)
+            if (cnt[b]) atomicAdd(&st->blk[b], (unsigned long long)cnt[b]);
+    }
+}
+
+// Whether the tile is summed in floating point (a non-finite value, or a bright outlier), as
+// the tile kernels decide it.
+__device__ __forceinline__ bool heavy_float(const HeavyState& st, long long n)
+{
+    const double m = __longlong_as_double((long long)st.m);
+    return st.nonfinite || m > kHdrRatio * (st.sa - m) / (double)(2 * n - 1);
+}
+
+// Adds the LDS sums (words, or doubles for FLOAT) to the tile's; true in the workgroup that
+// was the tile's last, with every piece's sums visible to it.
+template <int NT>
+__device__ __forceinline__ bool heavy_merge(const Heavy& h, const Piece& p,
+                                            const unsigned long long* acc, int nwords, bool flt,
+                                            int* last)
+{
+    unsigned long long* words = h.acc + (long long)p.tile * 2 * kPlane;
+    for (int c = threadIdx.x; c < nwords; c += NT) {
+        const unsigned long long x = acc[c];
+        if (x == 0ull) continue;
+        if (flt)
+            atomicAdd((double*)&words[c], __longlong_as_double((long long)x));
+        else
+            atomicAdd(&words[c], x);
+    }
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        *last = atomicAdd(&h.state[p.tile].done, 1u) == (unsigned)(p.t.np - 1) ? 1 : 0;
+    __syncthreads();
+    if (!*last) return false;
+    __threadfence();
+    return true;
+}
+__device__ __forceinline__ unsigned long long heavy_word(const Heavy& h, const Piece& p, int c)
+{
+    return __hip_atomic_load(&h.acc[(long long)p.tile * 2 * kPlane + c], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// FP32C: a piece's block bounds (add_block_bound) into its tile's state; tiles whose sums
+// need none (floating point, or two words a cell whatever the bounds) are left out.
+template <int WIN, int NT>
+__global__ __launch_bounds__(NT) void k_heavy_bounds(Geometry g, TileMap tm, const Entry32* entries,
+                                                      const float2* vis, Heavy h)
+{
+    __shared__ unsigned long long bsum[kNBlk * kNBlk];
+    Piece p;
+    if (!piece_at(g, tm, h, blockIdx.x, p)) return;
+    HeavyState* st = &h.state[p.tile];
+    const long long n = p.t.end - p.t.beg;
+    const float m = (float)__longlong_as_double((long long)st->m);
+    if (n >= kPkMaxEntries || m < 0x1p-100f || heavy_float(*st, n)) return;
+    const int tid = threadIdx.x, u0 = p.tu * kTile, v0 = p.tv * kTile;
+    for (int b = tid; b < kNBlk * kNBlk; b += NT) bsum[b] = 0ull;
+    __syncthreads();
+    const float rm = kBndUnit / m;
+    for (long long e = p.beg + tid; e < p.end; e += NT)
+        add_block_bound<WIN>(bsum, g, u0, v0, rm, entry_at(entries, vis, e));
+    __syncthreads();
+    for (int b = tid; b < kNBlk * kNBlk; b += NT)
+        if (bsum[b]) atomicAdd(&st->blk[b], bsum[b]);
+}
+
+// FP32C: one piece of a dense tile, with the sums k_grid_tiles_pk would take for the tile:
+// packed words, one 64-bit word per component, or doubles.
+template <int WIN, int NT>
+__global__ __launch_bounds__(NT) void k_grid_heavy32(Geometry g, TileMap tm, const Entry32* entries,
+                                                      const float2* vis, float2* cube, int sm_log,
+                                                      Heavy h)
+{
+    __shared__ __align__(16) unsigned long long acc[2 * kPlane];
+    __shared__ int dense_blk, tile_ex, last;
+    Piece p;
+    if (!piece_at(g, tm, h, blockIdx.x, p)) return;
+    const int tid = threadIdx.x, u0 = p.tu * kTile, v0 = p.tv * kTile;
+    const long long n = p.t.end - p.t.beg;
+    const HeavyState& st = h.state[p.tile];
+    const float m = (float)__longlong_as_double((long long)st.m);
+    const double norm = 0.5 / LOFAR_REF_PI;
+    for (int c = tid; c < kPlane; c += NT)  // 2*kPlane words, 16 bytes a store
+        ((ulonglong2*)acc)[c] = ulonglong2{0ull, 0ull};
+    if (tid == 0) {
+        dense_blk = 0;
+        tile_ex = -1074;
+    }
+    __syncthreads();
+    const bool flt = heavy_float(st, n);
+    bool dense = n >= kPkMaxEntries || m < 0x1p-100f;
+    if (!flt && !dense) {
+        for (int blk = tid; blk < kNBlk * kNBlk; blk += NT) {
+            const unsigned long long b = st.blk[blk];
+            if (b == 0ull) continue;
+            int ex = 0;
+            frexp((double)(b & ((1ull << kCntShift) - 1)) * (norm * (double)m / (double)kBndUnit),
+                  &ex);
+            atomicMax(&tile_ex, ex);
+            if ((b >> kCntShift) > (unsigned long long)kPkMaxBlk) dense_blk = 1;
+        }
+        __syncthreads();
+        dense = dense_blk != 0;
+    }
+    int S = 0;
+    if (flt) {
+        for (long long e = p.beg + tid; e < p.end; e += NT) {
+            const Entry32 en = entry_at(entries, vis, e);
+            accumulate_half<WIN, 0, false>(acc, g, u0, v0, norm, 0.0, en);
+            accumulate_half<WIN, 1, false>(acc + kPlane, g, u0, v0, norm, 0.0, en);
+        }
+    } else if (dense) {
+        int ex = 0;
+        frexp(norm * (double)(m > 0.0f ? m : 1.0f), &ex);
+        int hb = 2;
+        for (long long cnt = n; cnt > 1; cnt >>= 1) hb++;
+        S = kFixedBits - hb - ex;
+        const double scale = ldexp(1.0, S);
+        for (long long e = p.beg + tid; e < p.end; e += NT) {
+            const Entry32 en = entry_at(entries, vis, e);
+            accumulate_half<WIN, 0, true>(acc, g, u0, v0, norm, scale, en);
+            accumulate_half<WIN, 1, true>(acc + kPlane, g, u0, v0, norm, scale, en);
+        }
+    } else {
+        S = kPkHead - tile_ex;
+        const double scale = ldexp(1.0, S);
+        for (long long e = p.beg + tid; e < p.end; e += NT)
+            accumulate_pk32<WIN>(acc, g, u0, v0, norm, scale, entry_at(entries, vis, e));
+    }
+    __syncthreads();
+    const bool packed = !flt && !dense;
+    if (!heavy_merge<NT>(h, p, acc, packed ? kPlane : 2 * kPlane, flt, &last)) return;
+    const int tcols = min(kTile, g.nx - u0), trows = min(kTile, g.ny - v0);
+    const double inv = ldexp(1.0, -S);
+    for (int c = tid; c < kPlane; c += NT) {
+        const FlushCell f = flush_cell(c, sm_log, g, p.w, u0, v0);
+        if (f.row >= trows || f.col >= tcols) continue;
+        const unsigned long long a = heavy_word(h, p, f.a);
+        if (packed) {
+            cube[f.off] = packed_value(a, inv);
+        } else {
+            const unsigned long long b = heavy_word(h, p, kPlane + f.a);
+            cube[f.off] = flt ? float2{half_value<false>(a, inv), half_value<false>(b, inv)}
+                              : float2{half_value<true>(a, inv), half_value<true>(b, inv)};
+        }
+    }
+}
+
 template <int WIN, int NT>
 __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, const long long* offsets,
                                                        const Entry32* entries, const float2* vis,
                                                        float2* cube, unsigned long long* occ,
-                                                       int sm_log)
+                                                       int sm_log, Heavy h)
 {
     __shared__ __align__(16) unsigned long long acc[kPlane];
     __shared__ unsigned long long bsum[kNBlk * kNBlk];
@@ -659,6 +904,10 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, co
     __shared__ double wsum[NT / 64];
     __shared__ int wfin[NT / 64];
     __shared__ int dense_blk, tile_ex;
+    if (blockIdx.x >= tm.nbuckets()) {
+        heavy_stats<WIN, NT, false>(g, tm, h, blockIdx.x - tm.nbuckets(), entries, vis, nullptr);
+        return;
+    }
     long long w;
     int tv, tu;
     const long long bkt = tm.launch_bucket(blockIdx.x, g, w, tv, tu);
@@ -683,6 +932,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, co
         }
         return;
     }
+    if (end - beg > h.min) return;  // split (k_grid_heavy32)
     // the first 2*NT entries are loaded once and kept in registers
     const long long n = end - beg;
     const int lane = tid & 63, wave = tid >> 6;
@@ -773,10 +1023,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, co
     for (int c = tid; c < kPlane; c += NT) {
         const FlushCell f = flush_cell(c, sm_log, g, w, u0, v0);
         if (f.row < trows && f.col < tcols) {
-            const unsigned long long t = acc[f.a];
-            const int im = (int)(unsigned)t;
-            const long long re = (long long)(t - (unsigned long long)(long long)im) >> 32;
-            cube[f.off] = float2{(float)((double)re * inv), (float)((double)im * inv)};
+            cube[f.off] = packed_value(acc[f.a], inv);
         }
     }
 }
@@ -916,7 +1163,8 @@ template <int WIN, int NT>
 __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
                                                          const long long* offsets,
                                                          const Entry64* entries, double2* cube,
-                                                         unsigned long long* occ, int sm_log)
+                                                         unsigned long long* occ, int sm_log,
+                                                         Heavy h)
 {
     // the WIN x WIN square at a window's first cell reaches (WIN-1)*(kTile+1) words
     // past the tile's last cell (accumulate_fx64)
@@ -925,6 +1173,11 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     __shared__ double wred[NT / 64];
     __shared__ double wsum[NT / 64];
     __shared__ int wfin[NT / 64];
+    if (blockIdx.x >= tm.nbuckets()) {
+        heavy_stats<WIN, NT, true>(g, tm, h, blockIdx.x - tm.nbuckets(), entries, nullptr,
+                                   (unsigned*)acc);
+        return;
+    }
     long long w;
     int tv, tu;
     const long long bkt = tm.launch_bucket(blockIdx.x, g, w, tv, tu);
@@ -947,6 +1200,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
         }
         return;
     }
+    if (end - beg > h.min) return;  // split (k_grid_heavy64)
     // Entries are taken in rounds of NT; a round of r entries goes to ceil(r/32)
     // waves (at most all of them), so that a small tile still spreads over the
     // SIMDs.  The first round's entry is loaded once, before the LDS clear, and
@@ -1033,30 +1287,95 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     }
 }
 
+// One piece of a dense tile (FP64).
+template <int WIN, int NT>
+__global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, const Entry64* entries,
+                                                      double2* cube, int sm_log, Heavy h)
+{
+    constexpr int kPad = ((WIN - 1) * (kTile + 1) + 1) / 2 * 2;  // as k_grid_tiles_fx64
+    __shared__ __align__(16) unsigned long long acc[2 * kPlane + kPad];
+    __shared__ unsigned long long maxcnt;
+    __shared__ int last;
+    Piece p;
+    if (!piece_at(g, tm, h, blockIdx.x, p)) return;
+    const int tid = threadIdx.x, u0 = p.tu * kTile, v0 = p.tv * kTile;
+    const long long n = p.t.end - p.t.beg;
+    const HeavyState& st = h.state[p.tile];
+    const double m = __longlong_as_double((long long)st.m);
+    const double norm = 0.5 / LOFAR_REF_PI;
+    if (tid == 0) maxcnt = 1ull;
+    for (int c = tid; c < kPlane; c += NT)  // 2*kPlane words, 16 bytes a store
+        ((ulonglong2*)acc)[c] = ulonglong2{0ull, 0ull};
+    __syncthreads();
+    const bool flt = heavy_float(st, n);
+    int S = 0;
+    if (flt) {
+        for (long long e = p.beg + tid; e < p.end; e += NT)
+            accumulate_f64<WIN>((double*)acc, g, u0, v0, norm, entries[e]);
+    } else {
+        for (int b = tid; b < kNBlk * kNBlk; b += NT) atomicMax(&maxcnt, st.blk[b]);
+        __syncthreads();
+        int ex = 0;
+        frexp(norm * (m > 0.0 ? m : 1.0), &ex);  // norm*m < 2^ex
+        int hb = 2;
+        for (unsigned long long cnt = maxcnt; cnt > 1; cnt >>= 1) hb++;
+        S = kFixedBits64 - hb - ex;
+        const double scale = ldexp(1.0, S);
+        for (long long e = p.beg + tid; e < p.end; e += NT)
+            accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, entries[e]);
+    }
+    __syncthreads();
+    if (!heavy_merge<NT>(h, p, acc, 2 * kPlane, flt, &last)) return;
+    const int tcols = min(kTile, g.nx - u0), trows = min(kTile, g.ny - v0);
+    const double inv = ldexp(1.0, -S);
+    for (int c = tid; c < kPlane; c += NT) {
+        const FlushCell f = flush_cell(c, sm_log, g, p.w, u0, v0);
+        if (f.row >= trows || f.col >= tcols) continue;
+        const unsigned long long a = heavy_word(h, p, f.a), b = heavy_word(h, p, kPlane + f.a);
+        cube[f.off] = flt ? double2{__longlong_as_double((long long)a),
+                                    __longlong_as_double((long long)b)}
+                          : double2{from_fixed(a, inv), from_fixed(b, inv)};
+    }
+}
+
 // ---------------------------------------------------------------------------
 // degridding (adjoint of gridding)
 
 // One workgroup per home tile: the tile plus a halo of (WIN-1)/2 cells is staged
 // in LDS; one lane per sample gathers its window (same clipping and weights as
-// the gridder) and writes weight*sum for every channel and polarisation.
+// the gridder) and writes weight*sum for every channel and polarisation.  A dense tile's
+// further pieces (Heavy) are the workgroups beyond the tiles': 3.0M samples of a
+// core-dominated array on 2048x1024x12 took one workgroup 4.9 ms for the core's tile.
 template <int WIN, bool FP64>
 __global__ __launch_bounds__(256) void k_degrid_tiles(Geometry g, TileMap tm, const long long* offsets,
                                                       const DEntry* ents, const void* cube,
                                                       const float* weight, long long F,
-                                                      long long P, void* mre, void* mim)
+                                                      long long P, void* mre, void* mim, Heavy h)
 {
     using Real = typename std::conditional<FP64, double, float>::type;
     using T2 = typename cplx<Real>::type;
     constexpr int H = (WIN - 1) / 2;
     constexpr int RS = kTile + 2 * H;
     __shared__ T2 region[RS * RS];
-    long long w;
+    long long w, beg, end;
     int tv, tu;
-    const long long bkt = tm.launch_bucket(blockIdx.x, g, w, tv, tu);
-    if (bkt < 0) return;
+    if (blockIdx.x < tm.nbuckets()) {
+        const long long bkt = tm.launch_bucket(blockIdx.x, g, w, tv, tu);
+        if (bkt < 0) return;
+        beg = offsets[bkt];
+        end = offsets[bkt + 1];
+        if (beg == end) return;
+        if (end - beg > h.min) end = beg + h.piece;  // a dense tile's first piece
+    } else {
+        Piece p;
+        if (!piece_at(g, tm, h, blockIdx.x - tm.nbuckets(), p) || p.num == 0) return;
+        w = p.w;
+        tv = p.tv;
+        tu = p.tu;
+        beg = p.beg;
+        end = p.end;
+    }
     const int u0 = tu * kTile, v0 = tv * kTile;
-    const long long beg = offsets[bkt], end = offsets[bkt + 1];
-    if (beg == end) return;
     const T2* plane = (const T2*)cube + w * (long long)g.ny * g.nx;
     const int tid = threadIdx.x;
     // every load of the thread's part of the region is issued before the first LDS
@@ -1274,17 +1593,32 @@ static void launch_grid_nt(int precision, const Geometry& g, const Buckets& b, c
 {
     const dim3 grid((unsigned)b.map.nbuckets());
     const int cfg = grid_cfg();
-    if (precision == LOFAR_FP64 && !accumulate && cfg != 1)
-        hipLaunchKernelGGL((k_grid_tiles_fx64<WIN, NT>), grid, dim3(NT), 0, st, g, b.map,
-                           b.offsets, (const Entry64*)entries, (double2*)cube, occ, sm_log);
-    else if (precision == LOFAR_FP64)
+    // the packed and the FP64 fixed-point kernels split dense tiles: their launch has the
+    // pieces' statistics as further workgroups
+    const Heavy& h = b.heavy;
+    const dim3 split((unsigned)(b.map.nbuckets() + h.max_pieces)), pieces((unsigned)h.max_pieces);
+    constexpr int HT = 512;
+    if (precision == LOFAR_FP64 && !accumulate && cfg != 1) {
+        hipLaunchKernelGGL((k_grid_tiles_fx64<WIN, NT>), split, dim3(NT), 0, st, g, b.map,
+                           b.offsets, (const Entry64*)entries, (double2*)cube, occ, sm_log, h);
+        if (h.max_pieces > 0)
+            hipLaunchKernelGGL((k_grid_heavy64<WIN, HT>), pieces, dim3(HT), 0, st, g, b.map,
+                               (const Entry64*)entries, (double2*)cube, sm_log, h);
+    } else if (precision == LOFAR_FP64)
         hipLaunchKernelGGL((k_grid_tiles<WIN, true, NT>), grid, dim3(NT), 0, st, g, b.map,
                            b.offsets, entries, cube, accumulate, occ, sm_log);
-    else if (!accumulate && cfg == 0)
-        hipLaunchKernelGGL((k_grid_tiles_pk<WIN, NT>), grid, dim3(NT), 0, st, g, b.map, b.offsets,
+    else if (!accumulate && cfg == 0) {
+        hipLaunchKernelGGL((k_grid_tiles_pk<WIN, NT>), split, dim3(NT), 0, st, g, b.map, b.offsets,
                            (const Entry32*)entries, (const float2*)b.vis, (float2*)cube, occ,
-                           sm_log);
-    else if (!accumulate && cfg == 2)
+                           sm_log, h);
+        if (h.max_pieces > 0) {
+            hipLaunchKernelGGL((k_heavy_bounds<WIN, HT>), pieces, dim3(HT), 0, st, g, b.map,
+                               (const Entry32*)entries, (const float2*)b.vis, h);
+            hipLaunchKernelGGL((k_grid_heavy32<WIN, HT>), pieces, dim3(HT), 0, st, g, b.map,
+                               (const Entry32*)entries, (const float2*)b.vis, (float2*)cube,
+                               sm_log, h);
+        }
+    } else if (!accumulate && cfg == 2)
         hipLaunchKernelGGL((k_grid_tiles_fx<WIN, NT>), grid, dim3(NT), 0, st, g, b.map, b.offsets,
                            (const Entry32*)entries, (float2*)cube, occ, sm_log);
     else
@@ -1364,6 +1698,11 @@ hipError_t degrid_direct(int precision, long long n, long long F, long long P, c
     return hipGetLastError();
 }
 
+bool grid_splits(int precision, int accumulate)
+{
+    return !accumulate && (precision == LOFAR_FP64 ? grid_cfg() != 1 : grid_cfg() == 0);
+}
+
 bool grid_gathers(int precision, int accumulate)
 {
     return precision != LOFAR_FP64 && !accumulate && grid_cfg() == 0;
@@ -1395,12 +1734,13 @@ static void launch_degrid(int precision, const Geometry& g, const Buckets& b, co
                           const void* cube, const float* weight, long long F, long long P,
                           void* mre, void* mim, hipStream_t st)
 {
+    const dim3 grid((unsigned)(b.map.nbuckets() + b.heavy.max_pieces));
     if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL((k_degrid_tiles<WIN, true>), dim3((unsigned)b.map.nbuckets()), dim3(256), 0, st, g,
-                           b.map, b.offsets, ents, cube, weight, F, P, mre, mim);
+        hipLaunchKernelGGL((k_degrid_tiles<WIN, true>), grid, dim3(256), 0, st, g, b.map,
+                           b.offsets, ents, cube, weight, F, P, mre, mim, b.heavy);
     else
-        hipLaunchKernelGGL((k_degrid_tiles<WIN, false>), dim3((unsigned)b.map.nbuckets()), dim3(256), 0, st, g,
-                           b.map, b.offsets, ents, cube, weight, F, P, mre, mim);
+        hipLaunchKernelGGL((k_degrid_tiles<WIN, false>), grid, dim3(256), 0, st, g, b.map,
+                           b.offsets, ents, cube, weight, F, P, mre, mim, b.heavy);
 }
 
 hipError_t degrid_tiles(int precision, const Geometry& g, const Buckets& b, const DEntry* ents,

@@ -185,6 +185,36 @@ struct alignas(32) L2Block {
     long long k1, beg, end, pad;
 };
 
+// Dense tiles (more than `min` entries), split into pieces of `piece` entries that
+// workgroups of their own take: an array with a dense core puts a third of its samples into
+// a few tiles, and one workgroup each would outlast all others together.  The sort lists
+// the tiles (bucket, entries) and their pieces (tile, number); the gridder keeps a state and
+// 2*64*64 words of sums per tile.
+struct alignas(32) HeavyTile {
+    long long bkt, beg, end;
+    int np, pad;  // pieces
+};
+struct HeavyState {
+    unsigned long long m;  // bits of the largest |vis| component (a double)
+    double sa;             // sum of the |vis| components
+    unsigned nonfinite, done;
+    unsigned long long blk[256];  // FP64: entries touching each 4x4 block; FP32C: bound words
+};
+struct Heavy {
+    long long min = 0x7fffffffffffffffLL;  // no tile is split
+    int piece = 0;
+    HeavyTile* tile = nullptr;
+    int2* piece_of = nullptr;    // (tile, number) of every piece
+    int* count = nullptr;        // tiles, pieces
+    HeavyState* state = nullptr; // gridding
+    unsigned long long* acc = nullptr;
+    long long max_tiles = 0, max_pieces = 0;  // what the tables hold (host)
+};
+// Entries above which a tile is split, and per piece: 4096 of the FP64 gridder's 98 LDS
+// atomics are about 40 us of one CU, as are 8192 of the packed FP32C one's 49; a degridding
+// piece of 2048 takes about 10 us.  Merging a piece costs up to 8192 global atomics.
+constexpr int kHeavyFp64 = 4096, kHeavyFp32 = 8192, kHeavyHome = 2048;
+
 // Workspace of one bucketing of n samples (two-level counting sort).  Level 1
 // writes one record per (sample, super-tile its window touches), level 2
 // expands every record into one entry per tile of its window in the super-tile.
@@ -208,6 +238,7 @@ struct Buckets {
     void* zero;            // err, count1, count1e: nzero words to clear before the count
     long long nzero;
     volatile long long* status;  // host memory: entry total, validation flag, call number
+    Heavy heavy;                 // dense tiles, listed by the sort
     // level 2
     long long l2_block;       // records per level-2 block
     long long* l2_boff;       // [nk1+1] first block of each segment; [nk1] = block count
@@ -256,6 +287,8 @@ hipError_t bucket_sort_home(long long n, const double* uu, const double* vv, con
 // left unwritten (for a consumer that reads them as zeros).
 // sm_log >= 0 (without accumulate): the cube is written strip-major, each plane
 // [nx/L][ny][L] with L = 2^sm_log columns per strip.
+// whether grid_tiles splits dense tiles (b.heavy; the fixed-point kernels do)
+bool grid_splits(int precision, int accumulate);
 // whether grid_tiles takes index entries with b.vis (the packed FP32C kernel)
 bool grid_gathers(int precision, int accumulate);
 hipError_t grid_tiles(int precision, const Geometry& g, const Buckets& b, const void* entries,
