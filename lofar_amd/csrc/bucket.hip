@@ -20,6 +20,9 @@
 // Entries are self-contained (no side arrays), so every scattered write is one
 // aligned 16- or 32-byte store.
 //
+// A plan of few tiles (kStageMaxBins in all) is sorted by level 1 alone, with tiles for
+// super-tiles.
+//
 // Both scatters run staged where their bins fit one per thread (level 1 up to
 // kStageMaxBins super-tiles, level 2 always): a round's records are counted, scanned
 // and placed in an LDS buffer in bin order, then stored with consecutive lanes on
@@ -145,17 +148,50 @@ __device__ __forceinline__ T block_exscan(T v, T* wsum, T& total)
     return pre + x - v;
 }
 
+// Lists a dense tile and its pieces; the tile's place in the list is left in slots.
+__device__ __forceinline__ void list_heavy(const Heavy& h, long long bkt, long long beg,
+                                           long long n, int* slots, int* nslots)
+{
+    const int np = (int)((n + h.piece - 1) / h.piece);
+    const int t = atomicAdd(&h.count[0], 1), p0 = atomicAdd(&h.count[1], np);
+    HeavyTile d;
+    d.bkt = bkt;
+    d.beg = beg;
+    d.end = beg + n;
+    d.np = np;
+    d.pad = 0;
+    h.tile[t] = d;
+    for (int i = 0; i < np; i++) h.piece_of[p0 + i] = int2{t, i};
+    slots[atomicAdd(nslots, 1)] = t;
+}
+
+// Clears the states of the workgroup's listed tiles.
+template <int NT>
+__device__ __forceinline__ void clear_heavy(const Heavy& h, const int* slots, int nslots)
+{
+    if (!h.state) return;
+    constexpr int W = sizeof(HeavyState) / 4;
+    for (int i = threadIdx.x; i < nslots * W; i += NT)
+        ((unsigned*)&h.state[slots[i / W]])[i % W] = 0u;
+}
+
 // One workgroup: record, entry and level-2 block offsets of every super-tile, the block
 // table, and the call's status (entry total, validation flag, then seq, which the host waits
 // for) straight into host memory.  Nine scan launches and a copy took 45 us of a small
-// image's 220; this takes about 5 up to 8192 super-tiles.
+// image's 220; this takes about 5 up to 8192 super-tiles.  boff null: one level, the
+// super-tiles are the tiles; dense ones are listed here, and the largest count goes to the
+// host.
 __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned* count1,
                                                   const unsigned* count1e, long long* off1,
                                                   long long* eoff1, long long bs, long long* boff,
                                                   L2Block* blk, const int* err,
-                                                  volatile long long* status, long long seq)
+                                                  volatile long long* status, long long seq,
+                                                  Heavy h)
 {
     __shared__ long long ws[3][1024 / 64];
+    __shared__ int hslot[1024], hn;
+    __shared__ unsigned top;
+    if (threadIdx.x == 0) top = 0u;
     const int tid = threadIdx.x, lane = tid & 63;
     long long crec = 0, cent = 0, cblk = 0;
     for (long long c0 = 0; c0 < nk1; c0 += 1024) {
@@ -171,7 +207,14 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
             off1[k] = rec;
             eoff1[k] = ent;
         }
-        if (boff) {
+        if (!boff) {
+            if (tid == 0) hn = 0;
+            __syncthreads();
+            if (e > 0) atomicMax(&top, (unsigned)e);
+            if (e > h.min) list_heavy(h, k, ent, e, hslot, &hn);
+            __syncthreads();
+            clear_heavy<1024>(h, hslot, hn);
+        } else {
             if (k < nk1) boff[k] = b0;
             // block descriptors: the wave writes each of its lanes' segments together
             for (unsigned long long m = __ballot(nb > 0); m; m &= m - 1) {
@@ -199,6 +242,7 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
         if (boff) boff[nk1] = cblk;
         status[0] = cent;
         status[1] = *err;
+        status[3] = top;
         __threadfence_system();
         status[2] = seq;
     }
@@ -213,10 +257,22 @@ template <typename Rec, bool IDX>
 __device__ __forceinline__ Rec make_record(const Entry64& e, const TileMap& tm, int sv, int su,
                                            long long i)
 {
-    if constexpr (sizeof(Rec) == sizeof(Rec32)) {
+    if constexpr (std::is_same<Rec, Rec32>::value) {
         Rec32 r;
         r.u = rec_axis(e.pu, (su << tm.lsst) * kTile, tm.rfb);
         r.v = rec_axis(e.pv, (sv << tm.lsst) * kTile, tm.rfb);
+        r.vr = IDX ? __uint_as_float((unsigned)i) : (float)e.vr;
+        r.vi = (float)e.vi;
+        return r;
+    } else if constexpr (std::is_same<Rec, Entry32>::value) {
+        // one level: the entry of tile (sv, su), through the record's rounded position, so
+        // that both sorts give the same bits
+        const int u0 = su * kTile, v0 = sv * kTile;
+        const double pu = rec_pos(rec_axis(e.pu, u0, tm.rfb), u0, tm.rfb);
+        const double pv = rec_pos(rec_axis(e.pv, v0, tm.rfb), v0, tm.rfb);
+        Entry32 r;
+        r.wu = pack_cell((int)pu - u0, pu - (double)(int)pu);
+        r.wv = pack_cell((int)pv - v0, pv - (double)(int)pv);
         r.vr = IDX ? __uint_as_float((unsigned)i) : (float)e.vr;
         r.vi = (float)e.vi;
         return r;
@@ -227,8 +283,8 @@ __device__ __forceinline__ Rec make_record(const Entry64& e, const TileMap& tm, 
     }
 }
 
-// Rec: Entry64 (FP64 mode) or Rec32 (FP32 mode, position relative to the
-// super-tile, rec_axis)
+// Rec: Entry64 (FP64 mode), Rec32 (FP32 mode, position relative to the super-tile,
+// rec_axis) or Entry32 (FP32 mode, one level)
 // GLOBAL: base1 is one global cursor per super-tile (zeroed), taken with global atomics.
 // IDX: the records carry the sample's index (bits of the real part's slot, entry_index)
 // instead of its visibility, for a sort kept across calls (plan_fill).
@@ -592,33 +648,6 @@ __global__ __launch_bounds__(256) void k_l2_count(Geometry g, TileMap tm, const 
     for (int f = tid; f < nf; f += 256) cnt2[b * nf + f] = cnt[f];
 }
 
-// Lists a dense tile and its pieces; the tile's place in the list is left in slots.
-__device__ __forceinline__ void list_heavy(const Heavy& h, long long bkt, long long beg,
-                                           long long n, int* slots, int* nslots)
-{
-    const int np = (int)((n + h.piece - 1) / h.piece);
-    const int t = atomicAdd(&h.count[0], 1), p0 = atomicAdd(&h.count[1], np);
-    HeavyTile d;
-    d.bkt = bkt;
-    d.beg = beg;
-    d.end = beg + n;
-    d.np = np;
-    d.pad = 0;
-    h.tile[t] = d;
-    for (int i = 0; i < np; i++) h.piece_of[p0 + i] = int2{t, i};
-    slots[atomicAdd(nslots, 1)] = t;
-}
-
-// Clears the states of the workgroup's listed tiles.
-template <int NT>
-__device__ __forceinline__ void clear_heavy(const Heavy& h, const int* slots, int nslots)
-{
-    if (!h.state) return;
-    constexpr int W = sizeof(HeavyState) / 4;
-    for (int i = threadIdx.x; i < nslots * W; i += NT)
-        ((unsigned*)&h.state[slots[i / W]])[i % W] = 0u;
-}
-
 // one workgroup per segment, one fine tile per thread: running sums over the segment's
 // blocks (replacing the counts by block bases relative to the segment's first
 // entry), then the exclusive scan over fine tiles gives the bucket offsets.  The blocks'
@@ -828,7 +857,8 @@ hipError_t bucket_count(int mode, long long n, const double* uu, const double* v
 hipError_t bucket_scan(const Buckets& b, long long seq, hipStream_t st)
 {
     hipLaunchKernelGGL(k_l1_scan, dim3(1), dim3(1024), 0, st, b.map.nk1, b.count1, b.count1e,
-                       b.off1, b.eoff1, b.l2_block, b.l2_boff, b.l2_blk, b.err, b.status, seq);
+                       b.off1, b.eoff1, b.l2_block, b.one_level ? nullptr : b.l2_boff, b.l2_blk,
+                       b.err, b.status, seq, b.one_level ? b.heavy : Heavy());
     return hipGetLastError();
 }
 
@@ -859,18 +889,20 @@ static void launch_l1_scatter_grid(bool global_l1, bool index_vis, size_t lds, h
                                    const float* vi, const float* wt, const Geometry& g,
                                    const Buckets& b, Rec* rec)
 {
-    if ((b.stage & kStageL1) && !global_l1) {
+    if (((b.stage & kStageL1) && !global_l1) || std::is_same<Rec, Entry32>::value) {
         auto k = index_vis ? k_l1_scatter_staged<Rec, true> : k_l1_scatter_staged<Rec, false>;
         hipLaunchKernelGGL(k, dim3((unsigned)b.nwg), dim3(kStageThreads), 0, st, n, F, P, uu, vv,
                            ww, vr, vi, wt, g, b.map, b.chunk, b.off1, b.base1, rec);
         return;
     }
-    auto k = global_l1 ? (index_vis ? k_l1_scatter_grid<Rec, true, true>
-                                    : k_l1_scatter_grid<Rec, true, false>)
-                       : (index_vis ? k_l1_scatter_grid<Rec, false, true>
-                                    : k_l1_scatter_grid<Rec, false, false>);
-    hipLaunchKernelGGL(k, dim3((unsigned)b.nwg), dim3(256), lds, st, n, F, P, uu, vv, ww, vr, vi,
-                       wt, g, b.map, b.chunk, b.off1, b.base1, rec);
+    if constexpr (!std::is_same<Rec, Entry32>::value) {
+        auto k = global_l1 ? (index_vis ? k_l1_scatter_grid<Rec, true, true>
+                                        : k_l1_scatter_grid<Rec, true, false>)
+                           : (index_vis ? k_l1_scatter_grid<Rec, false, true>
+                                        : k_l1_scatter_grid<Rec, false, false>);
+        hipLaunchKernelGGL(k, dim3((unsigned)b.nwg), dim3(256), lds, st, n, F, P, uu, vv, ww, vr,
+                           vi, wt, g, b.map, b.chunk, b.off1, b.base1, rec);
+    }
 }
 
 hipError_t bucket_sort_grid(int precision, long long n, long long F, long long P,
@@ -882,6 +914,15 @@ hipError_t bucket_sort_grid(int precision, long long n, long long F, long long P
     if (n > 0 && b.global_l1) {
         hipError_t e = fill_u32(b.base1, b.map.nk1, 0u, st);
         if (e != hipSuccess) return e;
+    }
+    if (b.one_level) {
+        if (n > 0 && precision == LOFAR_FP64)
+            launch_l1_scatter_grid<Entry64>(false, index_vis, lds, st, n, F, P, uu, vv, ww, vr, vi,
+                                            wt, g, b, (Entry64*)entries);
+        else if (n > 0)
+            launch_l1_scatter_grid<Entry32>(false, index_vis, lds, st, n, F, P, uu, vv, ww, vr, vi,
+                                            wt, g, b, (Entry32*)entries);
+        return hipGetLastError();
     }
     if (precision == LOFAR_FP64) {
         if (n > 0)
@@ -977,6 +1018,7 @@ hipError_t bucket_sort_home(long long n, const double* uu, const double* vv, con
                             const float* wt1, const Geometry& g, const Buckets& b, DEntry* rec,
                             DEntry* entries, hipStream_t st)
 {
+    if (b.one_level) rec = entries;
     if (n > 0 && b.global_l1) {
         hipError_t e = fill_u32(b.base1, b.map.nk1, 0u, st);
         if (e != hipSuccess) return e;
@@ -990,6 +1032,7 @@ hipError_t bucket_sort_home(long long n, const double* uu, const double* vv, con
                            (size_t)b.map.nk1 * sizeof(unsigned), st, n, uu, vv, ww, wt1, g,
                            b.map, b.chunk, b.off1, b.base1, rec);
     }
+    if (b.one_level) return hipGetLastError();
     return level2<kOutHome>(g, b, (const DEntry*)rec, entries, st);
 }
 

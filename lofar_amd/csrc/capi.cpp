@@ -577,6 +577,7 @@ int tile_order_log(const TileMap& m)
 // bytes needed; with base set, assigns the pointer.
 size_t level2_layout(Buckets& b, long long total, char* base)
 {
+    if (b.one_level) return 0;
     b.l2_max_blocks = (total + b.l2_block - 1) / b.l2_block + b.map.nk1;
     const size_t nf = (size_t)b.map.sst * b.map.sst;
     if (base) b.l2_cnt = (unsigned*)base;
@@ -629,12 +630,18 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     };
     while (sst < 16 && super_tiles(sst) > kMaxSuperTiles) sst *= 2;  // large grids
     TileMap& m = b.map;
+    m.rfb = rec_fraction_bits(sst);
+    // Few tiles: level 1 alone sorts into them (positions rounded as the two levels' records
+    // are).  Two levels cost three more launches: 15-33 us each at 20000 samples, and the
+    // records' write and two reads where there are many.
+    b.one_level = (cfg.stage & kStageL1) && !cfg.forced &&
+                  super_tiles(1) <= std::min((long long)kStageMaxBins, l1_lds_max());
+    if (b.one_level) sst = 1;
     m.sst = sst;
     m.lsst = 0;
     while ((1 << m.lsst) < sst) m.lsst++;
     m.nstu = (g.ntu + sst - 1) / sst;
     m.nstv = (g.ntv + sst - 1) / sst;
-    m.rfb = rec_fraction_bits(sst);
     m.nk1 = super_tiles(sst);
     m.olog = tile_order_log(m);
     // beyond the LDS histograms' capacity, level 1 counts and places records with global
@@ -656,7 +663,8 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     const size_t off_l2boff = align256(off_offsets + (size_t)(m.nbuckets() + 1) * sizeof(long long));
     const size_t off_l2blk = align256(off_l2boff + (size_t)(m.nk1 + 1) * sizeof(long long));
     // a window (at most 17 cells) touches at most 4 super-tiles
-    const size_t max_blk = (size_t)((4LL * n + b.l2_block - 1) / b.l2_block + m.nk1);
+    const size_t max_blk =
+        b.one_level ? 0 : (size_t)((4LL * n + b.l2_block - 1) / b.l2_block + m.nk1);
     // Tables of the dense tiles (at most one entry per sample and touched tile).  The
     // allocation-free call does without: what fitted its array has to fit.
     Heavy& h = b.heavy;
@@ -669,7 +677,10 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     }
     const size_t off_htile = align256(off_l2blk + max_blk * sizeof(L2Block));
     const size_t off_hpiece = align256(off_htile + (size_t)h.max_tiles * sizeof(HeavyTile));
-    const size_t bytes = align256(off_hpiece + (size_t)h.max_pieces * sizeof(int2));
+    // one level: the states are cleared before the total is known (at most kStageMaxBins)
+    const size_t off_hstate = align256(off_hpiece + (size_t)h.max_pieces * sizeof(int2));
+    const size_t nstate = b.one_level ? (size_t)h.max_tiles : 0;
+    const size_t bytes = align256(off_hstate + nstate * sizeof(HeavyState));
     char* base = nullptr;
     int r = take(c, ar, c.meta, bytes, &base);
     if (r) return r;
@@ -687,6 +698,8 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     h.tile = (HeavyTile*)(base + off_htile);
     h.piece_of = (int2*)(base + off_hpiece);
     h.count = (int*)(base + off_hcount);
+    if (nstate > 0) h.state = (HeavyState*)(base + off_hstate);
+    if (b.one_level) b.offsets = b.off1;
     b.status = c.status_host;
     const long long seq = ++c.status_seq;
     HIPCHK(stage(c, kStCount, st,
@@ -705,10 +718,11 @@ int build_buckets(DeviceCtx& c, int mode, long n, const double* uu, const double
     total = c.status_host[0];
     if (h.max_pieces > 0) {
         h.max_tiles = std::min(total / h.min, h.max_tiles);
+        if (b.one_level && c.status_host[3] <= h.min) h.max_tiles = 0;
         h.max_pieces = h.max_tiles > 0 ? total / h.piece + h.max_tiles : 0;
     }
     // the block table was sized for any sample positions: give back what these cannot use
-    if (ar && ar->base) {
+    if (ar && ar->base && !b.one_level) {
         const size_t used = (size_t)((total + b.l2_block - 1) / b.l2_block + m.nk1);
         ar->used -= bytes - align256(off_l2blk + used * sizeof(L2Block));
     }
@@ -835,12 +849,14 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     // level-1 records (at most one per entry), the sorted entries, then the
     // level-2 counts
     const size_t esz = precision == LOFAR_FP64 ? sizeof(Entry64) : sizeof(Entry32);
-    const size_t rbytes = align256((size_t)total * sizeof(Entry64));
+    const size_t rbytes = b.one_level ? 0 : align256((size_t)total * sizeof(Entry64));
     const size_t ebytes = align256((size_t)total * esz);
     const size_t l2 = level2_layout(b, total, nullptr);
-    // the dense tiles' states; their sums take the place of the records, which are no longer
-    // read when the gridder runs (32 bytes a record, at most 16 an entry of a dense tile)
-    const size_t hs = align256((size_t)b.heavy.max_tiles * sizeof(HeavyState));
+    // the dense tiles' states and sums.  With two levels the sums take the place of the
+    // records, which are no longer read when the gridder runs (32 bytes a record, at most 16
+    // an entry of a dense tile); with one the states stand already.
+    const size_t hs = b.one_level ? (size_t)b.heavy.max_tiles * 2 * kTile * kTile * 8
+                                  : align256((size_t)b.heavy.max_tiles * sizeof(HeavyState));
     char* eb = nullptr;
     r = take(c, ar, c.ents, rbytes + ebytes + l2 + hs + 256, &eb);
     if (r) return r;
@@ -850,8 +866,11 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     static_assert(2 * kTile * kTile * 8 <= kHeavyFp64 * (int)sizeof(Entry64) &&
                       kHeavyFp64 <= kHeavyFp32,
                   "a dense tile's sums fit its records");
-    if (b.heavy.max_tiles > 0) {
-        b.heavy.state = (HeavyState*)(eb + rbytes + ebytes + l2);
+    char* dense = eb + rbytes + ebytes + l2;
+    if (b.one_level) {
+        b.heavy.acc = (unsigned long long*)dense;
+    } else if (b.heavy.max_tiles > 0) {
+        b.heavy.state = (HeavyState*)dense;
         b.heavy.acc = (unsigned long long*)eb;
     }
     b.nent = total;

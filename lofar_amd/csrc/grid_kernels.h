@@ -224,6 +224,7 @@ struct Buckets {
     bool global_l1;        // level-1 histograms and cursors in global memory (more
                            // super-tiles than the LDS histograms hold)
     int stage;             // kStageL1 | kStageL2: scatters staged through LDS
+    bool one_level;        // level 1 sorts into tiles (sst 1): its records are the entries
     unsigned* count1;      // [nk1] records per super-tile
     long long* off1;       // [nk1+1] record offsets
     unsigned* count1e;     // [nk1] entries per super-tile

@@ -34,3 +34,41 @@ def test_grid_and_degrid(cuda, n, nx, ny, nw):
     assert st == O.OK
     got = mr.cpu().numpy() + 1j * mi.cpu().numpy()
     assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+CHILD = r"""
+import hashlib, sys
+import numpy as np, torch
+from lofar_amd import imager
+rng = np.random.default_rng(5)
+n, nx, ny, nw = 30000, 200, 330, 4
+t = [torch.from_numpy(a).cuda() for a in (
+    rng.uniform(-0.01, 1.01, n), rng.uniform(-0.01, 1.01 * ny / nx, n), rng.uniform(0, 0.999, n),
+    rng.standard_normal(n).astype(np.float32), rng.standard_normal(n).astype(np.float32),
+    rng.uniform(0.5, 1.5, n).astype(np.float32))]
+for p in ("fp64", "fp32c"):
+    for support in (7, 17):
+        c = imager.grid(*t, nw, support, nx, ny, precision=p)
+        print(p, support, hashlib.sha256(c.cpu().numpy().tobytes()).hexdigest())
+"""
+
+
+def test_one_level_sort_gives_the_two_level_bits(cuda):
+    """Few tiles are sorted by level 1 alone; LOFAR_BUCKET_CFG keeps both levels."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    outs = []
+    for cfg in (None, "16,16384,8192", "2,1000,300"):
+        env = dict(os.environ, PYTHONPATH=root)
+        if cfg:
+            env["LOFAR_BUCKET_CFG"] = cfg
+        r = subprocess.run([sys.executable, "-c", CHILD], env=env, capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stderr[-2000:]
+        outs.append(r.stdout)
+    # FP32C positions are rounded to the super-tile side's bits: the default's and the first
+    # configuration's agree, the second's differ in FP32C only
+    assert outs[0] == outs[1]
+    assert outs[0].splitlines()[:2] == outs[2].splitlines()[:2]
