@@ -519,8 +519,19 @@ __device__ __forceinline__ void add_block_bound(unsigned long long* bsum, const 
     }
 }
 
-// One FP32C entry into the packed fixed-point tile at 2^S: the cells of its clipped
-// window.
+// Windows up to this side take all their columns in accumulate_pk32 (the others mask the
+// clipped ones: at 17 cells a quarter of the adds would be of zeros), and the words past a
+// tile that they reach.
+constexpr int kPkWhole = 9;
+constexpr int kPkPad = kPkWhole - 1;
+
+// One FP32C entry into the packed fixed-point tile at 2^S: the rows of its clipped window,
+// every column of the WIN at its first cell.  Columns past the clipped window have a zero
+// factor, whose contribution is the integer 0 (into the next row's words, or the kPkPad
+// words past the tile): a compare, a mask and a branch per cell cost more than the adds of
+// the 10 % of windows a tile's side clips.  A cell is two double FMAs, whose low words are
+// the rounded parts, and two integer operations: 64M samples on 4096x4096x32 took 2.65 ms
+// with a branch, a conversion and two more moves per cell, and take 2.58; with 9-cell windows 4.44 ms and 3.63.
 template <int WIN>
 __device__ __forceinline__ void accumulate_pk32(unsigned long long* acc, const Geometry& g, int u0,
                                                 int v0, double norm, double scale,
@@ -529,11 +540,11 @@ __device__ __forceinline__ void accumulate_pk32(unsigned long long* acc, const G
     const Win32 w32 = decode32(en, g, u0, v0);
     const int a0 = w32.t.a0, na = w32.t.na, b0 = w32.t.b0, nb = w32.t.nb;
     unsigned long long* base = &acc[b0 * kTile + a0];
-    float eu[WIN];
+    double eu[WIN];
 #pragma unroll
     for (int q = 0; q < WIN; q++) {
         const float du = (float)(w32.iu + q) + w32.hu;
-        eu[q] = (q <= na) ? expf(-(du * du) * 0.5f) : 0.0f;
+        eu[q] = (q <= na) ? (double)expf(-(du * du) * 0.5f) : 0.0;
     }
 #pragma unroll
     for (int kq = 0; kq < WIN; kq++) {
@@ -544,12 +555,10 @@ __device__ __forceinline__ void accumulate_pk32(unsigned long long* acc, const G
             unsigned long long* row = base + kq * kTile;
 #pragma unroll
             for (int q = 0; q < WIN; q++) {
-                if (q <= na) {
-                    const unsigned re = round_u32((double)eu[q] * fr);
-                    const unsigned im = round_u32((double)eu[q] * fi);
-                    atomicAdd(row + q, ((unsigned long long)re << 32) +
-                                           (unsigned long long)(long long)(int)im);
-                }
+                if (WIN > kPkWhole && q > na) continue;
+                const unsigned im = round_u32(eu[q] * fi);
+                const unsigned re = round_u32(eu[q] * fr) + (unsigned)((int)im >> 31);
+                atomicAdd(row + q, ((unsigned long long)re << 32) | im);
             }
         }
     }
@@ -898,7 +907,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, co
                                                        float2* cube, unsigned long long* occ,
                                                        int sm_log, Heavy h)
 {
-    __shared__ __align__(16) unsigned long long acc[kPlane];
+    __shared__ __align__(16) unsigned long long acc[kPlane + kPkPad];
     __shared__ unsigned long long bsum[kNBlk * kNBlk];
     __shared__ float wred[NT / 64];
     __shared__ double wsum[NT / 64];
@@ -1718,10 +1727,14 @@ hipError_t grid_tiles(int precision, const Geometry& g, const Buckets& b, const 
     // only the packed FP32C kernel gathers visibilities
     if (b.vis && !grid_gathers(precision, accumulate)) return hipErrorInvalidValue;
     const int win = 2 * g.K + 1;
-    if (win <= 7)
+    if (win <= 5)
+        launch_grid<5>(precision, g, b, entries, cube, accumulate, occ, sm_log, st);
+    else if (win <= 7)
         launch_grid<7>(precision, g, b, entries, cube, accumulate, occ, sm_log, st);
     else if (win <= 9)
         launch_grid<9>(precision, g, b, entries, cube, accumulate, occ, sm_log, st);
+    else if (win <= 13)
+        launch_grid<13>(precision, g, b, entries, cube, accumulate, occ, sm_log, st);
     else if (win <= kMaxTileWin)
         launch_grid<17>(precision, g, b, entries, cube, accumulate, occ, sm_log, st);
     else
@@ -1748,10 +1761,14 @@ hipError_t degrid_tiles(int precision, const Geometry& g, const Buckets& b, cons
                         void* mre, void* mim, hipStream_t st)
 {
     const int win = 2 * g.K + 1;
-    if (win <= 7)
+    if (win <= 5)
+        launch_degrid<5>(precision, g, b, ents, cube, weight, F, P, mre, mim, st);
+    else if (win <= 7)
         launch_degrid<7>(precision, g, b, ents, cube, weight, F, P, mre, mim, st);
     else if (win <= 9)
         launch_degrid<9>(precision, g, b, ents, cube, weight, F, P, mre, mim, st);
+    else if (win <= 13)
+        launch_degrid<13>(precision, g, b, ents, cube, weight, F, P, mre, mim, st);
     else if (win <= kMaxTileWin)
         launch_degrid<17>(precision, g, b, ents, cube, weight, F, P, mre, mim, st);
     else
