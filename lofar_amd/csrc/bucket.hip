@@ -191,8 +191,11 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
     __shared__ long long ws[3][1024 / 64];
     __shared__ int hslot[1024], hn;
     __shared__ unsigned top;
-    if (threadIdx.x == 0) top = 0u;
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        top = 0u;
+        hn = 0;
+    }
     long long crec = 0, cent = 0, cblk = 0;
     for (long long c0 = 0; c0 < nk1; c0 += 1024) {
         const long long k = c0 + tid;
@@ -206,36 +209,18 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
         if (k < nk1) {
             off1[k] = rec;
             eoff1[k] = ent;
+            if (boff) boff[k] = b0;
         }
         if (!boff) {
-            if (tid == 0) hn = 0;
-            __syncthreads();
             if (e > 0) atomicMax(&top, (unsigned)e);
             if (e > h.min) list_heavy(h, k, ent, e, hslot, &hn);
-            __syncthreads();
-            clear_heavy<1024>(h, hslot, hn);
-        } else {
-            if (k < nk1) boff[k] = b0;
-            // block descriptors: the wave writes each of its lanes' segments together
-            for (unsigned long long m = __ballot(nb > 0); m; m &= m - 1) {
-                const int src = __ffsll(m) - 1;
-                const long long sk = __shfl(k, src), sr = __shfl(rec, src), sn = __shfl(r, src);
-                const long long sb = __shfl(b0, src), snb = __shfl(nb, src);
-                for (long long j = lane; j < snb; j += 64) {
-                    L2Block d;
-                    d.k1 = sk;
-                    d.beg = sr + j * bs;
-                    d.end = sr + min(sn, (j + 1) * bs);
-                    d.pad = 0;
-                    blk[sb + j] = d;
-                }
-            }
         }
         crec += tr;
         cent += te;
         cblk += tb;
         __syncthreads();  // the wave sums are read: free for the next round
     }
+    // the status first: the host prepares the next launches while the rest is written
     if (tid == 0) {
         off1[nk1] = crec;
         eoff1[nk1] = cent;
@@ -245,6 +230,27 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
         status[3] = top;
         __threadfence_system();
         status[2] = seq;
+    }
+    if (!boff) {
+        clear_heavy<1024>(h, hslot, hn);
+        return;
+    }
+    // block descriptors, one thread each: its segment is the last that starts at or before it
+    for (long long j = tid; j < cblk; j += 1024) {
+        long long lo = 0, hi = nk1;  // boff[lo] <= j < boff[hi]
+        while (hi - lo > 1) {
+            const long long mid = (lo + hi) >> 1;
+            if (boff[mid] <= j)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        L2Block d;
+        d.k1 = lo;
+        d.beg = off1[lo] + (j - boff[lo]) * bs;
+        d.end = min(off1[lo + 1], d.beg + bs);
+        d.pad = 0;
+        blk[j] = d;
     }
 }
 
@@ -648,50 +654,66 @@ __global__ __launch_bounds__(256) void k_l2_count(Geometry g, TileMap tm, const 
     for (int f = tid; f < nf; f += 256) cnt2[b * nf + f] = cnt[f];
 }
 
-// one workgroup per segment, one fine tile per thread: running sums over the segment's
-// blocks (replacing the counts by block bases relative to the segment's first
-// entry), then the exclusive scan over fine tiles gives the bucket offsets.  The blocks'
-// counts are read 8 at a time: they come back to back instead of one latency each.  Dense
-// tiles are listed on the way (Heavy).
-__global__ __launch_bounds__(kMaxFine) void k_l2_scan(TileMap tm, const long long* eoff1,
-                                                      const long long* boff, unsigned* cnt2,
-                                                      long long* offsets, Heavy h)
+// One workgroup per segment: per fine tile, running sums over the segment's blocks (replacing
+// the counts by block bases relative to the segment's first entry); the exclusive scan over
+// fine tiles gives the bucket offsets.  Four groups of threads, a tile per thread, take a
+// quarter of the blocks each and read G blocks' counts at a time (kept for the write where
+// they are all): few segments with many blocks were 16 serial round trips, 25 us of a
+// 1M-sample image.  Dense tiles are listed on the way (Heavy).
+__global__ __launch_bounds__(4 * kMaxFine) void k_l2_scan(TileMap tm, const long long* eoff1,
+                                                          const long long* boff, unsigned* cnt2,
+                                                          long long* offsets, Heavy h)
 {
-    __shared__ unsigned ws[kMaxFine / 64];
+    __shared__ unsigned part[4][kMaxFine], tile0[kMaxFine], ws[4 * kMaxFine / 64];
     __shared__ int hslot[kMaxFine], hn;
-    constexpr int G = 8;
-    const int f = threadIdx.x;
+    constexpr int G = 16;
+    const int f = threadIdx.x % kMaxFine, grp = threadIdx.x / kMaxFine;
     const int nf = tm.sst * tm.sst;
     const long long k1 = blockIdx.x;
-    const long long b0 = boff[k1], b1 = boff[k1 + 1];
+    const long long s0 = boff[k1], s1 = boff[k1 + 1], q = (s1 - s0 + 3) / 4;
+    const long long b0 = min(s1, s0 + grp * q), b1 = min(s1, b0 + q);
     const bool on = f < nf;
-    unsigned tot = 0;
+    const bool whole = q <= G;  // one read of the counts
+    unsigned c[G], tot = 0;
     for (long long j = b0; j < b1; j += G) {
-        unsigned c[G];
 #pragma unroll
         for (int i = 0; i < G; i++) c[i] = on && j + i < b1 ? cnt2[(j + i) * nf + f] : 0u;
 #pragma unroll
         for (int i = 0; i < G; i++) tot += c[i];
     }
-    unsigned all;
-    unsigned run = block_exscan<kMaxFine>(tot, ws, all);
-    if (on) offsets[k1 * nf + f] = eoff1[k1] + run;
-    if (f == 0) hn = 0;
+    part[grp][f] = tot;
+    if (threadIdx.x == 0) hn = 0;
     __syncthreads();
-    if (on && (long long)tot > h.min) list_heavy(h, k1 * nf + f, eoff1[k1] + run, tot, hslot, &hn);
-    __syncthreads();
-    clear_heavy<kMaxFine>(h, hslot, hn);
-    for (long long j = b0; j < b1; j += G) {
-        unsigned c[G];
+    unsigned all = 0, before = 0;  // the tile's entries, and those of the groups before
 #pragma unroll
-        for (int i = 0; i < G; i++) c[i] = on && j + i < b1 ? cnt2[(j + i) * nf + f] : 0u;
+    for (int i = 0; i < 4; i++) {
+        const unsigned x = part[i][f];
+        before += i < grp ? x : 0u;
+        all += x;
+    }
+    unsigned sum;
+    const unsigned run0 = block_exscan<4 * kMaxFine>(grp == 0 ? all : 0u, ws, sum);
+    if (grp == 0) {
+        tile0[f] = run0;
+        if (on) offsets[k1 * nf + f] = eoff1[k1] + run0;
+        if (on && (long long)all > h.min)
+            list_heavy(h, k1 * nf + f, eoff1[k1] + run0, all, hslot, &hn);
+    }
+    __syncthreads();
+    clear_heavy<4 * kMaxFine>(h, hslot, hn);
+    unsigned run = tile0[f] + before;
+    for (long long j = b0; j < b1; j += G) {
+        if (!whole) {
+#pragma unroll
+            for (int i = 0; i < G; i++) c[i] = on && j + i < b1 ? cnt2[(j + i) * nf + f] : 0u;
+        }
 #pragma unroll
         for (int i = 0; i < G; i++) {
             if (on && j + i < b1) cnt2[(j + i) * nf + f] = run;
             run += c[i];
         }
     }
-    if (k1 == 0 && f == 0) offsets[tm.nk1 * nf] = eoff1[tm.nk1];
+    if (k1 == 0 && threadIdx.x == 0) offsets[tm.nk1 * nf] = eoff1[tm.nk1];
 }
 
 // The entry of record x (window s) for fine tile (fv, fu) of super-tile (sv, su).
@@ -871,7 +893,7 @@ static hipError_t level2(const Geometry& g, const Buckets& b, const Rec* rec, Ou
     const long long* nblocks = b.l2_boff + nk1;
     hipLaunchKernelGGL((k_l2_count<OUT, Rec>), dim3(grid), dim3(256), 0, st, g, b.map, nblocks,
                        b.l2_blk, rec, b.l2_cnt);
-    hipLaunchKernelGGL(k_l2_scan, dim3((unsigned)nk1), dim3(kMaxFine), 0, st, b.map, b.eoff1, b.l2_boff,
+    hipLaunchKernelGGL(k_l2_scan, dim3((unsigned)nk1), dim3(4 * kMaxFine), 0, st, b.map, b.eoff1, b.l2_boff,
                        b.l2_cnt, b.offsets, b.heavy);
     if (b.stage & kStageL2)
         hipLaunchKernelGGL((k_l2_scatter_staged<OUT, Rec, Out>), dim3(grid), dim3(kStageThreads),
