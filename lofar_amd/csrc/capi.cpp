@@ -383,11 +383,11 @@ int take(DeviceCtx& c, Arena* ar, Buffer& b, size_t bytes, char** out)
     return LOFAR_OK;
 }
 
-// exp(+2*pi*i*m/N), m < N, from long double arithmetic, rounded once; mixed: in the order
-// of the mixed-radix transforms' stages
-int twiddles(DeviceCtx& c, int n, int precision, void** out, bool mixed = false)
+// Twiddle table of length n (stage_twiddle_order with rx), from long double arithmetic,
+// rounded once
+int twiddles(DeviceCtx& c, int n, int precision, int rx, void** out)
 {
-    const long long key = (long long)n * 4 + (mixed ? 2 : 0) + precision;
+    const long long key = ((long long)n * 32 + rx) * 2 + precision;
     auto it = c.twiddles.find(key);
     if (it != c.twiddles.end()) {
         *out = it->second;
@@ -395,8 +395,7 @@ int twiddles(DeviceCtx& c, int n, int precision, void** out, bool mixed = false)
     }
     std::vector<double> tw(2 * (size_t)n);
     std::vector<int> order(n);
-    for (int i = 0; i < n; i++) order[i] = i;
-    if (mixed && !mixed_twiddle_order(n, order.data())) return fail(LOFAR_ESIZE);
+    if (!stage_twiddle_order(n, rx, order.data())) return fail(LOFAR_ESIZE);
     const long double two_pi = 6.283185307179586476925286766559005768L;
     for (int i = 0; i < n; i++) {
         const long double a = two_pi * (long double)order[i] / (long double)n;
@@ -420,15 +419,14 @@ int twiddles(DeviceCtx& c, int n, int precision, void** out, bool mixed = false)
 
 // Twiddles of the allocation-free entry point: a slice of the static workspace
 // filled on the device (no allocation and no host copy).
-int twiddles_for(DeviceCtx& c, Arena* ar, int n, int precision, hipStream_t st, void** out,
-                 bool mixed = false)
+int twiddles_for(DeviceCtx& c, Arena* ar, int n, int precision, int rx, hipStream_t st, void** out)
 {
-    if (!ar || !ar->base) return twiddles(c, n, precision, out, mixed);
+    if (!ar || !ar->base) return twiddles(c, n, precision, rx, out);
     Buffer unused;
     char* p = nullptr;
     int r = take(c, ar, unused, (size_t)n * (precision == LOFAR_FP64 ? 16 : 8), &p);
     if (r) return r;
-    HIPCHK(mixed ? fill_mixed_twiddles(precision, n, p, st) : fill_twiddles(precision, n, p, st));
+    HIPCHK(fill_stage_twiddles(precision, n, rx, p, st));
     *out = p;
     return LOFAR_OK;
 }
@@ -475,9 +473,9 @@ int fft_generic_planes(DeviceCtx& c, Arena* ar, int precision, int sign, const v
                        bool rows_first = false)
 {
     void *twx, *twy;
-    int r = twiddles_for(c, ar, nx, precision, st, &twx, true);
+    int r = twiddles_for(c, ar, nx, precision, 0, st, &twx);
     if (r) return r;
-    r = twiddles_for(c, ar, ny, precision, st, &twy, true);
+    r = twiddles_for(c, ar, ny, precision, 0, st, &twy);
     if (r) return r;
     auto cols = [&](const void* src) {
         return precision == LOFAR_FP64
@@ -892,9 +890,9 @@ int fft_impl(DeviceCtx& c, int precision, int sign, const void* in, void* out, i
     if (!pow2_ok(nx) || !pow2_ok(ny))
         return fft_generic_planes(c, nullptr, precision, sign, in, out, nx, ny, nw, scale, st);
     void *twx, *twy;
-    int r = twiddles(c, nx, precision, &twx);
+    int r = twiddles(c, nx, precision, 16, &twx);
     if (r) return r;
-    r = twiddles(c, ny, precision, &twy);
+    r = twiddles(c, ny, precision, 16, &twy);
     if (r) return r;
     const long long lines = (long long)nw * ny;
     if (precision == LOFAR_FP64) {
@@ -1158,9 +1156,9 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
         return LOFAR_OK;
     }
     void *twx, *twy;
-    r = twiddles_for(c, ar, grid_size_x, precision, st, &twx);
+    r = twiddles_for(c, ar, grid_size_x, precision, split ? 16 : 8, st, &twx);
     if (r) return r;
-    r = twiddles_for(c, ar, grid_size_y, precision, st, &twy);
+    r = twiddles_for(c, ar, grid_size_y, precision, 16, st, &twy);
     if (r) return r;
     const PhaseParams pp =
         phase_params(num_w_planes, grid_size_x, grid_size_y, resolution, wmin, wmax);
@@ -1301,11 +1299,6 @@ static int degrid_transform(DeviceCtx& c, hipStream_t st, int precision, int num
                             void* cube, const unsigned long long* need = nullptr)
 {
     int r = LOFAR_OK;
-    void *twx, *twy;
-    r = twiddles(c, grid_size_x, precision, &twx);
-    if (r) return r;
-    r = twiddles(c, grid_size_y, precision, &twy);
-    if (r) return r;
     const PhaseParams pp =
         phase_params(num_w_planes, grid_size_x, grid_size_y, resolution, wmin, wmax);
     const double scale = 1.0 / ((double)grid_size_x * (double)grid_size_y);
@@ -1319,8 +1312,15 @@ static int degrid_transform(DeviceCtx& c, hipStream_t st, int precision, int num
         }));
         r = fft_generic_planes(c, nullptr, precision, -1, cube, cube, grid_size_x,
                                grid_size_y, num_w_planes, scale, st, true);
-        if (r) return r;
-    } else if (grid_size_x >= 8192 && rows_split()) {
+        return r;
+    }
+    const bool split = grid_size_x >= 8192 && rows_split();
+    void *twx, *twy;
+    r = twiddles(c, grid_size_x, precision, split ? 16 : 8, &twx);
+    if (r) return r;
+    r = twiddles(c, grid_size_y, precision, 16, &twy);
+    if (r) return r;
+    if (split) {
         // rows of 8192: the fused adjoint row pass does not fit its 1024-thread
         // workgroups' registers, so the conjugate screen (every plane written) and
         // the forward row transform (in place) run as two passes

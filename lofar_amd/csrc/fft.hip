@@ -526,16 +526,6 @@ static hipError_t launch_cols_n(int sign, const void* in, void* out, const void*
     }
 }
 
-static int phase_cfg()
-{
-    static int cfg = -1;
-    if (cfg < 0) {
-        const char* s = getenv("LOFAR_PHASE_CFG");
-        cfg = s ? atoi(s) : 0;
-    }
-    return cfg;
-}
-
 template <typename Real, int N, int E, bool RECUR, bool TWREG, bool PF = false>
 static hipError_t launch_rows_phase_cfg(const void* cube, const void* tw, int ny, int nw,
                                         const PhaseParams& pp, double scale, double* re,
@@ -556,26 +546,17 @@ static hipError_t launch_rows_phase_cfg(const void* cube, const void* tw, int ny
     return hipGetLastError();
 }
 
-// fused row-pass configurations (elements per thread, phase recurrence or direct
-// sincos, twiddles in registers, next row prefetched into LDS); entry 0 is the
-// default
+// the fused row pass: 8 elements per thread, phase recurrence, twiddles in registers, next
+// row prefetched into LDS where it fits
 template <typename Real, int N>
 static hipError_t launch_rows_phase_n(const void* cube, const void* tw, int ny, int nw,
                                       const PhaseParams& pp, double scale, double* re, double* im,
                                       int accumulate, int sm_log, hipStream_t st)
 {
 #define ARGS_ cube, tw, ny, nw, pp, scale, re, im, accumulate, sm_log, st
-    switch (phase_cfg()) {
-        case 1: return launch_rows_phase_cfg<Real, N, 8, false, true>(ARGS_);
-        case 2: return launch_rows_phase_cfg<Real, N, 8, true, false>(ARGS_);
-        case 3: return launch_rows_phase_cfg<Real, N, 16, true, true>(ARGS_);
-        case 4: return launch_rows_phase_cfg<Real, N, 4, true, true>(ARGS_);
-        case 5: return launch_rows_phase_cfg<Real, N, 8, true, true>(ARGS_);
-        default:
-            return launch_rows_phase_cfg<Real, N, 8, true, true,
-                                         (Plan<N, 8>::TPL >= 64 &&
-                                          rows_prefetch_fits<Real, N, 8>())>(ARGS_);
-    }
+    return launch_rows_phase_cfg<Real, N, 8, true, true,
+                                 (Plan<N, 8>::TPL >= 64 && rows_prefetch_fits<Real, N, 8>())>(
+        ARGS_);
 #undef ARGS_
 }
 
@@ -645,26 +626,6 @@ hipError_t rows_phase_adj(void* cube, const void* tw, int nx, int ny, int nw,
 #define CALL_(n) launch_rows_phase_adj_n<Real, n>(cube, tw, ny, nw, pp, scale, re, im, st)
     LOFAR_FFT_SWITCH(nx, CALL_)
 #undef CALL_
-}
-
-template <typename Real>
-__global__ __launch_bounds__(256) void k_twiddles(C2<Real>* tw, int n)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    double sn, cs;
-    sincospi(2.0 * (double)m / (double)n, &sn, &cs);
-    tw[m] = C2<Real>{(Real)cs, (Real)sn};
-}
-
-hipError_t fill_twiddles(int precision, int n, void* tw, hipStream_t st)
-{
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL((k_twiddles<double>), dim3(blocks), dim3(256), 0, st, (double2*)tw, n);
-    else
-        hipLaunchKernelGGL((k_twiddles<float>), dim3(blocks), dim3(256), 0, st, (float2*)tw, n);
-    return hipGetLastError();
 }
 
 int device_cus()

@@ -199,11 +199,19 @@ __device__ __forceinline__ void dft(T2* v)
 // lds[Plan<N,E>::pad(i)*ls] (Plan<N,E>::LDS slots per line).  With ROUNDS > 1
 // the lines of a workgroup take turns on a shared LDS buffer: a thread
 // exchanges in round my_round only (all threads pass every barrier).
-// Twiddles: tw[m] = exp(+2*pi*i*m/N), conjugated for SIGN < 0.
+// Twiddles: exp(+2*pi*i*q*k/(NS*R)) at stage_tw<P>(tw, NS)[(q-1)*NS + k] (the radix-RX order
+// of stage_twiddle_order), conjugated for SIGN < 0: the lanes of a wave hold consecutive k
+// and read runs of the table.  From one table in the order of m, every lane read a cache
+// line of its own: rows of 8192 complex floats spent as long on it as on their data.
 // RT: the twiddles of butterfly m are the powers w^q of one root per butterfly,
-// rt[m] = tw[k*N/(NS*R)] (load_roots), taken from registers loaded when the
+// rt[m] = the q = 1 entry (load_roots), taken from registers loaded when the
 // kernel starts instead of R-1 table loads at the stage (whose latency a stage
 // otherwise waits out); q-1 complex products per power, a few ulp in FP64.
+template <typename P, typename T2>
+__device__ __forceinline__ const T2* stage_tw(const T2* tw, int ns)
+{
+    return tw + (ns - P::R0);
+}
 template <typename T2, int N, int EREQ, int SIGN, int NS, int ROUNDS = 1, bool RT = false>
 __device__ __forceinline__ void stages(T2* v, T2* lds, int ls, int t, const T2* __restrict__ tw,
                                        int my_round = 0, const T2* rt = nullptr)
@@ -229,7 +237,8 @@ __device__ __forceinline__ void stages(T2* v, T2* lds, int ls, int t, const T2* 
                 const int k = b & (NS - 1);
 #pragma unroll
                 for (int q = 1; q < R; q++)
-                    v[m * R + q] = c_mul_tw<SIGN>(v[m * R + q], tw[q * k * (N / (NS * R))]);
+                    v[m * R + q] =
+                        c_mul_tw<SIGN>(v[m * R + q], stage_tw<P>(tw, NS)[(q - 1) * NS + k]);
             }
         }
         dft<R, SIGN>(&v[m * R]);
@@ -310,7 +319,7 @@ __device__ __forceinline__ void load_roots(T2* rt, int t, const T2* __restrict__
 #pragma unroll
         for (int m = 0; m < M; m++) {
             const int k = (t + m * P::TPL) & (NS - 1);
-            rt[m] = tw[k * (N / (NS * R))];
+            rt[m] = stage_tw<P>(tw, NS)[k];
         }
     }
     if constexpr (NS * R < N) load_roots<T2, N, EREQ, NS * R>(rt + (NS > 1 ? M : 0), t, tw);
@@ -344,7 +353,8 @@ __device__ __forceinline__ void load_twiddles(T2* twr, int t, const T2* __restri
         for (int m = 0; m < M; m++) {
             const int k = (t + m * P::TPL) & (NS - 1);
 #pragma unroll
-            for (int q = 1; q < R; q++) twr[m * (R - 1) + q - 1] = tw[q * k * (N / (NS * R))];
+            for (int q = 1; q < R; q++)
+                twr[m * (R - 1) + q - 1] = stage_tw<P>(tw, NS)[(q - 1) * NS + k];
         }
     }
     if constexpr (NS * R < N)
@@ -477,24 +487,27 @@ __device__ __forceinline__ void phase_rotation(const PhaseParams& pp, double fac
 // phase constants of phase_correction.cu:92-94 (phase.hip)
 PhaseParams phase_params(int nw, int xtot, int ytot, double resolution, double wmin, double wmax);
 
-// tw[m] = exp(+2*pi*i*m/n), m < n, computed on the device (sincospi in double, then
-// rounded to float for LOFAR_FP32C): the allocation-free entry point's twiddle tables
-hipError_t fill_twiddles(int precision, int n, void* tw, hipStream_t st);
+// Twiddle tables of n entries in the order the stages read them (fft_mixed.hip): entry i is
+// exp(2 pi i order[i]/n); (ns, R)'s entries [q-1][k] lie from ns - R0 on, R0 the first radix.
+// rx: the largest radix of a power of two (16, or 8 for the fused row passes), 0 for the
+// mixed-radix plan of n.  fill_stage_twiddles computes the same table on the device
+// (sincospi in double, then rounded to float for LOFAR_FP32C): the allocation-free entry
+// point's.
+bool stage_twiddle_order(int n, int rx, int* order);
+hipError_t fill_stage_twiddles(int precision, int n, int rx, void* tw, hipStream_t st);
 
 // Mixed-radix line transforms for sides that are not powers of two (prime factors at most
 // 13, side at most 8192; fft_mixed.hip): line l of `lines` starts at (l / per) * plane + (l %
 // per) * lstride, its elements estride apart (1: rows); out may alias in.  tw: the length's
-// table in the order of mixed_twiddle_order (n entries), or filled by fill_mixed_twiddles.
-// fft_size_ok: a side either the power-of-two kernels or these take.
-bool mixed_twiddle_order(int n, int* order);
-hipError_t fill_mixed_twiddles(int precision, int n, void* tw, hipStream_t st);
+// table with rx 0.  fft_size_ok: a side either the power-of-two kernels or these take.
 bool fft_size_ok(int n);
 template <typename Real>
 hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int n, long long lines,
                        long long per, long long plane, long long lstride, long long estride,
                        double scale, hipStream_t st);
 
-// host dispatch (fft.hip); all return hipErrorInvalidValue for unsupported sizes
+// host dispatch (fft.hip); all return hipErrorInvalidValue for unsupported sizes.  tw: the
+// line length's table with rx 16 (fft_rows, fft_cols) or 8 (rows_phase, rows_phase_adj).
 template <typename Real>
 hipError_t fft_rows(int sign, const void* in, void* out, const void* tw, int nx, long long lines,
                     double scale, hipStream_t st);

@@ -11,7 +11,7 @@
 // mod Ns, Ns the product of the radices before this stage) takes x[j + q*N/P], q < P, times
 // exp(2 pi i q k / (Ns P)), DFT over q, and gives y[(j - k)*P + k + r*Ns].  Each stage's
 // twiddles are laid out [q-1][k], so that a wave's butterflies read runs of the table
-// (mixed_twiddle_order; read from an N-entry table in order, every lane took a cache line of
+// (stage_twiddle_order; read from an N-entry table in order, every lane took a cache line of
 // its own); the small DFTs have their roots as constants
 // (odd primes by the even and odd parts of their inputs, half the products of the
 // definition).  Inverse signs swap the real and imaginary parts on the way in and out.
@@ -295,7 +295,7 @@ __device__ __forceinline__ void mix_stage(MixThread<Real, ROWS> m, int ns, unsig
     // of the switch that picks one (170-350 spilled registers)
     asm volatile("" : "+v"(m.j0), "+v"(m.l));
     const int nb = m.n / P;
-    const T2* tw = m.tw + (FIRST ? 0 : ns - m.r0);  // mixed_twiddle_order
+    const T2* tw = m.tw + (FIRST ? 0 : ns - m.r0);  // stage_twiddle_order
     if constexpr (FIRST || LAST) {
         if (m.active) {
 #pragma unroll 1
@@ -432,13 +432,26 @@ bool mixed_plan(int n, MixPlan& p)
     return true;
 }
 
-// Entry i of a mixed-radix length's table is exp(2 pi i order[i]/n): stage after stage (the
-// first has no twiddles), (ns, P)'s entries [q-1][k] from entry ns - radix[0] on (n -
-// radix[0] in all); the last radix[0] entries are unused.
-bool mixed_twiddle_order(int n, int* order)
+// stages of a table: the mixed-radix plan (rx 0), or radix rx and the remainder of a power of
+// two (Plan in fft_kernels.h)
+static bool table_plan(int n, int rx, MixPlan& p)
+{
+    if (rx == 0) return mixed_plan(n, p);
+    if (n < 2 || n > kMixMaxN || (n & (n - 1))) return false;
+    p.n = n;
+    p.nstages = 0;
+    for (int ns = 1; ns < n; ns *= p.radix[p.nstages++]) {
+        p.ns[p.nstages] = ns;
+        p.radix[p.nstages] = std::min(rx, n / ns);
+        p.magic[p.nstages] = 0u;
+    }
+    return true;
+}
+
+bool stage_twiddle_order(int n, int rx, int* order)
 {
     MixPlan p;
-    if (!mixed_plan(n, p)) return false;
+    if (!table_plan(n, rx, p)) return false;
     std::fill(order, order + n, 0);
     for (int s = 1; s < p.nstages; s++) {
         const int ns = p.ns[s], turn = n / (ns * p.radix[s]);
@@ -449,9 +462,8 @@ bool mixed_twiddle_order(int n, int* order)
     return true;
 }
 
-// the same table computed on the device (fill_twiddles' arithmetic)
 template <typename Real>
-__global__ __launch_bounds__(256) void k_mixed_twiddles(typename cplx<Real>::type* tw, MixPlan p)
+__global__ __launch_bounds__(256) void k_stage_twiddles(typename cplx<Real>::type* tw, MixPlan p)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.n) return;
@@ -466,15 +478,15 @@ __global__ __launch_bounds__(256) void k_mixed_twiddles(typename cplx<Real>::typ
     tw[i] = typename cplx<Real>::type{(Real)cs, (Real)sn};
 }
 
-hipError_t fill_mixed_twiddles(int precision, int n, void* tw, hipStream_t st)
+hipError_t fill_stage_twiddles(int precision, int n, int rx, void* tw, hipStream_t st)
 {
     MixPlan p;
-    if (!mixed_plan(n, p)) return hipErrorInvalidValue;
+    if (!table_plan(n, rx, p)) return hipErrorInvalidValue;
     const dim3 blocks((unsigned)((n + 255) / 256));
     if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL(k_mixed_twiddles<double>, blocks, dim3(256), 0, st, (double2*)tw, p);
+        hipLaunchKernelGGL(k_stage_twiddles<double>, blocks, dim3(256), 0, st, (double2*)tw, p);
     else
-        hipLaunchKernelGGL(k_mixed_twiddles<float>, blocks, dim3(256), 0, st, (float2*)tw, p);
+        hipLaunchKernelGGL(k_stage_twiddles<float>, blocks, dim3(256), 0, st, (float2*)tw, p);
     return hipGetLastError();
 }
 
