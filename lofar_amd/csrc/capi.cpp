@@ -966,17 +966,6 @@ int sm_log_cfg(int precision)
     return precision == LOFAR_FP64 ? 6 : -1;
 }
 
-// 8192-wide rows: split row passes (LOFAR_ROWS_SPLIT=0 keeps the fused ones, for
-// measurement)
-int rows_split()
-{
-    static int v = -1;
-    if (v < 0) {
-        const char* e = getenv("LOFAR_ROWS_SPLIT");
-        v = e ? atoi(e) != 0 : 1;
-    }
-    return v;
-}
 }  // namespace
 }  // namespace lofar
 
@@ -1133,7 +1122,7 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
     // of a plane row apart; FP32C keeps row-major planes (no gain measured there).
     // LOFAR_SM_LOG overrides, for measurement (-1: row-major; at most the tile width).
     // rows of 8192 run the split row passes, which read row-major planes
-    const bool split = grid_size_x >= 8192 && rows_split();
+    const bool split = grid_size_x >= 8192;
     const int sm_pref = (direct || generic || split) ? -1 : sm_log_cfg(precision);
     const int sm_log = (sm_pref >= 0 && (1 << sm_pref) <= kTile &&
                         grid_size_x % (1 << sm_pref) == 0 &&
@@ -1314,7 +1303,7 @@ static int degrid_transform(DeviceCtx& c, hipStream_t st, int precision, int num
                                grid_size_y, num_w_planes, scale, st, true);
         return r;
     }
-    const bool split = grid_size_x >= 8192 && rows_split();
+    const bool split = grid_size_x >= 8192;
     void *twx, *twy;
     r = twiddles(c, grid_size_x, precision, split ? 16 : 8, &twx);
     if (r) return r;

@@ -7,6 +7,7 @@
 // plane, scaled by 1/(nx*ny).  Column transforms run first, then rows, so the
 // last pass (rows, contiguous) fuses the w-phase screen and the plane sum of
 // phase_correction() (phase_correction.cu:151-210) and the image is written once.
+#include <algorithm>
 #include <cstdlib>
 
 #include "fft_kernels.h"
@@ -134,6 +135,12 @@ __global__ __launch_bounds__((W * Plan<N, E>::TPL)) void k_fft_cols(const C2<Rea
     constexpr int NRT = kRoots ? root_count<N, E>(1) : 0;
     T2 rt[NRT > 0 ? NRT : 1];
     if constexpr (NRT > 0) load_roots<T2, N, E, 1>(rt, t, tw);
+    // complex floats: the second stage's twiddles (each row's are shared by the W columns and
+    // recur every 16 rows) from LDS, written ahead of the first exchange's barrier
+    constexpr int kTwSpan = !kRoots && sizeof(T2) < 16 && N > 256 ? 256 : 0;
+    constexpr int NTL = kTwSpan ? kTwSpan - P::R0 : 0;
+    __shared__ T2 twl[NTL > 0 ? NTL : 1];
+    for (int i = threadIdx.x; i < NTL; i += W * P::TPL) twl[i] = tw[i];
     T2 v[P::E];
     if constexpr (OCC) {
         // An offset past the plane (rows of tiles without samples, columns past the
@@ -171,7 +178,8 @@ __global__ __launch_bounds__((W * Plan<N, E>::TPL)) void k_fft_cols(const C2<Rea
         for (int q = 0; q < P::E; q++)
             v[q] = active ? in[base + (long long)P::in_index(t, q) * rs] : T2{0, 0};
     }
-    stages<T2, N, E, SIGN, 1, ROUNDS, (NRT > 0)>(v, lds + c % WR, WR, t, tw, c / WR, rt);
+    stages<T2, N, E, SIGN, 1, ROUNDS, (NRT > 0), kTwSpan>(v, lds + c % WR, WR, t, tw, c / WR, rt,
+                                                          twl);
     if (active) {
         const __amdgpu_buffer_rsrc_t wsrc = __builtin_amdgcn_make_buffer_rsrc(
             (void*)(out + plane0), (short)0, plane_bytes, 0x00020000);
@@ -204,49 +212,12 @@ __device__ __forceinline__ double pixel_fac(const PhaseParams& pp, int iu, doubl
     return sqrt(1 - radius2);
 }
 
-// Per-pixel phase state of the fused row passes.  RECUR: plane factors by the
-// complex recurrence z_{w+1} = z_w*step (two complex numbers per pixel);
-// otherwise each plane's factor is evaluated directly with sincos_w (one double
-// per pixel).
-template <bool RECUR>
-struct PixelPhase;
-
-template <>
-struct PixelPhase<true> {
-    double2 z, stp;
-    __device__ __forceinline__ void init(const PhaseParams& pp, double fac)
-    {
-        phase_rotation(pp, fac, z, stp);
-    }
-    __device__ __forceinline__ double2 next(const PhaseParams&, double)
-    {
-        const double2 f = z;
-        z = cmul(z, stp);
-        return f;
-    }
-};
-
-template <>
-struct PixelPhase<false> {
-    double fac;
-    __device__ __forceinline__ void init(const PhaseParams&, double f) { fac = f; }
-    // factor of the plane whose 2*PI*wterm is c2w
-    __device__ __forceinline__ double2 next(const PhaseParams& pp, double c2w)
-    {
-        if (!pp.phase_on) return double2{1.0, 0.0};
-        double sn, cs;
-        sincos_w(c2w * (fac - 1.0), &sn, &cs);
-        const double f = pp.dwnorm * fac;
-        return double2{cs * f, sn * f};
-    }
-};
-
-// Row transforms of every plane of one image row; each output is multiplied by
-// its w-phase factor exp(i*phi_w)*dwnorm*sqrt(1-r^2) (phase_correction.cu:160,
-// 182-183,193-195) and summed over planes in registers, and the image row is
-// written once.  The thread's twiddle factors are loaded into registers once
-// (TWREG) since every plane's row uses the same ones.  FP64 phase and
-// accumulation in both precision modes.
+// Row transforms of every plane of one image row, summed over the planes with their w-phase
+// factors z0*step^w (phase_start, phase_step; phase_correction.cu:160,182-183,193-195) in registers,
+// last plane first: acc = acc*step + v, and the row written once is acc*z0 (Horner: no
+// running factor per pixel, a third less state and half the products).  The last
+// stage's twiddles stay in registers and the others' in LDS, since every plane's row uses
+// the same ones.  FP64 phase and accumulation in both precision modes.
 // Row prefetch for k_rows_phase: row iv of plane psrc goes straight into
 // pbuf[0, N) with 16-byte direct-to-LDS loads (global_load_lds_dwordx4); wave
 // instruction c of the row writes 1 KiB, elements [c*K, (c+1)*K) with K = 1024 /
@@ -279,150 +250,185 @@ __device__ __forceinline__ void prefetch_row(const T2* psrc, T2* pbuf, int t, in
     }
 }
 
+// The fused row passes of complex floats from 2048 on are compiled for two workgroups of
+// 4096 a CU (128 VGPRs, 72 KiB of LDS), which overlap each other's loads, exchanges and
+// arithmetic: the last stage's twiddles in registers, the others' in LDS.  Shorter rows have
+// several workgroups a CU either way, and complex doubles (172-256 VGPRs) one: theirs are
+// all in registers, since LDS is what bounds them (1024 rows of 1024 complex doubles and 8
+// planes: 48 us, 73 with the early stages' twiddles in LDS).
+template <typename Real, int N>
+constexpr bool kRowPair = sizeof(Real) == 4 && N >= 2048;
+template <typename Real, int N, int E>
+constexpr int row_tw_from()
+{
+    return kRowPair<Real, N> ? last_span<N, E>() : 1;
+}
+
 // LDS bytes of k_rows_phase with the row prefetch buffer
 template <typename Real, int N, int E>
 constexpr bool rows_prefetch_fits()
 {
-    return (Plan<N, E>::LDS + N) * (int)sizeof(C2<Real>) <= 160 * 1024;
+    return (Plan<N, E>::LDS + N + tw_lds<N, E>(row_tw_from<Real, N, E>())) * (int)sizeof(C2<Real>) <= 160 * 1024;
 }
 
-template <typename Real, int N, int E, bool RECUR, bool TWREG, bool PF>
-__global__ __launch_bounds__((Plan<N, E>::TPL)) void k_rows_phase(const C2<Real>* cube,
-                                                                const C2<Real>* tw, int ny, int nw,
-                                                                PhaseParams pp, double scale,
-                                                                double* img_re, double* img_im,
-                                                                int accumulate, int sm_log)
+// x, hidden from the compiler: what is computed from it again is not kept in registers
+__device__ __forceinline__ int opaque(int x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Groups of threads of a workgroup that share an image row's planes (launch_rows_phase_n);
+// rows of short images, whose few workgroups would wait out one plane after the other.
+constexpr int kRowGroups = 4;
+
+// G: groups of Plan::TPL threads, group g takes planes [g*ceil(nw/G), ...); their sums meet in
+// LDS and group 0 writes the row.
+template <typename Real, int N, int E, bool PF, int G>
+__global__ __launch_bounds__((G * Plan<N, E>::TPL), (kRowPair<Real, N> ? 4 : 1)) void k_rows_phase(
+    const C2<Real>* cube, const C2<Real>* tw, int ny, int nw, PhaseParams pp, double scale,
+    double* img_re, double* img_im, int accumulate, int sm_log)
 {
     using T2 = C2<Real>;
     using P = Plan<N, E>;
-    constexpr int NTW = tw_count<N, E>(1);
-    __shared__ T2 lds[P::LDS];
-    // PF: plane iw+1's row is loaded into pbuf while plane iw is transformed
+    static_assert(G == 1 || !PF, "the prefetch buffer is one group's");
+    constexpr int FROM = row_tw_from<Real, N, E>();
+    constexpr int NTW = tw_regs<N, E>(FROM), NTL = tw_lds<N, E>(FROM);
+    __shared__ T2 lds_all[G * P::LDS];
+    __shared__ T2 twl[NTL > 0 ? NTL : 1];
+    // PF: plane iw-1's row is loaded into pbuf while plane iw is transformed
     __shared__ __align__(16) T2 pbuf[PF ? N : 1];
+    __shared__ double2 sums[G > 1 ? (G - 1) * N : 1];
     const int iv = blockIdx.x;
-    const int t = threadIdx.x;
+    const int grp = G > 1 ? threadIdx.x / P::TPL : 0;
+    const int t = G > 1 ? threadIdx.x % P::TPL : threadIdx.x;
+    T2* lds = lds_all + grp * P::LDS;
+    const int per = (nw + G - 1) / G, first = grp * per;
     const long long img_row = (long long)iv * N;
+    const long long plane_stride = (long long)ny * N;
+    const T2* plane = cube + (long long)(first + per - 1) * plane_stride;
+    if constexpr (PF) prefetch_row<T2, N, P::TPL>(plane, pbuf, t, iv, ny, sm_log);
+    pp.wmin += first * pp.dw;
     const double ycoord = pp.phase_on ? pp.coord(iv, pp.ytot) : 0.0;
-    PixelPhase<RECUR> ph[P::E];
-    double2 acc[P::E];
+    for (int i = threadIdx.x; i < NTL; i += G * P::TPL) twl[i] = tw[i];  // read after barriers
+    T2 twr[NTW > 0 ? NTW : 1];
+    if constexpr (NTW > 0) load_twiddles<T2, N, E, FROM>(twr, t, tw);
+    double2 acc[P::E], step[P::E];
+    double fac[P::E];  // kept where there are registers, else computed again at the end
 #pragma unroll
     for (int e = 0; e < P::E; e++) {
-        ph[e].init(pp, pixel_fac(pp, P::out_index(t, e), ycoord));
-        if constexpr (RECUR) {
-            // the transform's scale 1/(nx*ny) (a power of two: exact) rides in the
-            // recurrence's first factor
-            ph[e].z.x *= scale;
-            ph[e].z.y *= scale;
-        }
+        fac[e] = pixel_fac(pp, P::out_index(t, e), ycoord);
+        step[e] = phase_step(pp, fac[e]);
         acc[e] = double2{0.0, 0.0};
     }
-    T2 twr[NTW > 0 ? NTW : 1];
-    if constexpr (TWREG && NTW > 0) load_twiddles<T2, N, E, 1>(twr, t, tw);
-    const long long plane_stride = (long long)ny * N;
-    // element u of the row: at u (row-major planes) or, in strip-major planes
-    // ([N/L][ny][L], L = 2^sm_log), at (u/L)*ny*L + iv*L + u%L
-    long long off[P::E];
-#pragma unroll
-    for (int q = 0; q < P::E; q++) {
-        const int u = P::in_index(t, q);
-        off[q] = sm_log < 0 ? img_row + u
-                            : ((((long long)(u >> sm_log) * ny + iv) << sm_log) |
-                               (u & ((1 << sm_log) - 1)));
-    }
-    if constexpr (PF) prefetch_row<T2, N, P::TPL>(cube, pbuf, t, iv, ny, sm_log);
     T2 v[P::E];
-    for (int iw = 0; iw < nw; iw++) {
+    for (int iw = per - 1; iw >= 0; iw--, plane -= plane_stride) {
         if constexpr (PF) {
             wait_loads();
             lds_barrier();  // every wave's part of the row is in pbuf
 #pragma unroll
             for (int q = 0; q < P::E; q++) v[q] = pbuf[P::in_index(t, q)];
             lds_barrier();  // pbuf read by every wave: free for the next plane
-            if (iw + 1 < nw)
-                prefetch_row<T2, N, P::TPL>(cube + (long long)(iw + 1) * plane_stride, pbuf, t, iv,
-                                            ny, sm_log);
+            if (iw > 0)
+                prefetch_row<T2, N, P::TPL>(plane - plane_stride, pbuf, t, iv, ny, sm_log);
         } else {
-            const T2* psrc = cube + (long long)iw * plane_stride;
+            // element u of the row: at u (row-major planes) or, in strip-major planes
+            // ([N/L][ny][L], L = 2^sm_log), at (u/L)*ny*L + iv*L + u%L
+            const bool there = G == 1 || first + iw < nw;
 #pragma unroll
-            for (int q = 0; q < P::E; q++) v[q] = psrc[off[q]];
+            for (int q = 0; q < P::E; q++) {
+                const int u = P::in_index(t, q);
+                const long long o = sm_log < 0
+                                        ? img_row + u
+                                        : ((((long long)(u >> sm_log) * ny + iv) << sm_log) |
+                                           (u & ((1 << sm_log) - 1)));
+                v[q] = there ? plane[o] : T2{0, 0};
+            }
         }
-        if constexpr (TWREG)
-            stages_rt<T2, N, E, 1, 1, PF>(v, lds, t, twr);
-        else
-            stages<T2, N, E, 1, 1>(v, lds, 1, t, tw);
-        const double c2w = 2.0 * LOFAR_REF_PI * (pp.wmin + iw * pp.dw);
+        stages_rt<T2, N, E, 1, FROM, PF>(v, lds, t, twr, twl);
 #pragma unroll
         for (int e = 0; e < P::E; e++) {
-            if constexpr (RECUR) {
-                // acc += v*z as four fused multiply-adds
-                const double2 z = ph[e].next(pp, c2w);
-                const double vx = (double)v[e].x, vy = (double)v[e].y;
-                acc[e].x = fma(vx, z.x, fma(-vy, z.y, acc[e].x));
-                acc[e].y = fma(vx, z.y, fma(vy, z.x, acc[e].y));
-            } else {
-                const double2 pq = double2{(double)v[e].x * scale, (double)v[e].y * scale};
-                const double2 term = cmul(pq, ph[e].next(pp, c2w));
-                acc[e].x += term.x;
-                acc[e].y += term.y;
-            }
+            const double2 a = acc[e], s = step[e];
+            acc[e].x = fma(a.x, s.x, fma(-a.y, s.y, (double)v[e].x));
+            acc[e].y = fma(a.x, s.y, fma(a.y, s.x, (double)v[e].y));
         }
     }
 #pragma unroll
     for (int e = 0; e < P::E; e++) {
-        const long long o = img_row + P::out_index(t, e);
+        const int u = P::out_index(t, e);
+        double2 z0 = phase_start(pp, kRowPair<Real, N> ? pixel_fac(pp, opaque(u), ycoord) : fac[e]);
+        z0.x *= scale;  // the transform's 1/(nx*ny), a power of two: exact
+        z0.y *= scale;
+        acc[e] = cmul(acc[e], z0);
+        if (G > 1 && grp > 0) sums[(grp - 1) * N + u] = acc[e];
+    }
+    if constexpr (G > 1) {
+        __syncthreads();
+        if (grp > 0) return;
+    }
+#pragma unroll
+    for (int e = 0; e < P::E; e++) {
+        const int u = P::out_index(t, e);
+        double2 x = acc[e];
+#pragma unroll
+        for (int g = 1; g < G; g++) {
+            const double2 y = sums[(g - 1) * N + u];
+            x.x += y.x;
+            x.y += y.y;
+        }
+        const long long o = img_row + u;
         if (accumulate) {
-            img_re[o] += acc[e].x;
-            img_im[o] += acc[e].y;
+            img_re[o] += x.x;
+            img_im[o] += x.y;
         } else {
-            img_re[o] = acc[e].x;
-            img_im[o] = acc[e].y;
+            img_re[o] = x.x;
+            img_im[o] = x.y;
         }
     }
 }
 
 // Adjoint of k_rows_phase: for every plane, the image row times the conjugate
-// w-phase factor, forward row transform, plane row written out.
-template <typename Real, int N, int E, bool RECUR, bool TWREG>
-__global__ __launch_bounds__((Plan<N, E>::TPL)) void k_rows_phase_adj(C2<Real>* cube,
-                                                                    const C2<Real>* tw, int ny,
-                                                                    int nw, PhaseParams pp,
-                                                                    double scale,
-                                                                    const double* img_re,
-                                                                    const double* img_im)
+// w-phase factor (the row times conj(z0), turned by conj(step) from plane to plane), forward
+// row transform, plane row written out.
+template <typename Real, int N, int E>
+__global__ __launch_bounds__((Plan<N, E>::TPL), (kRowPair<Real, N> ? 4 : 1)) void k_rows_phase_adj(
+    C2<Real>* cube, const C2<Real>* tw, int ny, int nw, PhaseParams pp, double scale,
+    const double* img_re, const double* img_im)
 {
     using T2 = C2<Real>;
     using P = Plan<N, E>;
-    constexpr int NTW = tw_count<N, E>(1);
+    constexpr int FROM = row_tw_from<Real, N, E>();
+    constexpr int NTW = tw_regs<N, E>(FROM), NTL = tw_lds<N, E>(FROM);
     __shared__ T2 lds[P::LDS];
+    __shared__ T2 twl[NTL > 0 ? NTL : 1];
     const int iv = blockIdx.x;
     const int t = threadIdx.x;
     const long long img_row = (long long)iv * N;
+    const int per = (nw + gridDim.y - 1) / gridDim.y, first = blockIdx.y * per;
+    const int last = min(nw, first + per);
+    pp.wmin += first * pp.dw;
     const double ycoord = pp.phase_on ? pp.coord(iv, pp.ytot) : 0.0;
-    PixelPhase<RECUR> ph[P::E];
-    double2 a[P::E];
+    for (int i = t; i < NTL; i += P::TPL) twl[i] = tw[i];  // read after a stage's barriers
+    T2 twr[NTW > 0 ? NTW : 1];
+    if constexpr (NTW > 0) load_twiddles<T2, N, E, FROM>(twr, t, tw);
+    double2 a[P::E], step[P::E];
 #pragma unroll
     for (int q = 0; q < P::E; q++) {
         const int iu = P::in_index(t, q);
-        ph[q].init(pp, pixel_fac(pp, iu, ycoord));
-        a[q] = double2{img_re[img_row + iu], img_im[img_row + iu]};
+        const double fac = pixel_fac(pp, iu, ycoord);
+        const double2 z0 = phase_start(pp, fac);
+        step[q] = phase_step(pp, fac);
+        a[q] = cmul_conj(double2{img_re[img_row + iu], img_im[img_row + iu]}, z0);
     }
-    T2 twr[NTW > 0 ? NTW : 1];
-    if constexpr (TWREG && NTW > 0) load_twiddles<T2, N, E, 1>(twr, t, tw);
     const long long plane_stride = (long long)ny * N;
-    for (int iw = 0; iw < nw; iw++) {
-        const double c2w = 2.0 * LOFAR_REF_PI * (pp.wmin + iw * pp.dw);
+    for (int iw = first; iw < last; iw++) {
         T2 v[P::E];
 #pragma unroll
         for (int q = 0; q < P::E; q++) {
-            const double2 z = ph[q].next(pp, c2w);
-            // a * conj(z)
-            v[q].x = (Real)(a[q].x * z.x + a[q].y * z.y);
-            v[q].y = (Real)(a[q].y * z.x - a[q].x * z.y);
+            v[q] = T2{(Real)a[q].x, (Real)a[q].y};
+            a[q] = cmul_conj(a[q], step[q]);
         }
-        if constexpr (TWREG)
-            stages_rt<T2, N, E, -1, 1>(v, lds, t, twr);
-        else
-            stages<T2, N, E, -1, 1>(v, lds, 1, t, tw);
+        stages_rt<T2, N, E, -1, FROM, true>(v, lds, t, twr, twl);
         T2* dst = cube + (long long)iw * plane_stride + img_row;
 #pragma unroll
         for (int e = 0; e < P::E; e++) {
@@ -512,8 +518,10 @@ static hipError_t launch_cols_n(int sign, const void* in, void* out, const void*
     constexpr int W64 = 64 / (2 * (int)sizeof(Real));
     // 8192-long complex-double columns at 32 elements a thread would need 128 VGPRs
     // of data alone at 1024 threads (they spilled: 0.74 TB/s); 16 elements, 2 columns
-    // and 2 LDS rounds run without spills (2.5 TB/s)
-    if constexpr (sizeof(Real) == 8 && N >= 8192)
+    // and 2 LDS rounds run without spills (2.5 TB/s).  Columns up to 1024 complex doubles
+    // also take 16: twice the waves for a strip (54 -> 46 us for 8 planes of 1024 x 1024);
+    // 2048 measured the same at 16 and 32, 4096 3.55 ms at 16 and 3.44 at 32.
+    if constexpr (sizeof(Real) == 8 && (N >= 8192 || N <= 1024))
         if (col_cfg() == 0 || sm_log >= 0)
             return launch_cols_cfg<Real, N, 16, W64, 2>(sign, in, out, tw, nx, nw, scale, occ, sm_log, st);
     if (sm_log >= 0)
@@ -526,38 +534,38 @@ static hipError_t launch_cols_n(int sign, const void* in, void* out, const void*
     }
 }
 
-template <typename Real, int N, int E, bool RECUR, bool TWREG, bool PF = false>
-static hipError_t launch_rows_phase_cfg(const void* cube, const void* tw, int ny, int nw,
-                                        const PhaseParams& pp, double scale, double* re,
-                                        double* im, int accumulate, int sm_log, hipStream_t st)
+// Parts an image row's planes are split into: kRowGroups where one workgroup per row is at
+// most 4 waves a CU (rows up to 512 of images as tall) and there are as many planes.
+static int row_groups(int tpl, int ny, int nw)
 {
-    using T2 = C2<Real>;
-    if constexpr (PF) {
-        // the prefetch reads whole 1 KiB runs: row-major rows, or strips at least
-        // that wide
-        constexpr int K = 1024 / (int)sizeof(T2);
-        if (sm_log >= 0 && (1 << sm_log) < K)
-            return launch_rows_phase_cfg<Real, N, E, RECUR, TWREG, false>(
-                cube, tw, ny, nw, pp, scale, re, im, accumulate, sm_log, st);
-    }
-    hipLaunchKernelGGL((k_rows_phase<Real, N, E, RECUR, TWREG, PF>), dim3(ny),
-                       dim3(Plan<N, E>::TPL), 0, st, (const T2*)cube, (const T2*)tw, ny, nw, pp,
-                       scale, re, im, accumulate, sm_log);
-    return hipGetLastError();
+    return (long long)ny * std::max(tpl, 64) <= 4 * 64 * 256 && nw >= kRowGroups ? kRowGroups : 1;
 }
 
-// the fused row pass: 8 elements per thread, phase recurrence, twiddles in registers, next
-// row prefetched into LDS where it fits
+// the fused row pass: 8 elements per thread, the next row prefetched into LDS where it fits
+// and planes hold whole 1 KiB runs (row-major rows, or strips at least that wide)
 template <typename Real, int N>
 static hipError_t launch_rows_phase_n(const void* cube, const void* tw, int ny, int nw,
                                       const PhaseParams& pp, double scale, double* re, double* im,
                                       int accumulate, int sm_log, hipStream_t st)
 {
-#define ARGS_ cube, tw, ny, nw, pp, scale, re, im, accumulate, sm_log, st
-    return launch_rows_phase_cfg<Real, N, 8, true, true,
-                                 (Plan<N, 8>::TPL >= 64 && rows_prefetch_fits<Real, N, 8>())>(
-        ARGS_);
-#undef ARGS_
+    using T2 = C2<Real>;
+    constexpr int E = kPhaseE;
+    constexpr int K = 1024 / (int)sizeof(T2);
+    constexpr bool fits = Plan<N, E>::TPL >= 64 && rows_prefetch_fits<Real, N, E>();
+    constexpr int TPL = Plan<N, E>::TPL;
+    if constexpr (N <= 512) {
+        if (row_groups(TPL, ny, nw) > 1) {
+            hipLaunchKernelGGL((k_rows_phase<Real, N, E, false, kRowGroups>), dim3(ny),
+                               dim3(kRowGroups * TPL), 0, st, (const T2*)cube, (const T2*)tw, ny,
+                               nw, pp, scale, re, im, accumulate, sm_log);
+            return hipGetLastError();
+        }
+    }
+    auto k = fits && (sm_log < 0 || (1 << sm_log) >= K) ? k_rows_phase<Real, N, E, fits, 1>
+                                                        : k_rows_phase<Real, N, E, false, 1>;
+    hipLaunchKernelGGL(k, dim3(ny), dim3(TPL), 0, st, (const T2*)cube, (const T2*)tw, ny, nw, pp,
+                       scale, re, im, accumulate, sm_log);
+    return hipGetLastError();
 }
 
 template <typename Real, int N>
@@ -566,26 +574,35 @@ static hipError_t launch_rows_phase_adj_n(void* cube, const void* tw, int ny, in
                                           const double* im, hipStream_t st)
 {
     using T2 = C2<Real>;
-    hipLaunchKernelGGL((k_rows_phase_adj<Real, N, kPhaseE, true, true>), dim3(ny),
-                       dim3(Plan<N, kPhaseE>::TPL), 0, st, (T2*)cube, (const T2*)tw, ny, nw, pp,
+    constexpr int TPL = Plan<N, kPhaseE>::TPL;
+    hipLaunchKernelGGL((k_rows_phase_adj<Real, N, kPhaseE>), dim3(ny, row_groups(TPL, ny, nw)),
+                       dim3(TPL), 0, st, (T2*)cube, (const T2*)tw, ny, nw, pp,
                        scale, re, im);
     return hipGetLastError();
 }
 
+// sides up to 4096 (the fused row passes), and up to 8192
+#define LOFAR_FFT_CASES(CALL)     \
+    case 2: return CALL(2);       \
+    case 4: return CALL(4);       \
+    case 8: return CALL(8);       \
+    case 16: return CALL(16);     \
+    case 32: return CALL(32);     \
+    case 64: return CALL(64);     \
+    case 128: return CALL(128);   \
+    case 256: return CALL(256);   \
+    case 512: return CALL(512);   \
+    case 1024: return CALL(1024); \
+    case 2048: return CALL(2048); \
+    case 4096: return CALL(4096);
+#define LOFAR_FFT_SWITCH_4096(N_, CALL)       \
+    switch (N_) {                             \
+        LOFAR_FFT_CASES(CALL)                 \
+        default: return hipErrorInvalidValue; \
+    }
 #define LOFAR_FFT_SWITCH(N_, CALL)            \
     switch (N_) {                             \
-        case 2: return CALL(2);               \
-        case 4: return CALL(4);               \
-        case 8: return CALL(8);               \
-        case 16: return CALL(16);             \
-        case 32: return CALL(32);             \
-        case 64: return CALL(64);             \
-        case 128: return CALL(128);           \
-        case 256: return CALL(256);           \
-        case 512: return CALL(512);           \
-        case 1024: return CALL(1024);         \
-        case 2048: return CALL(2048);         \
-        case 4096: return CALL(4096);         \
+        LOFAR_FFT_CASES(CALL)                 \
         case 8192: return CALL(8192);         \
         default: return hipErrorInvalidValue; \
     }
@@ -614,7 +631,7 @@ hipError_t rows_phase(const void* cube, const void* tw, int nx, int ny, int nw,
                       hipStream_t st, int sm_log)
 {
 #define CALL_(n) launch_rows_phase_n<Real, n>(cube, tw, ny, nw, pp, scale, re, im, accumulate, sm_log, st)
-    LOFAR_FFT_SWITCH(nx, CALL_)
+    LOFAR_FFT_SWITCH_4096(nx, CALL_)
 #undef CALL_
 }
 
@@ -624,7 +641,7 @@ hipError_t rows_phase_adj(void* cube, const void* tw, int nx, int ny, int nw,
                           hipStream_t st)
 {
 #define CALL_(n) launch_rows_phase_adj_n<Real, n>(cube, tw, ny, nw, pp, scale, re, im, st)
-    LOFAR_FFT_SWITCH(nx, CALL_)
+    LOFAR_FFT_SWITCH_4096(nx, CALL_)
 #undef CALL_
 }
 

@@ -46,6 +46,68 @@ __device__ __forceinline__ long long xcd_remap(long long b, long long g)
     return (b % 8) * (g / 8) + b / 8;
 }
 
+// sin and cos of x in double precision, from the mathematics: x = n*pi/2 + t
+// with a three-part Cody-Waite pi/2 (the first two parts have 33 significant
+// bits, so n*part is exact for |n| < 2^20), then Taylor series to t^17 / t^16 on
+// |t| <= pi/4 (truncation below 1e-18).  |x| beyond 1e5 falls back to sincos().
+constexpr double kPio2Hi = 1.5707963267341256;
+constexpr double kPio2Mid = 6.077100506303966e-11;
+constexpr double kPio2Lo = 2.0222662487959506e-21;
+constexpr double kTwoOverPi = 0.6366197723675814;
+__device__ __forceinline__ double sin_poly(double t)
+{
+    const double t2 = t * t;
+    // 1/k! for k = 3..17 (odd), Horner in t^2
+    double ps = 2.8114572543455206e-15;
+    ps = fma(ps, t2, -7.647163731819816e-13);
+    ps = fma(ps, t2, 1.6059043836821613e-10);
+    ps = fma(ps, t2, -2.505210838544172e-08);
+    ps = fma(ps, t2, 2.7557319223985893e-06);
+    ps = fma(ps, t2, -0.0001984126984126984);
+    ps = fma(ps, t2, 0.008333333333333333);
+    ps = fma(ps, t2, -0.16666666666666666);
+    return fma(ps * t2, t, t);
+}
+__device__ __forceinline__ void sincos_w(double x, double* sn, double* cs)
+{
+    if (!(fabs(x) < 1.0e5)) {
+        sincos(x, sn, cs);
+        return;
+    }
+    const double n = rint(x * kTwoOverPi);
+    double t = fma(-n, kPio2Hi, x);
+    t = fma(-n, kPio2Mid, t);
+    t = fma(-n, kPio2Lo, t);
+    const double t2 = t * t;
+    const double st = sin_poly(t);
+    // 1/k! for k = 2..16 (even)
+    double pc = 4.779477332387385e-14;
+    pc = fma(pc, t2, -1.1470745597729725e-11);
+    pc = fma(pc, t2, 2.08767569878681e-09);
+    pc = fma(pc, t2, -2.755731922398589e-07);
+    pc = fma(pc, t2, 2.48015873015873e-05);
+    pc = fma(pc, t2, -0.001388888888888889);
+    pc = fma(pc, t2, 0.041666666666666664);
+    pc = fma(pc, t2, -0.5);
+    const double ct = fma(pc, t2, 1.0);
+    const int q = ((int)n) & 3;
+    const double s_ = (q & 1) ? ct : st;
+    const double c_ = (q & 1) ? st : ct;
+    *sn = (q & 2) ? -s_ : s_;
+    *cs = ((q + 1) & 2) ? -c_ : c_;
+}
+
+// sin of a pixel coordinate's angle: below pi/4 (every coordinate of a field up to 1.5
+// radians across) the polynomial alone, where the library's sin took as long as a plane's
+// transform
+__device__ __forceinline__ double sin_w(double x)
+{
+    if (fabs(x) <= 0.785) return sin_poly(x);
+    double sn, cs;
+    sincos_w(x, &sn, &cs);
+    return sn;
+}
+
 // w-phase geometry of phase_correction.cu:92-94,164-172
 struct PhaseParams {
     int xtot, ytot;
@@ -55,7 +117,7 @@ struct PhaseParams {
     {
         double c = (double)(i - tot / 2);
         if (c < 0.0) c = (double)(i + tot / 2);
-        return sin(c * resolution);
+        return sin_w(c * resolution);
     }
 };
 
@@ -80,6 +142,19 @@ __device__ __forceinline__ T2 c_mul_tw(T2 a, T2 w)
         return T2{a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x};
     else
         return T2{a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y};
+}
+// The same in the fused row passes.  Which product of a complex float each part rounds first
+// is written out: left to the compiler it depends on whether the twiddle comes from a
+// register or from LDS, and the FP32C results should not.
+template <int SIGN, typename T2>
+__device__ __forceinline__ T2 c_mul_tw_row(T2 a, T2 w)
+{
+    if constexpr (sizeof(T2) != 8)
+        return c_mul_tw<SIGN>(a, w);
+    else if constexpr (SIGN > 0)
+        return T2{fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.x, w.y, a.y * w.x)};
+    else
+        return T2{fmaf(a.x, w.x, a.y * w.y), fmaf(a.y, w.x, -(a.x * w.y))};
 }
 // a * (S*i)
 template <int S, typename T2>
@@ -193,6 +268,36 @@ __device__ __forceinline__ void dft(T2* v)
     }
 }
 
+// dft() of the fused row passes: in complex floats the products by cos(pi/4) of the radix-8
+// rotations are written out (see c_mul_tw_row): one product of each pair is rounded and
+// shared, the other fused.
+template <int R, int S, typename T2>
+__device__ __forceinline__ void dft_row(T2* v)
+{
+    if constexpr (R == 8 && sizeof(T2) == 8) {
+        dft4<S>(v[0], v[2], v[4], v[6]);
+        dft4<S>(v[1], v[3], v[5], v[7]);
+        constexpr float k = (float)kC2;
+        const T2 a = v[3], b = v[7];  // times exp(S*2*pi*i/8) and exp(S*6*pi*i/8)
+        const float ka = k * a.x, kb = S > 0 ? -k * b.y : -k * b.x;
+        v[3] = S > 0 ? T2{fmaf(a.y, -k, ka), fmaf(k, a.y, ka)}
+                     : T2{fmaf(a.y, k, ka), fmaf(a.y, k, -ka)};
+        v[5] = c_muli<S>(v[5]);
+        v[7] = S > 0 ? T2{fmaf(b.x, -k, kb), fmaf(k, b.x, kb)}
+                     : T2{fmaf(b.y, k, kb), fmaf(-k, b.y, kb)};
+        T2 o[8];
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++) {
+            o[k1] = c_add(v[2 * k1], v[2 * k1 + 1]);
+            o[k1 + 4] = c_sub(v[2 * k1], v[2 * k1 + 1]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = o[j];
+    } else {
+        dft<R, S>(v);
+    }
+}
+
 // Stockham stages from span NS on.  On entry v[m*R+q] holds element b+q*(N/R)
 // of butterfly b = t + m*TPL; on return v holds the outputs in the order of
 // Plan<N,E>::out_index.  `lds` addresses element i of this line at
@@ -212,9 +317,13 @@ __device__ __forceinline__ const T2* stage_tw(const T2* tw, int ns)
 {
     return tw + (ns - P::R0);
 }
-template <typename T2, int N, int EREQ, int SIGN, int NS, int ROUNDS = 1, bool RT = false>
+// LDS_TW: the twiddles of spans below LDS_TW are read from twl (the table's first entries, in
+// LDS).
+template <typename T2, int N, int EREQ, int SIGN, int NS, int ROUNDS = 1, bool RT = false,
+          int LDS_TW = 0>
 __device__ __forceinline__ void stages(T2* v, T2* lds, int ls, int t, const T2* __restrict__ tw,
-                                       int my_round = 0, const T2* rt = nullptr)
+                                       int my_round = 0, const T2* rt = nullptr,
+                                       const T2* twl = nullptr)
 {
     using P = Plan<N, EREQ>;
     constexpr int E = P::E;
@@ -237,8 +346,9 @@ __device__ __forceinline__ void stages(T2* v, T2* lds, int ls, int t, const T2* 
                 const int k = b & (NS - 1);
 #pragma unroll
                 for (int q = 1; q < R; q++)
-                    v[m * R + q] =
-                        c_mul_tw<SIGN>(v[m * R + q], stage_tw<P>(tw, NS)[(q - 1) * NS + k]);
+                    v[m * R + q] = c_mul_tw<SIGN>(
+                        v[m * R + q],
+                        stage_tw<P>(NS < LDS_TW ? twl : tw, NS)[(q - 1) * NS + k]);
             }
         }
         dft<R, SIGN>(&v[m * R]);
@@ -288,8 +398,8 @@ __device__ __forceinline__ void stages(T2* v, T2* lds, int ls, int t, const T2* 
                 }
             }
         }
-        stages<T2, N, EREQ, SIGN, NS2, ROUNDS, RT>(v, lds, ls, t, tw, my_round,
-                                                  RT ? rt + (NS > 1 ? M : 0) : rt);
+        stages<T2, N, EREQ, SIGN, NS2, ROUNDS, RT, LDS_TW>(
+            v, lds, ls, t, tw, my_round, RT ? rt + (NS > 1 ? M : 0) : rt, twl);
     }
 }
 
@@ -325,30 +435,50 @@ __device__ __forceinline__ void load_roots(T2* rt, int t, const T2* __restrict__
     if constexpr (NS * R < N) load_roots<T2, N, EREQ, NS * R>(rt + (NS > 1 ? M : 0), t, tw);
 }
 
-// Number of twiddle factors one thread applies from span NS to the last stage.
+// Twiddles of loops over many lines of one length (the fused row passes), loaded once: those
+// of the stages from span FROM on (which differ from thread to thread) stay in registers, the
+// earlier stages' (few entries, shared by the threads) in LDS.  last_span: the span of the
+// last stage; tw_regs: twiddles a thread applies from span FROM on; tw_lds: the first
+// entries of the length's table, up to span FROM.
 template <int N, int EREQ>
-constexpr int tw_count(int ns)
+constexpr int last_span()
 {
     using P = Plan<N, EREQ>;
-    int total = 0;
+    int ns = 1;
     while (ns < N) {
         const int r = (N / ns >= P::RX) ? P::RX : N / ns;
-        if (ns > 1) total += (P::E / r) * (r - 1);
+        if (ns * r >= N) return ns;
+        ns *= r;
+    }
+    return ns;
+}
+template <int N, int EREQ>
+constexpr int tw_regs(int from)
+{
+    using P = Plan<N, EREQ>;
+    int total = 0, ns = 1;
+    while (ns < N) {
+        const int r = (N / ns >= P::RX) ? P::RX : N / ns;
+        if (ns > 1 && ns >= from) total += (P::E / r) * (r - 1);
         ns *= r;
     }
     return total;
 }
+template <int N, int EREQ>
+constexpr int tw_lds(int from)
+{
+    return from > Plan<N, EREQ>::R0 ? from - Plan<N, EREQ>::R0 : 0;
+}
 
-// Loads, once, every twiddle factor thread t applies in stages(), in the order
-// stages_rt() consumes them, so loops over many lines of the same length keep
-// them in registers instead of re-reading the table at every stage.
-template <typename T2, int N, int EREQ, int NS>
+// Loads thread t's register twiddles in the order stages_rt consumes them.
+template <typename T2, int N, int EREQ, int FROM, int NS = 1>
 __device__ __forceinline__ void load_twiddles(T2* twr, int t, const T2* __restrict__ tw)
 {
     using P = Plan<N, EREQ>;
     constexpr int R = (N / NS >= P::RX) ? P::RX : N / NS;
     constexpr int M = P::E / R;
-    if constexpr (NS > 1) {
+    constexpr bool mine = NS > 1 && NS >= FROM;
+    if constexpr (mine) {
 #pragma unroll
         for (int m = 0; m < M; m++) {
             const int k = (t + m * P::TPL) & (NS - 1);
@@ -358,7 +488,7 @@ __device__ __forceinline__ void load_twiddles(T2* twr, int t, const T2* __restri
         }
     }
     if constexpr (NS * R < N)
-        load_twiddles<T2, N, EREQ, NS * R>(twr + (NS > 1 ? M * (R - 1) : 0), t, tw);
+        load_twiddles<T2, N, EREQ, FROM, NS * R>(twr + (mine ? M * (R - 1) : 0), t, tw);
 }
 
 template <bool LB>
@@ -370,24 +500,29 @@ __device__ __forceinline__ void stage_barrier()
         __syncthreads();
 }
 
-// stages() with the twiddle factors taken from registers filled by load_twiddles().
+// stages() with the twiddles from span FROM on from registers (load_twiddles) and the earlier
+// stages' from twl, the table's first tw_lds entries in LDS.
 // LB: exchange barriers wait for LDS operations only (lds_barrier).
-template <typename T2, int N, int EREQ, int SIGN, int NS, bool LB = false>
-__device__ __forceinline__ void stages_rt(T2* v, T2* lds, int t, const T2* twr)
+template <typename T2, int N, int EREQ, int SIGN, int FROM, bool LB = false, int NS = 1>
+__device__ __forceinline__ void stages_rt(T2* v, T2* lds, int t, const T2* twr, const T2* twl)
 {
     using P = Plan<N, EREQ>;
     constexpr int E = P::E;
     constexpr int TPL = P::TPL;
     constexpr int R = (N / NS >= P::RX) ? P::RX : N / NS;
     constexpr int M = E / R;
+    constexpr bool regs = NS > 1 && NS >= FROM;
 #pragma unroll
     for (int m = 0; m < M; m++) {
         if constexpr (NS > 1) {
+            const int k = (t + m * TPL) & (NS - 1);
 #pragma unroll
             for (int q = 1; q < R; q++)
-                v[m * R + q] = c_mul_tw<SIGN>(v[m * R + q], twr[m * (R - 1) + q - 1]);
+                v[m * R + q] = c_mul_tw_row<SIGN>(
+                    v[m * R + q], regs ? twr[m * (R - 1) + q - 1]
+                                       : stage_tw<P>(twl, NS)[(q - 1) * NS + k]);
         }
-        dft<R, SIGN>(&v[m * R]);
+        dft_row<R, SIGN>(&v[m * R]);
     }
     if constexpr (NS * R < N) {
         constexpr int NS2 = NS * R;
@@ -409,53 +544,9 @@ __device__ __forceinline__ void stages_rt(T2* v, T2* lds, int t, const T2* twr)
 #pragma unroll
             for (int q = 0; q < R2; q++) v[m * R2 + q] = lds[P::pad(b + q * (N / R2))];
         }
-        stages_rt<T2, N, EREQ, SIGN, NS2, LB>(v, lds, t, twr + (NS > 1 ? M * (R - 1) : 0));
+        stages_rt<T2, N, EREQ, SIGN, FROM, LB, NS2>(
+            v, lds, t, twr + (regs ? M * (R - 1) : 0), twl);
     }
-}
-
-// sin and cos of x in double precision, from the mathematics: x = n*pi/2 + t
-// with a three-part Cody-Waite pi/2 (the first two parts have 33 significant
-// bits, so n*part is exact for |n| < 2^20), then Taylor series to t^17 / t^16 on
-// |t| <= pi/4 (truncation below 1e-18).  |x| beyond 1e5 falls back to sincos().
-constexpr double kPio2Hi = 1.5707963267341256;
-constexpr double kPio2Mid = 6.077100506303966e-11;
-constexpr double kPio2Lo = 2.0222662487959506e-21;
-constexpr double kTwoOverPi = 0.6366197723675814;
-__device__ __forceinline__ void sincos_w(double x, double* sn, double* cs)
-{
-    if (!(fabs(x) < 1.0e5)) {
-        sincos(x, sn, cs);
-        return;
-    }
-    const double n = rint(x * kTwoOverPi);
-    double t = fma(-n, kPio2Hi, x);
-    t = fma(-n, kPio2Mid, t);
-    t = fma(-n, kPio2Lo, t);
-    const double t2 = t * t;
-    // 1/k! for k = 3..17 (odd) and 2..16 (even), Horner in t^2
-    double ps = 2.8114572543455206e-15;
-    ps = fma(ps, t2, -7.647163731819816e-13);
-    ps = fma(ps, t2, 1.6059043836821613e-10);
-    ps = fma(ps, t2, -2.505210838544172e-08);
-    ps = fma(ps, t2, 2.7557319223985893e-06);
-    ps = fma(ps, t2, -0.0001984126984126984);
-    ps = fma(ps, t2, 0.008333333333333333);
-    ps = fma(ps, t2, -0.16666666666666666);
-    const double st = fma(ps * t2, t, t);
-    double pc = 4.779477332387385e-14;
-    pc = fma(pc, t2, -1.1470745597729725e-11);
-    pc = fma(pc, t2, 2.08767569878681e-09);
-    pc = fma(pc, t2, -2.755731922398589e-07);
-    pc = fma(pc, t2, 2.48015873015873e-05);
-    pc = fma(pc, t2, -0.001388888888888889);
-    pc = fma(pc, t2, 0.041666666666666664);
-    pc = fma(pc, t2, -0.5);
-    const double ct = fma(pc, t2, 1.0);
-    const int q = ((int)n) & 3;
-    const double s_ = (q & 1) ? ct : st;
-    const double c_ = (q & 1) ? st : ct;
-    *sn = (q & 2) ? -s_ : s_;
-    *cs = ((q + 1) & 2) ? -c_ : c_;
 }
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b)
@@ -463,25 +554,30 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b)
     return double2{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
 
-// w-phase factor of one pixel for the plane recurrence: z0 = dwnorm*fac*exp(i*phi_0)
-// and step = exp(i*(phi_1-phi_0)), with phi_w = 2*PI*(wmin + w*dw)*(fac-1)
-// (phase_correction.cu:160,182-183,193-195), so plane w's factor is z0*step^w.
-// Without the phase (a single plane) both are 1.  FP64 throughout.
-__device__ __forceinline__ void phase_rotation(const PhaseParams& pp, double fac, double2& z0,
-                                               double2& step)
+// a * conj(b)
+__device__ __forceinline__ double2 cmul_conj(double2 a, double2 b)
 {
-    if (!pp.phase_on) {
-        z0 = double2{1.0, 0.0};
-        step = double2{1.0, 0.0};
-        return;
-    }
-    const double n1 = fac - 1.0;
+    return double2{a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y};
+}
+
+// w-phase factor of one pixel for the plane recurrence: phase_start is z0 =
+// dwnorm*fac*exp(i*phi_0) and phase_step exp(i*(phi_1-phi_0)), with phi_w = 2*PI*(wmin +
+// w*dw)*(fac-1) (phase_correction.cu:160,182-183,193-195), so plane w's factor is
+// z0*step^w.  Without the phase (a single plane) both are 1.  FP64 throughout.
+__device__ __forceinline__ double2 phase_start(const PhaseParams& pp, double fac)
+{
+    if (!pp.phase_on) return double2{1.0, 0.0};
     double sn, cs;
-    sincos_w(2.0 * LOFAR_REF_PI * pp.wmin * n1, &sn, &cs);
+    sincos_w(2.0 * LOFAR_REF_PI * pp.wmin * (fac - 1.0), &sn, &cs);
     const double f = pp.dwnorm * fac;
-    z0 = double2{cs * f, sn * f};
-    sincos_w(2.0 * LOFAR_REF_PI * pp.dw * n1, &sn, &cs);
-    step = double2{cs, sn};
+    return double2{cs * f, sn * f};
+}
+__device__ __forceinline__ double2 phase_step(const PhaseParams& pp, double fac)
+{
+    if (!pp.phase_on) return double2{1.0, 0.0};
+    double sn, cs;
+    sincos_w(2.0 * LOFAR_REF_PI * pp.dw * (fac - 1.0), &sn, &cs);
+    return double2{cs, sn};
 }
 
 // phase constants of phase_correction.cu:92-94 (phase.hip)

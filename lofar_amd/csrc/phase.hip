@@ -11,7 +11,7 @@ namespace lofar {
 // when there is a single plane.  FP64 cubes (the phase_correction() drop-in) evaluate
 // every plane's factor directly; complex-float cubes (the 8192-wide split row passes,
 // where the direct FP64 sincos per pixel and plane would bound the pass) advance it by
-// the FP64 rotation recurrence of the fused row pass (phase_rotation).
+// the FP64 rotation recurrence of the fused row pass (phase_start, phase_step).
 template <typename Real>
 __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::type* cube,
                                                    double* img_re, double* img_im, int xaxis,
@@ -32,8 +32,8 @@ __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::ty
     }
     double sr = 0.0, si = 0.0;
     if constexpr (sizeof(Real) == 4) {
-        double2 z, stp;
-        phase_rotation(pp, fac, z, stp);
+        double2 z = phase_start(pp, fac);
+        const double2 stp = phase_step(pp, fac);
         for (int iw = 0; iw < nw; iw++) {
             const T2 x = cube[(long long)iw * npix + pix];
             const double p = (double)x.x, q = (double)x.y;
@@ -85,8 +85,8 @@ __global__ __launch_bounds__(256) void k_phase_adjoint(const double* img_re, con
     }
     const double a = img_re[pix], b = img_im[pix];
     if constexpr (sizeof(Real) == 4) {
-        double2 z, stp;
-        phase_rotation(pp, fac, z, stp);
+        double2 z = phase_start(pp, fac);
+        const double2 stp = phase_step(pp, fac);
         for (int iw = 0; iw < nw; iw++) {
             // image * conj(z)
             cube[(long long)iw * npix + pix] =
