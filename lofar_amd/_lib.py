@@ -62,6 +62,7 @@ SIGNATURES = {
     "lofar_plan_create": (_i, [_i, _i, _l, _l, _l, _vp, _vp, _vp, _vp, _d, _d, _i, _i, _i, _vp,
                                C.POINTER(_vp)]),
     "lofar_plan_image": (_i, [_vp, _vp, _vp, _vp, _d, _d, _d, _vp, _vp, _vp, _i, _vp]),
+    "lofar_plan_image64": (_i, [_vp, _vp, _vp, _vp, _d, _d, _d, _vp, _vp, _vp, _i, _vp]),
     "lofar_plan_degrid": (_i, [_vp, _d, _d, _d, _vp, _vp, _vp, _vp, _vp, _vp]),
     "lofar_plan_destroy": (_i, [_vp]),
 }

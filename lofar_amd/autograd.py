@@ -19,9 +19,10 @@ real loss L is (Re, Im) of A^H g with g = dL/dm_re + i dL/dm_im.  For the weight
 sum_i w_i |V_i - (A0 x)_i|^2 with the unweighted operator A0, the gradient is -2 times the
 dirty image of the weighted residuals, and ``chi2_descent`` runs gradient descent on it.
 
-The imaging path takes float32 visibilities, as wstack() does (w-stacking.h:12-29).  In FP64
-mode the backward pass therefore splits the float64 cotangent into a float32 high part and a
-float32 remainder and images both (the operator is linear), so the adjoint keeps ~2^-48
+The imaging path takes float32 visibilities, as wstack() does (w-stacking.h:12-29); an FP64
+plan also takes float64 ones (lofar_plan_image64), which is what the backward pass hands it.
+Without a plan, the FP64 backward pass splits the float64 cotangent into a float32 high part
+and a float32 remainder and images both (the operator is linear), so the adjoint keeps ~2^-48
 relative accuracy; the per-sample weight is applied in float64 before the split and the
 imaging calls use unit weights.
 """
@@ -108,6 +109,14 @@ class ImagingOperator:
             # rounded exact product, the same value as rounding the double product below
             return self._image(vis_re.contiguous(), vis_im.contiguous(),
                                self.weight.contiguous())
+        if (self.precision == FP64 and self._use_plan and self.weight.dtype == torch.float32 and
+                vis_re.shape == vis_im.shape == self.weight.shape and
+                vis_re.device == vis_im.device == self.weight.device):
+            # a plan takes the float64 cotangents and the weights as they are
+            f64 = torch.float64
+            return self.plan().image64(vis_re.to(f64).contiguous(), vis_im.to(f64).contiguous(),
+                                       self.weight.contiguous(), self.resolution, self.wmin,
+                                       self.wmax, cube=self.cube)
         w = self.weight.to(torch.float64)
         gr = vis_re.to(torch.float64) * w
         gi = vis_im.to(torch.float64) * w

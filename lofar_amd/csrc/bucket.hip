@@ -959,15 +959,15 @@ hipError_t bucket_sort_grid(int precision, long long n, long long F, long long P
     return level2<kOutFp32>(g, b, (const Rec32*)rec32, (Entry32*)entries, st);
 }
 
-// A plan's entries, with this call's visibilities, in two passes: every sample's
-// channel/polarisation-summed weighted visibility as k_l1_scatter_grid forms it (in the
-// samples' order, coalesced; rounded to float for Entry32, as the entries hold it), then
-// each entry's sample index (left in its real part's slot by the sort) replaced by its
-// sample's sum, one 8- or 16-byte gather per entry.
-template <typename V2>
+// A plan's visibilities: every sample's channel/polarisation-summed weighted visibility as
+// k_l1_scatter_grid forms it, in the samples' order (coalesced; rounded to float for
+// Entry32, as the entries hold it).  The gridder gathers each entry's by the sample index
+// the sort left in its real part's slot; where it takes filled entries only (accumulation
+// variants), k_plan_fill writes them, one 8- or 16-byte gather per entry.
+template <typename V2, typename V>
 __global__ __launch_bounds__(256) void k_plan_vis(long long n, long long F, long long P,
-                                                  const float* vr, const float* vi,
-                                                  const float* wt, V2* vis)
+                                                  const V* vr, const V* vi, const float* wt,
+                                                  V2* vis)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -985,16 +985,7 @@ __global__ __launch_bounds__(256) void k_plan_fill(long long total, const Ent* p
 {
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= total) return;
-    Ent x = pent[e];
-    long long i;
-    if constexpr (sizeof(Ent) == sizeof(Entry64))
-        i = __double_as_longlong(x.vr);
-    else
-        i = (long long)__float_as_uint(x.vr);
-    const V2 v = vis[i];
-    x.vr = v.x;
-    x.vi = v.y;
-    ent[e] = x;
+    ent[e] = entry_at(pent, vis, e);
 }
 
 size_t plan_vis_bytes(int precision, long long n)
@@ -1002,37 +993,35 @@ size_t plan_vis_bytes(int precision, long long n)
     return (size_t)n * (precision == LOFAR_FP64 ? sizeof(double2) : sizeof(float2));
 }
 
-hipError_t plan_vis(int precision, long long n, long long F, long long P, const float* vr,
-                    const float* vi, const float* wt, void* vis, hipStream_t st)
+hipError_t plan_vis(int precision, long long n, long long F, long long P, const void* vr,
+                    const void* vi, bool vis64, const float* wt, void* vis, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
     const dim3 gs(blocks_for(n, 256));
-    if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL((k_plan_vis<double2>), gs, dim3(256), 0, st, n, F, P, vr, vi, wt,
-                           (double2*)vis);
+    if (vis64 && precision != LOFAR_FP64) return hipErrorInvalidValue;
+    if (vis64)
+        hipLaunchKernelGGL((k_plan_vis<double2, double>), gs, dim3(256), 0, st, n, F, P,
+                           (const double*)vr, (const double*)vi, wt, (double2*)vis);
+    else if (precision == LOFAR_FP64)
+        hipLaunchKernelGGL((k_plan_vis<double2, float>), gs, dim3(256), 0, st, n, F, P,
+                           (const float*)vr, (const float*)vi, wt, (double2*)vis);
     else
-        hipLaunchKernelGGL((k_plan_vis<float2>), gs, dim3(256), 0, st, n, F, P, vr, vi, wt,
-                           (float2*)vis);
+        hipLaunchKernelGGL((k_plan_vis<float2, float>), gs, dim3(256), 0, st, n, F, P,
+                           (const float*)vr, (const float*)vi, wt, (float2*)vis);
     return hipGetLastError();
 }
 
-hipError_t plan_fill(int precision, long long n, long long total, const void* pent, void* ent,
-                     long long F, long long P, const float* vr, const float* vi, const float* wt,
-                     void* vis, hipStream_t st)
+hipError_t plan_fill(int precision, long long total, const void* pent, void* ent, const void* vis,
+                     hipStream_t st)
 {
     if (total <= 0) return hipSuccess;
-    const dim3 gs(blocks_for(n, 256)), grid(blocks_for(total, 256));
-    if (precision == LOFAR_FP64) {
-        hipLaunchKernelGGL((k_plan_vis<double2>), gs, dim3(256), 0, st, n, F, P, vr, vi, wt,
-                           (double2*)vis);
+    const dim3 grid(blocks_for(total, 256));
+    if (precision == LOFAR_FP64)
         hipLaunchKernelGGL((k_plan_fill<Entry64, double2>), grid, dim3(256), 0, st, total,
                            (const Entry64*)pent, (Entry64*)ent, (const double2*)vis);
-    } else {
-        hipLaunchKernelGGL((k_plan_vis<float2>), gs, dim3(256), 0, st, n, F, P, vr, vi, wt,
-                           (float2*)vis);
+    else
         hipLaunchKernelGGL((k_plan_fill<Entry32, float2>), grid, dim3(256), 0, st, total,
                            (const Entry32*)pent, (Entry32*)ent, (const float2*)vis);
-    }
     return hipGetLastError();
 }
 

@@ -757,12 +757,14 @@ int validate_direct(DeviceCtx& c, Arena* ar, long n, const double* uu, const dou
 }
 
 // plan: the samples' sort from lofar_plan_create (uu, vv, ww unused): its entries get
-// this call's visibilities, without validation, sorting or host synchronisation.
+// this call's visibilities, without validation, sorting or host synchronisation; vis64: vr
+// and vi are doubles (plans only).
 int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long F, long P,
-              const double* uu, const double* vv, const double* ww, const float* vr,
-              const float* vi, const float* wt, double dx, double dw, int support, int nx, int ny,
+              const double* uu, const double* vv, const double* ww, const void* vr,
+              const void* vi, const float* wt, double dx, double dw, int support, int nx, int ny,
               void* cube, hipStream_t st, unsigned long long* occ = nullptr, int sm_log = -1,
-              Arena* ar = nullptr, const lofar_plan_s* plan = nullptr, long long nocc = 0)
+              Arena* ar = nullptr, const lofar_plan_s* plan = nullptr, long long nocc = 0,
+              bool vis64 = false)
 {
     int r = check_grid_args(precision, nw, n, F, P, dx, dw, support, nx, ny);
     if (r) return fail(r);
@@ -772,8 +774,8 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     if (plan && plan->direct) {
         if (occ || sm_log >= 0) return fail(LOFAR_EARG);
         HIPCHK(stage(c, kStGrid, st, [&] {
-            return grid_direct(precision, n, F, P, plan->uu, plan->vv, plan->ww, vr, vi, wt, g,
-                               cube, accumulate, st);
+            return grid_direct(precision, n, F, P, plan->uu, plan->vv, plan->ww, vr, vi, vis64, wt,
+                               g, cube, accumulate, st);
         }));
         return LOFAR_OK;
     }
@@ -802,7 +804,7 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
             r = dense(vb + vbytes);
             if (r) return r;
             HIPCHK(stage(c, kStScatter, st, [&] {
-                return plan_vis(precision, n, F, P, vr, vi, wt, vb, st);
+                return plan_vis(precision, n, F, P, vr, vi, vis64, wt, vb, st);
             }));
             HIPCHK(stage(c, kStGrid, st, [&] {
                 return grid_tiles(precision, g, b, plan->gent, cube, accumulate, occ, sm_log, st);
@@ -818,8 +820,11 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
         r = dense(eb + ebytes + vbytes);
         if (r) return r;
         HIPCHK(stage(c, kStScatter, st, [&] {
-            return plan_fill(precision, n, plan->gtotal, plan->gent, eb, F, P, vr, vi, wt,
-                             eb + ebytes, st);
+            const hipError_t e =
+                plan_vis(precision, n, F, P, vr, vi, vis64, wt, eb + ebytes, st);
+            return e != hipSuccess
+                       ? e
+                       : plan_fill(precision, plan->gtotal, plan->gent, eb, eb + ebytes, st);
         }));
         HIPCHK(stage(c, kStGrid, st, [&] {
             return grid_tiles(precision, g, b, eb, cube, accumulate, occ, sm_log, st);
@@ -833,8 +838,8 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
         if (r) return r;
         if (occ || sm_log >= 0) return fail(LOFAR_EARG);
         HIPCHK(stage(c, kStGrid, st, [&] {
-            return grid_direct(precision, n, F, P, uu, vv, ww, vr, vi, wt, g, cube, accumulate,
-                               st);
+            return grid_direct(precision, n, F, P, uu, vv, ww, vr, vi, false, wt, g, cube,
+                               accumulate, st);
         }));
         return LOFAR_OK;
     }
@@ -873,7 +878,8 @@ int grid_impl(DeviceCtx& c, int precision, int accumulate, int nw, long n, long 
     }
     b.nent = total;
     HIPCHK(stage(c, kStScatter, st, [&] {
-        return bucket_sort_grid(precision, n, F, P, uu, vv, ww, vr, vi, wt, g, b, rec, ents, st);
+        return bucket_sort_grid(precision, n, F, P, uu, vv, ww, (const float*)vr,
+                                (const float*)vi, wt, g, b, rec, ents, st);
     }));
     HIPCHK(stage(c, kStGrid, st,
                  [&] { return grid_tiles(precision, g, b, ents, cube, accumulate, occ, sm_log, st); }));
@@ -1087,11 +1093,12 @@ int lofar_phase_adjoint_dev(int precision, const double* image_real, const doubl
 // selects where the workspace comes from (nullptr: the context's buffers).
 static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, int num_w_planes,
                       long num_points, long freq_per_chan, long polarizations, const double* uu,
-                      const double* vv, const double* ww, const float* vis_real,
-                      const float* vis_img, const float* weight, double dx, double dw,
+                      const double* vv, const double* ww, const void* vis_real,
+                      const void* vis_img, const float* weight, double dx, double dw,
                       int w_support, int grid_size_x, int grid_size_y, double resolution,
                       double wmin, double wmax, void* cube, double* image_real,
-                      double* image_imag, int accumulate, const lofar_plan_s* plan = nullptr)
+                      double* image_imag, int accumulate, const lofar_plan_s* plan = nullptr,
+                      bool vis64 = false)
 {
     // per-tile occupancy bits: the gridder skips empty tiles and the column pass
     // reads them as zeros (through 32-bit plane offsets, so for planes below 2 GiB;
@@ -1131,7 +1138,7 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
                            : -1;
     r = grid_impl(c, precision, 0, num_w_planes, num_points, freq_per_chan, polarizations, uu, vv,
                   ww, vis_real, vis_img, weight, dx, dw, w_support, grid_size_x, grid_size_y, cube,
-                  st, occ, sm_log, ar, plan, nocc);
+                  st, occ, sm_log, ar, plan, nocc, vis64);
     if (r) return r;
     if (generic) {
         r = fft_generic_planes(c, ar, precision, 1, cube, cube, grid_size_x, grid_size_y,
@@ -1610,19 +1617,38 @@ int lofar_plan_create(int precision, int num_w_planes, long num_points, long fre
     return LOFAR_OK;
 }
 
-int lofar_plan_image(lofar_plan plan, const float* vis_real, const float* vis_img,
-                     const float* weight, double resolution, double wmin, double wmax,
-                     void* cube, double* image_real, double* image_imag, int accumulate,
-                     void* stream)
+static int plan_image_impl(lofar_plan plan, const void* vis_real, const void* vis_img, bool vis64,
+                           const float* weight, double resolution, double wmin, double wmax,
+                           void* cube, double* image_real, double* image_imag, int accumulate,
+                           void* stream)
 {
     if (!plan || !image_real || !image_imag) return fail(LOFAR_EARG);
+    if (vis64 && plan->precision != LOFAR_FP64) return fail(LOFAR_EARG);
     CallGuard cg(stream);
     if (cg.status) return cg.status;
     if (cg.c->device != plan->device) return fail(LOFAR_EARG);
     return image_impl(*cg.c, cg.st, nullptr, plan->precision, plan->nw, plan->n, plan->F,
                       plan->P, nullptr, nullptr, nullptr, vis_real, vis_img, weight, plan->dx,
                       plan->dw, plan->support, plan->nx, plan->ny, resolution, wmin, wmax, cube,
-                      image_real, image_imag, accumulate, plan);
+                      image_real, image_imag, accumulate, plan, vis64);
+}
+
+int lofar_plan_image(lofar_plan plan, const float* vis_real, const float* vis_img,
+                     const float* weight, double resolution, double wmin, double wmax,
+                     void* cube, double* image_real, double* image_imag, int accumulate,
+                     void* stream)
+{
+    return plan_image_impl(plan, vis_real, vis_img, false, weight, resolution, wmin, wmax, cube,
+                           image_real, image_imag, accumulate, stream);
+}
+
+int lofar_plan_image64(lofar_plan plan, const double* vis_real, const double* vis_img,
+                       const float* weight, double resolution, double wmin, double wmax,
+                       void* cube, double* image_real, double* image_imag, int accumulate,
+                       void* stream)
+{
+    return plan_image_impl(plan, vis_real, vis_img, true, weight, resolution, wmin, wmax, cube,
+                           image_real, image_imag, accumulate, stream);
 }
 
 int lofar_plan_degrid(lofar_plan plan, double resolution, double wmin, double wmax,

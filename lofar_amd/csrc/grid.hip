@@ -619,19 +619,6 @@ __device__ __forceinline__ float2 packed_value(unsigned long long t, double inv)
     return float2{(float)((double)re * inv), (float)((double)im * inv)};
 }
 
-// Entry e; with vis (a plan's entries, whose real part's slot holds the sample index),
-// its visibility is the sample's summed visibility in vis.
-__device__ __forceinline__ Entry32 entry_at(const Entry32* entries, const float2* vis, long long e)
-{
-    Entry32 x = entries[e];
-    if (vis) {
-        const float2 v = vis[__float_as_uint(x.vr)];
-        x.vr = v.x;
-        x.vi = v.y;
-    }
-    return x;
-}
-
 // A tile in two passes through one 32 KiB LDS tile (cleared on entry): real parts,
 // stored to the cube's real halves, then imaginary parts; S is the fixed-point
 // scale (FX).
@@ -708,9 +695,9 @@ __device__ __forceinline__ void count_blocks(unsigned* cnt, const Geometry& g, i
 
 // Statistics of one piece into its tile's state (FP64: the block counts too, through cnt in
 // LDS), and its share of clearing the tile's sum words.
-template <int WIN, int NT, bool FP64, typename Ent>
+template <int WIN, int NT, bool FP64, typename Ent, typename V2>
 __device__ __forceinline__ void heavy_stats(const Geometry& g, const TileMap& tm, const Heavy& h,
-                                            long long id, const Ent* entries, const float2* vis,
+                                            long long id, const Ent* entries, const V2* vis,
                                             unsigned* cnt)
 {
     Piece p;
@@ -727,11 +714,7 @@ __device__ __forceinline__ void heavy_stats(const Geometry& g, const TileMap& tm
     double m = 0.0, sa = 0.0;
     bool finite = true;
     for (long long e = p.beg + tid; e < p.end; e += NT) {
-        Ent en;
-        if constexpr (FP64)
-            en = entries[e];
-        else
-            en = entry_at(entries, vis, e);
+        const Ent en = entry_at(entries, vis, e);
         const double vr = fabs((double)en.vr), vi = fabs((double)en.vi);
         finite = finite && isfinite(vr) && isfinite(vi);
         m = fmax(m, fmax(vr, vi));
@@ -1171,7 +1154,8 @@ __device__ __forceinline__ void accumulate_f64(double* acc, const Geometry& g, i
 template <int WIN, int NT>
 __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
                                                          const long long* offsets,
-                                                         const Entry64* entries, double2* cube,
+                                                         const Entry64* entries, const double2* vis,
+                                                         double2* cube,
                                                          unsigned long long* occ, int sm_log,
                                                          Heavy h)
 {
@@ -1183,7 +1167,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     __shared__ double wsum[NT / 64];
     __shared__ int wfin[NT / 64];
     if (blockIdx.x >= tm.nbuckets()) {
-        heavy_stats<WIN, NT, true>(g, tm, h, blockIdx.x - tm.nbuckets(), entries, nullptr,
+        heavy_stats<WIN, NT, true>(g, tm, h, blockIdx.x - tm.nbuckets(), entries, vis,
                                    (unsigned*)acc);
         return;
     }
@@ -1224,7 +1208,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     };
     const long long j0 = slot(0);
     Entry64 en0 = {0.0, 0.0, 0.0, 0.0};
-    if (j0 >= 0) en0 = entries[beg + j0];
+    if (j0 >= 0) en0 = entry_at(entries, vis, beg + j0);
     for (int c = tid; c < kPlane; c += NT)  // 2*kPlane words, 16 bytes a store
         ((ulonglong2*)acc)[c] = ulonglong2{0ull, 0ull};  // also 0.0 as double
     double m = fmax(fabs(en0.vr), fabs(en0.vi));
@@ -1233,7 +1217,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     for (long long q0 = NT; q0 < n; q0 += NT) {
         const long long j = slot(q0);
         if (j >= 0) {
-            const Entry64 en = entries[beg + j];
+            const Entry64 en = entry_at(entries, vis, beg + j);
             finite = finite && isfinite(en.vr) && isfinite(en.vi);
             m = fmax(m, fmax(fabs(en.vr), fabs(en.vi)));
             sa += fabs(en.vr) + fabs(en.vi);
@@ -1265,7 +1249,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
         if (j0 >= 0) accumulate_f64<WIN>(dacc, g, u0, v0, norm, en0);
         for (long long q0 = NT; q0 < n; q0 += NT) {
             const long long j = slot(q0);
-            if (j >= 0) accumulate_f64<WIN>(dacc, g, u0, v0, norm, entries[beg + j]);
+            if (j >= 0) accumulate_f64<WIN>(dacc, g, u0, v0, norm, entry_at(entries, vis, beg + j));
         }
         __syncthreads();
         for (int c = tid; c < kPlane; c += NT) {
@@ -1285,7 +1269,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
     if (j0 >= 0) accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, en0);
     for (long long q0 = NT; q0 < n; q0 += NT) {
         const long long j = slot(q0);
-        if (j >= 0) accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, entries[beg + j]);
+        if (j >= 0) accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, entry_at(entries, vis, beg + j));
     }
     __syncthreads();
     const double inv = ldexp(1.0, -S);
@@ -1299,7 +1283,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
 // One piece of a dense tile (FP64).
 template <int WIN, int NT>
 __global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, const Entry64* entries,
-                                                      double2* cube, int sm_log, Heavy h)
+                                                      const double2* vis, double2* cube, int sm_log, Heavy h)
 {
     constexpr int kPad = ((WIN - 1) * (kTile + 1) + 1) / 2 * 2;  // as k_grid_tiles_fx64
     __shared__ __align__(16) unsigned long long acc[2 * kPlane + kPad];
@@ -1320,7 +1304,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, con
     int S = 0;
     if (flt) {
         for (long long e = p.beg + tid; e < p.end; e += NT)
-            accumulate_f64<WIN>((double*)acc, g, u0, v0, norm, entries[e]);
+            accumulate_f64<WIN>((double*)acc, g, u0, v0, norm, entry_at(entries, vis, e));
     } else {
         for (int b = tid; b < kNBlk * kNBlk; b += NT) atomicMax(&maxcnt, st.blk[b]);
         __syncthreads();
@@ -1331,7 +1315,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, con
         S = kFixedBits64 - hb - ex;
         const double scale = ldexp(1.0, S);
         for (long long e = p.beg + tid; e < p.end; e += NT)
-            accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, entries[e]);
+            accumulate_fx64<WIN>(acc, g, u0, v0, norm, scale, entry_at(entries, vis, e));
     }
     __syncthreads();
     if (!heavy_merge<NT>(h, p, acc, 2 * kPlane, flt, &last)) return;
@@ -1481,11 +1465,11 @@ __global__ __launch_bounds__(256) void k_validate(long long n, const double* uu,
 // One thread per sample adds weight*vis*norm*exp(-(du^2+dv^2)/2) to every cell of its
 // clipped window with global atomic adds, as the reference's OpenMP loop does
 // (w-stacking.cu:222-307, `omp atomic` on each cell); the order of the sums is not fixed.
-template <typename Real>
+template <typename Real, typename V>
 __global__ __launch_bounds__(256) void k_grid_direct(long long n, long long F, long long P,
                                                      const double* uu, const double* vv,
-                                                     const double* ww, const float* vr,
-                                                     const float* vi, const float* wt,
+                                                     const double* ww, const V* vr,
+                                                     const V* vi, const float* wt,
                                                      Geometry g, Real* cube)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1609,10 +1593,11 @@ static void launch_grid_nt(int precision, const Geometry& g, const Buckets& b, c
     constexpr int HT = 512;
     if (precision == LOFAR_FP64 && !accumulate && cfg != 1) {
         hipLaunchKernelGGL((k_grid_tiles_fx64<WIN, NT>), split, dim3(NT), 0, st, g, b.map,
-                           b.offsets, (const Entry64*)entries, (double2*)cube, occ, sm_log, h);
+                           b.offsets, (const Entry64*)entries, (const double2*)b.vis, (double2*)cube, occ,
+                           sm_log, h);
         if (h.max_pieces > 0)
             hipLaunchKernelGGL((k_grid_heavy64<WIN, HT>), pieces, dim3(HT), 0, st, g, b.map,
-                               (const Entry64*)entries, (double2*)cube, sm_log, h);
+                               (const Entry64*)entries, (const double2*)b.vis, (double2*)cube, sm_log, h);
     } else if (precision == LOFAR_FP64)
         hipLaunchKernelGGL((k_grid_tiles<WIN, true, NT>), grid, dim3(NT), 0, st, g, b.map,
                            b.offsets, entries, cube, accumulate, occ, sm_log);
@@ -1672,10 +1657,11 @@ hipError_t validate_samples(long long n, const double* uu, const double* vv, con
 }
 
 hipError_t grid_direct(int precision, long long n, long long F, long long P, const double* uu,
-                       const double* vv, const double* ww, const float* vr, const float* vi,
-                       const float* wt, const Geometry& g, void* cube, int accumulate,
-                       hipStream_t st)
+                       const double* vv, const double* ww, const void* vr, const void* vi,
+                       bool vis64, const float* wt, const Geometry& g, void* cube,
+                       int accumulate, hipStream_t st)
 {
+    if (vis64 && precision != LOFAR_FP64) return hipErrorInvalidValue;
     const long long words = 2LL * g.nw * g.ny * g.nx * (precision == LOFAR_FP64 ? 2 : 1);
     if (!accumulate) {
         hipError_t e = fill_u32((unsigned*)cube, words, 0u, st);
@@ -1683,12 +1669,15 @@ hipError_t grid_direct(int precision, long long n, long long F, long long P, con
     }
     if (n <= 0) return hipGetLastError();
     const dim3 blocks((unsigned)((n + 255) / 256));
-    if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL((k_grid_direct<double>), blocks, dim3(256), 0, st, n, F, P, uu, vv, ww,
-                           vr, vi, wt, g, (double*)cube);
+    if (vis64)
+        hipLaunchKernelGGL((k_grid_direct<double, double>), blocks, dim3(256), 0, st, n, F, P, uu,
+                           vv, ww, (const double*)vr, (const double*)vi, wt, g, (double*)cube);
+    else if (precision == LOFAR_FP64)
+        hipLaunchKernelGGL((k_grid_direct<double, float>), blocks, dim3(256), 0, st, n, F, P, uu,
+                           vv, ww, (const float*)vr, (const float*)vi, wt, g, (double*)cube);
     else
-        hipLaunchKernelGGL((k_grid_direct<float>), blocks, dim3(256), 0, st, n, F, P, uu, vv, ww,
-                           vr, vi, wt, g, (float*)cube);
+        hipLaunchKernelGGL((k_grid_direct<float, float>), blocks, dim3(256), 0, st, n, F, P, uu,
+                           vv, ww, (const float*)vr, (const float*)vi, wt, g, (float*)cube);
     return hipGetLastError();
 }
 
@@ -1714,7 +1703,7 @@ bool grid_splits(int precision, int accumulate)
 
 bool grid_gathers(int precision, int accumulate)
 {
-    return precision != LOFAR_FP64 && !accumulate && grid_cfg() == 0;
+    return grid_splits(precision, accumulate);
 }
 
 hipError_t grid_tiles(int precision, const Geometry& g, const Buckets& b, const void* entries,
@@ -1724,7 +1713,7 @@ hipError_t grid_tiles(int precision, const Geometry& g, const Buckets& b, const 
     // strip-major flushes need whole strips no wider than a tile
     if (sm_log >= 0 && (accumulate || (1 << sm_log) > kTile || g.nx % (1 << sm_log) != 0))
         return hipErrorInvalidValue;
-    // only the packed FP32C kernel gathers visibilities
+    // only the kernels that split dense tiles gather visibilities
     if (b.vis && !grid_gathers(precision, accumulate)) return hipErrorInvalidValue;
     const int win = 2 * g.K + 1;
     if (win <= 5)

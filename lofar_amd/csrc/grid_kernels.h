@@ -46,10 +46,11 @@ __device__ __forceinline__ bool sample_window(double u, double v, double w, cons
 }
 
 // Channel/polarisation sum of one sample with the reference's weighting:
-// float product weight*vis, promoted to double, NaN real parts skipped
-// (w-stacking_omp.c:116-133).
-__device__ __forceinline__ void sample_vis(long long i, long long F, long long P, const float* vr,
-                                           const float* vi, const float* wt, double& sr,
+// product weight*vis in the visibilities' type (float; double for a plan's 64-bit ones),
+// promoted to double, NaN real parts skipped (w-stacking_omp.c:116-133).
+template <typename V>
+__device__ __forceinline__ void sample_vis(long long i, long long F, long long P, const V* vr,
+                                           const V* vi, const float* wt, double& sr,
                                            double& si)
 {
     sr = 0.0;
@@ -58,16 +59,39 @@ __device__ __forceinline__ void sample_vis(long long i, long long F, long long P
     for (long long f = 0; f < F; f++) {
         for (long long p = 0; p < P; p++) {
             const long long ifine = vbase + f * P + p;
-            const float x = vr[ifine];
+            const V x = vr[ifine];
             if (!isnan(x)) {
-                const float w = wt[i * P + p];
-                const float a = w * x;
-                const float b = w * vi[ifine];
+                const V w = (V)wt[i * P + p];
+                const V a = w * x;
+                const V b = w * vi[ifine];
                 sr += (double)a;
                 si += (double)b;
             }
         }
     }
+}
+
+// Entry e; with vis (a plan's entries, whose real part's slot holds the sample index),
+// its visibility is the sample's summed visibility in vis.
+__device__ __forceinline__ Entry32 entry_at(const Entry32* entries, const float2* vis, long long e)
+{
+    Entry32 x = entries[e];
+    if (vis) {
+        const float2 v = vis[__float_as_uint(x.vr)];
+        x.vr = v.x;
+        x.vi = v.y;
+    }
+    return x;
+}
+__device__ __forceinline__ Entry64 entry_at(const Entry64* entries, const double2* vis, long long e)
+{
+    Entry64 x = entries[e];
+    if (vis) {
+        const double2 v = vis[__double_as_longlong(x.vr)];
+        x.vr = v.x;
+        x.vi = v.y;
+    }
+    return x;
 }
 
 // Home cell of a sample for degridding: its truncated position clamped to the grid.
@@ -233,8 +257,8 @@ struct Buckets {
                            // ([nk1] global cursors when global_l1)
     long long* offsets;    // [nbuckets+1] entries of every (w, tile) bucket, bucket order
     long long nent = 0;    // entries in all buckets, when the host knows it (else 0)
-    const void* vis = nullptr;  // index entries: each sample's summed visibility (float2),
-                                // gathered by the gridder (grid_gathers)
+    const void* vis = nullptr;  // index entries: each sample's summed visibility (float2 or
+                                // double2), gathered by the gridder (grid_gathers)
     int* err;              // validation flag (device)
     void* zero;            // err, count1, count1e: nzero words to clear before the count
     long long nzero;
@@ -270,15 +294,14 @@ hipError_t bucket_sort_grid(int precision, long long n, long long F, long long P
                             const double* uu, const double* vv, const double* ww, const float* vr,
                             const float* vi, const float* wt, const Geometry& g, const Buckets& b,
                             Entry64* rec, void* entries, hipStream_t st, bool index_vis = false);
-// total entries of index_vis sorted entries (pent) with this call's visibilities of the n
-// samples, into ent; vis: plan_vis_bytes(precision, n) bytes of scratch
+// each sample's summed visibility into vis (plan_vis_bytes), in the samples' order; vis64: vr
+// and vi are doubles
 size_t plan_vis_bytes(int precision, long long n);
-// each sample's summed visibility into vis (plan_fill's first pass alone)
-hipError_t plan_vis(int precision, long long n, long long F, long long P, const float* vr,
-                    const float* vi, const float* wt, void* vis, hipStream_t st);
-hipError_t plan_fill(int precision, long long n, long long total, const void* pent, void* ent,
-                     long long F, long long P, const float* vr, const float* vi, const float* wt,
-                     void* vis, hipStream_t st);
+hipError_t plan_vis(int precision, long long n, long long F, long long P, const void* vr,
+                    const void* vi, bool vis64, const float* wt, void* vis, hipStream_t st);
+// total entries of index_vis sorted entries (pent) with their samples' visibilities, into ent
+hipError_t plan_fill(int precision, long long total, const void* pent, void* ent, const void* vis,
+                     hipStream_t st);
 // wt1 (one polarisation): the samples' weights, stored in the entries' spare word
 hipError_t bucket_sort_home(long long n, const double* uu, const double* vv, const double* ww,
                             const float* wt1, const Geometry& g, const Buckets& b, DEntry* rec,
@@ -290,7 +313,7 @@ hipError_t bucket_sort_home(long long n, const double* uu, const double* vv, con
 // [nx/L][ny][L] with L = 2^sm_log columns per strip.
 // whether grid_tiles splits dense tiles (b.heavy; the fixed-point kernels do)
 bool grid_splits(int precision, int accumulate);
-// whether grid_tiles takes index entries with b.vis (the packed FP32C kernel)
+// whether grid_tiles takes index entries with b.vis (the fixed-point kernels that split)
 bool grid_gathers(int precision, int accumulate);
 hipError_t grid_tiles(int precision, const Geometry& g, const Buckets& b, const void* entries,
                       void* cube, int accumulate, unsigned long long* occ, int sm_log,
@@ -303,9 +326,9 @@ hipError_t fill_u32(unsigned* p, long long n, unsigned v, hipStream_t st);
 hipError_t validate_samples(long long n, const double* uu, const double* vv, const double* ww,
                             const Geometry& g, int* err, hipStream_t st);
 hipError_t grid_direct(int precision, long long n, long long F, long long P, const double* uu,
-                       const double* vv, const double* ww, const float* vr, const float* vi,
-                       const float* wt, const Geometry& g, void* cube, int accumulate,
-                       hipStream_t st);
+                       const double* vv, const double* ww, const void* vr, const void* vi,
+                       bool vis64, const float* wt, const Geometry& g, void* cube,
+                       int accumulate, hipStream_t st);
 hipError_t degrid_direct(int precision, long long n, long long F, long long P, const double* uu,
                          const double* vv, const double* ww, const float* wt, const Geometry& g,
                          const void* cube, void* model_re, void* model_im, hipStream_t st);

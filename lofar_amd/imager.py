@@ -322,6 +322,20 @@ class Plan:
     def image(self, vis_real, vis_img, weight, resolution, wmin, wmax, cube=None,
               image_real=None, image_imag=None, accumulate=False):
         """``image`` on the planned samples; returns (image_real, image_imag)."""
+        return self._image("lofar_plan_image", _torch().float32, vis_real, vis_img, weight,
+                           resolution, wmin, wmax, cube, image_real, image_imag, accumulate)
+
+    def image64(self, vis_real, vis_img, weight, resolution, wmin, wmax, cube=None,
+                image_real=None, image_imag=None, accumulate=False):
+        """``image`` of float64 visibilities (FP64 plans): weight*vis is formed in float64."""
+        need = self.n * self.F * self.P
+        if vis_real.numel() < need or vis_img.numel() < need:
+            raise ValueError("visibility arrays too short")
+        return self._image("lofar_plan_image64", _torch().float64, vis_real, vis_img, weight,
+                           resolution, wmin, wmax, cube, image_real, image_imag, accumulate)
+
+    def _image(self, name, vt, vis_real, vis_img, weight, resolution, wmin, wmax, cube,
+               image_real, image_imag, accumulate):
         torch = _torch()
         if cube is None:
             cube = torch.empty((self.nw, self.ny, self.nx), dtype=cube_dtype(self.precision),
@@ -331,9 +345,8 @@ class Plan:
             image_real = torch.empty((self.ny, self.nx), dtype=torch.float64, device=self.device)
             image_imag = torch.empty((self.ny, self.nx), dtype=torch.float64, device=self.device)
             accumulate = False
-        check("lofar_plan_image", lib().lofar_plan_image(
-            self._h, _ptr(vis_real, torch.float32, "vis_real"),
-            _ptr(vis_img, torch.float32, "vis_img"), _ptr(weight, torch.float32, "weight"),
+        check(name, getattr(lib(), name)(
+            self._h, _ptr(vis_real, vt, "vis_real"), _ptr(vis_img, vt, "vis_img"), _ptr(weight, torch.float32, "weight"),
             resolution, wmin, wmax, cp, _ptr(image_real, torch.float64, "image_real"),
             _ptr(image_imag, torch.float64, "image_imag"), int(accumulate), _stream()))
         return image_real, image_imag
