@@ -1339,8 +1339,8 @@ __global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, con
 // the gridder) and writes weight*sum for every channel and polarisation.  A dense tile's
 // further pieces (Heavy) are the workgroups beyond the tiles': 3.0M samples of a
 // core-dominated array on 2048x1024x12 took one workgroup 4.9 ms for the core's tile.
-template <int WIN, bool FP64>
-__global__ __launch_bounds__(256) void k_degrid_tiles(Geometry g, TileMap tm, const long long* offsets,
+template <int WIN, bool FP64, int NT>
+__global__ __launch_bounds__(NT) void k_degrid_tiles(Geometry g, TileMap tm, const long long* offsets,
                                                       const DEntry* ents, const void* cube,
                                                       const float* weight, long long F,
                                                       long long P, void* mre, void* mim, Heavy h)
@@ -1373,11 +1373,11 @@ __global__ __launch_bounds__(256) void k_degrid_tiles(Geometry g, TileMap tm, co
     const int tid = threadIdx.x;
     // every load of the thread's part of the region is issued before the first LDS
     // store (a load-store loop keeps one load in flight per thread)
-    constexpr int NLD = (RS * RS + 255) / 256;
+    constexpr int NLD = (RS * RS + NT - 1) / NT;
     T2 xs[NLD];
 #pragma unroll
     for (int k = 0; k < NLD; k++) {
-        const int c = tid + k * 256;
+        const int c = tid + k * NT;
         const int rr = c / RS, cc = c % RS;
         const int gv = v0 - H + rr, gu = u0 - H + cc;
         xs[k] = T2{0, 0};
@@ -1386,12 +1386,12 @@ __global__ __launch_bounds__(256) void k_degrid_tiles(Geometry g, TileMap tm, co
     }
 #pragma unroll
     for (int k = 0; k < NLD; k++) {
-        const int c = tid + k * 256;
+        const int c = tid + k * NT;
         if (c < RS * RS) region[c] = xs[k];
     }
     __syncthreads();
     const double norm = 0.5 / LOFAR_REF_PI;
-    for (long long e = beg + tid; e < end; e += 256) {
+    for (long long e = beg + tid; e < end; e += NT) {
         const DEntry en = ents[e];
         const int gu = (int)en.pu, gv = (int)en.pv;
         const int j0 = (gu > g.K - 1) ? gu - g.K : 0;
@@ -1403,25 +1403,29 @@ __global__ __launch_bounds__(256) void k_degrid_tiles(Geometry g, TileMap tm, co
         // noise-like cubes, and float sums would cost ~1e-6 of the result
         double sr = 0, si = 0;
         if (na >= 0 && nb >= 0) {
-            Real eu[WIN];
+            Real eu[WIN], ev[FP64 ? WIN : 1];
+            if constexpr (FP64) {
+                // two exponentials per axis, as the gridder
+                gauss_row<WIN>((double)j0 + 0.5 - en.pu, eu);
+                gauss_row<WIN>((double)k0 + 0.5 - en.pv, ev);
+            } else {
 #pragma unroll
-            for (int q = 0; q < WIN; q++) {
-                const double du = (double)(j0 + q) + 0.5 - en.pu;
-                if constexpr (FP64)
-                    eu[q] = (q <= na) ? exp(-(du * du) * 0.5) : 0.0;
-                else
+                for (int q = 0; q < WIN; q++) {
+                    const double du = (double)(j0 + q) + 0.5 - en.pu;
                     eu[q] = (q <= na) ? expf(-(float)(du * du) * 0.5f) : 0.0f;
+                }
             }
             const T2* base = &region[(k0 - (v0 - H)) * RS + (j0 - (u0 - H))];
 #pragma unroll
             for (int kq = 0; kq < WIN; kq++) {
                 if (kq <= nb) {
-                    const double dv = (double)(k0 + kq) + 0.5 - en.pv;
                     Real f;
-                    if constexpr (FP64)
-                        f = norm * exp(-(dv * dv) * 0.5);
-                    else
+                    if constexpr (FP64) {
+                        f = norm * ev[kq];
+                    } else {
+                        const double dv = (double)(k0 + kq) + 0.5 - en.pv;
                         f = (float)norm * expf(-(float)(dv * dv) * 0.5f);
+                    }
                     double rr = 0, ri = 0;
                     const T2* row = base + kq * RS;
 #pragma unroll
@@ -1737,11 +1741,16 @@ static void launch_degrid(int precision, const Geometry& g, const Buckets& b, co
                           void* mre, void* mim, hipStream_t st)
 {
     const dim3 grid((unsigned)(b.map.nbuckets() + b.heavy.max_pieces));
+    // complex-double regions (78-102 KiB of LDS) leave one or two workgroups a CU: 1024
+    // threads each.  FP64, 256 / 512 / 1024 threads: 3.0M samples along tracks, S=9, 428 /
+    // 246 / 220 us; 16M on 4096x4096x32, S=7, 2303 / 2394 / 2291.  Complex-float ones (39-51
+    // KiB) keep 256: 16M, S=7, 1.21 ms (512: 1.28).
+    constexpr int NT64 = 1024;
     if (precision == LOFAR_FP64)
-        hipLaunchKernelGGL((k_degrid_tiles<WIN, true>), grid, dim3(256), 0, st, g, b.map,
+        hipLaunchKernelGGL((k_degrid_tiles<WIN, true, NT64>), grid, dim3(NT64), 0, st, g, b.map,
                            b.offsets, ents, cube, weight, F, P, mre, mim, b.heavy);
     else
-        hipLaunchKernelGGL((k_degrid_tiles<WIN, false>), grid, dim3(256), 0, st, g, b.map,
+        hipLaunchKernelGGL((k_degrid_tiles<WIN, false, 256>), grid, dim3(256), 0, st, g, b.map,
                            b.offsets, ents, cube, weight, F, P, mre, mim, b.heavy);
 }
 
