@@ -959,8 +959,18 @@ void report_once(const char* what, int code)
                 lofar_error_string(code));
 }
 
-// strip width (log2 columns) of the fused path's scratch cube; -1 = row-major
-int sm_log_cfg(int precision)
+// Strip width (log2 columns) of the images' scratch cubes; -1: row-major.  A
+// strip is [ny][L], so that the column transforms read and write 32- or 64-byte runs L cells
+// apart instead of a plane row apart.
+//  FP64: 64 columns, the tile width (a tile's row is one run): 32 planes of 4096 x 4096,
+//    columns 4.17 -> 3.42 ms, rows and gridder as row-major.  Strips of 4, which the columns
+//    read in order: 2.95, but rows of 64-byte runs 2.76 for 2.35.
+//  FP32C: 16 columns, a cache line: 32 planes of 4096 x 4096, columns 2.32 -> 2.01 ms, rows
+//    1.16 -> 1.18; 2048 x 2048: 473 -> 422 and 341 -> 351 us.  Strips of 8: 1.84 and 1.30 ms,
+//    408 and 378 us.  64 where the rows run as two passes (8192): 32 planes of 8192 x 8192,
+//    columns 13.7 -> 10.6 ms, rows 7.0 -> 7.7, plane sum 3.6 -> 3.9 (16: 11.0, 7.5, 4.2).
+// LOFAR_SM_LOG overrides, for measurement (-1: row-major; at most the tile width).
+int sm_log_cfg(int precision, bool split)
 {
     static int v = -2;
     if (v == -2) {
@@ -969,7 +979,21 @@ int sm_log_cfg(int precision)
         if (v < -1 || v > 6) v = -3;
     }
     if (v != -3) return v;
-    return precision == LOFAR_FP64 ? 6 : -1;
+    return precision == LOFAR_FP64 || split ? 6 : 4;
+}
+
+// the strips of a power-of-two grid's cube.  The column kernels take whole strips of 4 (FP64)
+// or 8 columns.  Adjoints keep row-major cubes: the row pass's stores and the degridder's
+// loads lose what the columns gain (FP32C 32 planes of 4096 x 4096, 16M samples, columns,
+// rows and interpolation together: row-major 4.80 ms, strips of 16 4.75, of 64 4.83).
+int strip_log(int precision, int nx, int ny)
+{
+    if (!pow2_ok(nx) || !pow2_ok(ny)) return -1;
+    const int sm = sm_log_cfg(precision, nx >= 8192);
+    if (sm < 0 || (1 << sm) > kTile || nx % (1 << sm) != 0 ||
+        (1 << sm) % (precision == LOFAR_FP64 ? 4 : 8) != 0)
+        return -1;
+    return sm;
 }
 
 }  // namespace
@@ -1123,19 +1147,9 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
         if (r) return r;
         occ = (unsigned long long*)op;  // cleared by grid_impl
     }
-    // FP64: the scratch cube is laid out strip-major, in strips of 2^sm_log whole
-    // columns (the 64-column tile width by default), so every tile flush is one
-    // contiguous block and the column transforms read 64-byte runs 1 KiB apart instead
-    // of a plane row apart; FP32C keeps row-major planes (no gain measured there).
-    // LOFAR_SM_LOG overrides, for measurement (-1: row-major; at most the tile width).
-    // rows of 8192 run the split row passes, which read row-major planes
     const bool split = grid_size_x >= 8192;
-    const int sm_pref = (direct || generic || split) ? -1 : sm_log_cfg(precision);
-    const int sm_log = (sm_pref >= 0 && (1 << sm_pref) <= kTile &&
-                        grid_size_x % (1 << sm_pref) == 0 &&
-                        (1 << sm_pref) % (precision == LOFAR_FP64 ? 4 : 8) == 0)
-                           ? sm_pref
-                           : -1;
+    const int sm_log =
+        direct || generic ? -1 : strip_log(precision, grid_size_x, grid_size_y);
     r = grid_impl(c, precision, 0, num_w_planes, num_points, freq_per_chan, polarizations, uu, vv,
                   ww, vis_real, vis_img, weight, dx, dw, w_support, grid_size_x, grid_size_y, cube,
                   st, occ, sm_log, ar, plan, nocc, vis64);
@@ -1173,13 +1187,15 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
         const long long lines = (long long)num_w_planes * grid_size_y;
         HIPCHK(stage(c, kStRows, st, [&] {
             return precision == LOFAR_FP64
-                       ? fft_rows<double>(1, cube, cube, twx, grid_size_x, lines, scale, st)
-                       : fft_rows<float>(1, cube, cube, twx, grid_size_x, lines, scale, st);
+                       ? fft_rows<double>(1, cube, cube, twx, grid_size_x, lines, scale, st,
+                                          grid_size_y, sm_log)
+                       : fft_rows<float>(1, cube, cube, twx, grid_size_x, lines, scale, st,
+                                         grid_size_y, sm_log);
         }));
         HIPCHK(stage(c, kStPhase, st, [&] {
             return phase_sum(precision, cube, image_real, image_imag, grid_size_x, grid_size_y,
                              num_w_planes, grid_size_x, grid_size_y, resolution, wmin, wmax,
-                             accumulate, st);
+                             accumulate, st, sm_log);
         }));
     } else {
         HIPCHK(stage(c, kStRowsPhase, st, [&] {

@@ -48,28 +48,36 @@ __device__ __forceinline__ void store_at(T2 x, __amdgpu_buffer_rsrc_t r, unsigne
 // ---------------------------------------------------------------------------
 // standalone passes
 
-// Row transforms: one line (row) per workgroup.
-template <typename Real, int N, int E, int SIGN>
+// Row transforms: one line (row) per workgroup.  STRIP: rows of strip-major planes
+// ([N/L][ny][L], L = 2^sm_log at most TPL; in and out alike), line l row l%ny of plane l/ny.
+template <typename Real, int N, int E, int SIGN, bool STRIP>
 __global__ __launch_bounds__((Plan<N, E>::TPL)) void k_fft_rows(const C2<Real>* in, C2<Real>* out,
-                                                              const C2<Real>* tw, Real scale)
+                                                              const C2<Real>* tw, Real scale,
+                                                              int ny, int sm_log)
 {
     using T2 = C2<Real>;
     using P = Plan<N, E>;
     __shared__ T2 lds[P::LDS];
     const long long line = blockIdx.x;
-    const T2* src = in + line * N;
-    T2* dst = out + line * N;
     const int t = threadIdx.x;
+    // element t + d of the row, d a multiple of TPL (whole strips): d*per_u from element t
+    const long long base =
+        STRIP ? (line / ny) * ny * N + ((((long long)(t >> sm_log) * ny + line % ny) << sm_log) |
+                                        (t & ((1 << sm_log) - 1)))
+              : line * N + t;
+    const int per_u = STRIP ? ny : 1;
+    const T2* src = in + base;
+    T2* dst = out + base;
     T2 v[P::E];
 #pragma unroll
-    for (int q = 0; q < P::E; q++) v[q] = src[P::in_index(t, q)];
+    for (int q = 0; q < P::E; q++) v[q] = src[P::in_index(0, q) * (long long)per_u];
     stages<T2, N, E, SIGN, 1>(v, lds, 1, t, tw);
 #pragma unroll
     for (int e = 0; e < P::E; e++) {
         T2 x = v[e];
         x.x *= scale;
         x.y *= scale;
-        dst[P::out_index(t, e)] = x;
+        dst[P::out_index(0, e) * (long long)per_u] = x;
     }
 }
 
@@ -221,8 +229,8 @@ __device__ __forceinline__ double pixel_fac(const PhaseParams& pp, int iu, doubl
 // Row prefetch for k_rows_phase: row iv of plane psrc goes straight into
 // pbuf[0, N) with 16-byte direct-to-LDS loads (global_load_lds_dwordx4); wave
 // instruction c of the row writes 1 KiB, elements [c*K, (c+1)*K) with K = 1024 /
-// sizeof(T2) (one run of a row-major row, or of one strip of a strip-major plane
-// when its strips are at least K elements wide).
+// sizeof(T2): one run of a row-major row, or a run of each of K/L strips of a strip-major
+// plane (every lane has an address of its own).
 template <typename T2, int N, int TPL>
 __device__ __forceinline__ void prefetch_row(const T2* psrc, T2* pbuf, int t, int iv, int ny,
                                              int sm_log)
@@ -233,17 +241,21 @@ __device__ __forceinline__ void prefetch_row(const T2* psrc, T2* pbuf, int t, in
     static_assert(NWAVE >= 1 && N % K == 0, "whole waves, whole 1 KiB runs");
     const int lane = t & 63, wave = t >> 6;
     constexpr int ITER = (N / K + NWAVE - 1) / NWAVE;
-    // wave-uniform run start (scalar registers) plus a per-lane offset
+    // wave-uniform part (scalar registers) plus a per-lane offset: with L <= K columns a
+    // strip, element u + k of a wave's K is in strip u/L + k/L
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const T2* lane_src = psrc + lane * PER;
+    const int k = lane * PER;
+    const T2* lane_src =
+        psrc + (sm_log < 0 ? (long long)iv * N + k
+                           : ((((long long)(k >> sm_log) * ny + iv) << sm_log) |
+                              (k & ((1 << sm_log) - 1))));
+    const long long per_u = sm_log < 0 ? 1 : ny;
 #pragma unroll
     for (int i = 0; i < ITER; i++) {
         const int c = wave_u + i * NWAVE;
         if (c >= N / K) break;
-        const int u = c * K;  // the run never crosses a strip: strips are >= K wide
-        const long long o = sm_log < 0 ? (long long)iv * N + u
-                                        : ((((long long)(u >> sm_log) * ny + iv) << sm_log) |
-                                           (u & ((1 << sm_log) - 1)));
+        const int u = c * K;
+        const long long o = u * per_u;
         __builtin_amdgcn_global_load_lds((const void*)(lane_src + o),
                                          (__attribute__((address_space(3))) void*)(pbuf + u), 16,
                                          0, 0);
@@ -299,7 +311,8 @@ __global__ __launch_bounds__((G * Plan<N, E>::TPL), (kRowPair<Real, N> ? 4 : 1))
     // PF: plane iw-1's row is loaded into pbuf while plane iw is transformed
     __shared__ __align__(16) T2 pbuf[PF ? N : 1];
     __shared__ double2 sums[G > 1 ? (G - 1) * N : 1];
-    const int iv = blockIdx.x;
+    // rows of one XCD are adjacent (strips may be narrower than a cache line of its L2)
+    const int iv = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int grp = G > 1 ? threadIdx.x / P::TPL : 0;
     const int t = G > 1 ? threadIdx.x % P::TPL : threadIdx.x;
     T2* lds = lds_all + grp * P::LDS;
@@ -460,17 +473,20 @@ static int col_cfg()
 
 template <typename Real, int N>
 static hipError_t launch_rows_n(int sign, const void* in, void* out, const void* tw,
-                                long long lines, double scale, hipStream_t st)
+                                long long lines, double scale, hipStream_t st, int ny, int sm_log)
 {
     using T2 = C2<Real>;
     constexpr int TPL = Plan<N, kRowE>::TPL;
     if (lines <= 0) return hipSuccess;
-    if (sign > 0)
-        hipLaunchKernelGGL((k_fft_rows<Real, N, kRowE, 1>), dim3((unsigned)lines), dim3(TPL), 0,
-                           st, (const T2*)in, (T2*)out, (const T2*)tw, (Real)scale);
-    else
-        hipLaunchKernelGGL((k_fft_rows<Real, N, kRowE, -1>), dim3((unsigned)lines), dim3(TPL), 0,
-                           st, (const T2*)in, (T2*)out, (const T2*)tw, (Real)scale);
+    auto k = sign > 0 ? k_fft_rows<Real, N, kRowE, 1, false> : k_fft_rows<Real, N, kRowE, -1, false>;
+    if (sm_log >= 0) {
+        // the images' two-pass rows; shorter rows of strips run in the fused pass
+        if (N <= 4096 || sign < 0 || (1 << sm_log) > TPL || ny < 1 || lines % ny)
+            return hipErrorInvalidValue;
+        if constexpr (N > 4096) k = k_fft_rows<Real, N, kRowE, 1, true>;
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)lines), dim3(TPL), 0, st, (const T2*)in, (T2*)out,
+                       (const T2*)tw, (Real)scale, ny, sm_log);
     return hipGetLastError();
 }
 
@@ -542,7 +558,7 @@ static int row_groups(int tpl, int ny, int nw)
 }
 
 // the fused row pass: 8 elements per thread, the next row prefetched into LDS where it fits
-// and planes hold whole 1 KiB runs (row-major rows, or strips at least that wide)
+// and strips are of whole 16-byte loads and no wider than a wave's 1 KiB
 template <typename Real, int N>
 static hipError_t launch_rows_phase_n(const void* cube, const void* tw, int ny, int nw,
                                       const PhaseParams& pp, double scale, double* re, double* im,
@@ -561,8 +577,10 @@ static hipError_t launch_rows_phase_n(const void* cube, const void* tw, int ny, 
             return hipGetLastError();
         }
     }
-    auto k = fits && (sm_log < 0 || (1 << sm_log) >= K) ? k_rows_phase<Real, N, E, fits, 1>
-                                                        : k_rows_phase<Real, N, E, false, 1>;
+    constexpr int PER = 16 / (int)sizeof(T2);
+    auto k = fits && (sm_log < 0 || ((1 << sm_log) >= PER && (1 << sm_log) <= K))
+                 ? k_rows_phase<Real, N, E, fits, 1>
+                 : k_rows_phase<Real, N, E, false, 1>;
     hipLaunchKernelGGL(k, dim3(ny), dim3(TPL), 0, st, (const T2*)cube, (const T2*)tw, ny, nw, pp,
                        scale, re, im, accumulate, sm_log);
     return hipGetLastError();
@@ -609,9 +627,9 @@ static hipError_t launch_rows_phase_adj_n(void* cube, const void* tw, int ny, in
 
 template <typename Real>
 hipError_t fft_rows(int sign, const void* in, void* out, const void* tw, int nx, long long lines,
-                    double scale, hipStream_t st)
+                    double scale, hipStream_t st, int ny, int sm_log)
 {
-#define CALL_(n) launch_rows_n<Real, n>(sign, in, out, tw, lines, scale, st)
+#define CALL_(n) launch_rows_n<Real, n>(sign, in, out, tw, lines, scale, st, ny, sm_log)
     LOFAR_FFT_SWITCH(nx, CALL_)
 #undef CALL_
 }
@@ -659,9 +677,9 @@ int device_cus()
 }
 
 template hipError_t fft_rows<double>(int, const void*, void*, const void*, int, long long, double,
-                                     hipStream_t);
+                                     hipStream_t, int, int);
 template hipError_t fft_rows<float>(int, const void*, void*, const void*, int, long long, double,
-                                    hipStream_t);
+                                    hipStream_t, int, int);
 template hipError_t fft_cols<double>(int, const void*, void*, const void*, int, int, int, double,
                                      hipStream_t, const unsigned long long*, int);
 template hipError_t fft_cols<float>(int, const void*, void*, const void*, int, int, int, double,

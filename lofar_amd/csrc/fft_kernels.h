@@ -605,8 +605,9 @@ hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int 
 // host dispatch (fft.hip); all return hipErrorInvalidValue for unsupported sizes.  tw: the
 // line length's table with rx 16 (fft_rows, fft_cols) or 8 (rows_phase, rows_phase_adj).
 template <typename Real>
+// sm_log >= 0: strip-major planes of ny rows of 8192, strips of 2^sm_log columns, in and out
 hipError_t fft_rows(int sign, const void* in, void* out, const void* tw, int nx, long long lines,
-                    double scale, hipStream_t st);
+                    double scale, hipStream_t st, int ny = 0, int sm_log = -1);
 template <typename Real>
 // occ (optional): for forward transforms (sign +1), per-tile occupancy bits from
 // grid_tiles, rows of empty tiles read as zeros; for inverse transforms (sign -1),

@@ -341,9 +341,10 @@ hipError_t need_tiles(const Geometry& g, const Buckets& b, unsigned long long* n
 hipError_t degrid_tiles(int precision, const Geometry& g, const Buckets& b, const DEntry* entries,
                         const void* cube, const float* weight, long long F, long long P,
                         void* model_re, void* model_im, hipStream_t st);
+// sm_log >= 0: the planes are strip-major, [xaxis/L][yaxis][L] with L = 2^sm_log
 hipError_t phase_sum(int precision, const void* cube, double* re, double* im, int xaxis, int yaxis,
                      int nw, int xtot, int ytot, double resolution, double wmin, double wmax,
-                     int accumulate, hipStream_t st);
+                     int accumulate, hipStream_t st, int sm_log = -1);
 hipError_t phase_adjoint(int precision, const double* re, const double* im, void* cube, int xaxis,
                          int yaxis, int nw, int xtot, int ytot, double resolution, double wmin,
                          double wmax, hipStream_t st);

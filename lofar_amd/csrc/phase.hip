@@ -16,13 +16,21 @@ template <typename Real>
 __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::type* cube,
                                                    double* img_re, double* img_im, int xaxis,
                                                    int yaxis, int nw, PhaseParams pp,
-                                                   int accumulate)
+                                                   int accumulate, int sm_log)
 {
     using T2 = typename cplx<Real>::type;
     const long long npix = (long long)xaxis * yaxis;
-    const long long pix = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pix >= npix) return;
-    const int iu = (int)(pix % xaxis), iv = (int)(pix / xaxis);
+    // consecutive threads on consecutive cells of a plane: row-major, or strip-major
+    // ([xaxis/L][yaxis][L], L = 2^sm_log)
+    const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell >= npix) return;
+    int iu = (int)(cell % xaxis), iv = (int)(cell / xaxis);
+    if (sm_log >= 0) {
+        const long long s = cell >> sm_log;
+        iv = (int)(s % yaxis);
+        iu = (int)(s / yaxis << sm_log) | (int)(cell & ((1 << sm_log) - 1));
+    }
+    const long long pix = (long long)iv * xaxis + iu;
     double fac = 1.0;
     if (pp.phase_on) {
         const double xcoord = pp.coord(iu, pp.xtot);
@@ -35,7 +43,7 @@ __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::ty
         double2 z = phase_start(pp, fac);
         const double2 stp = phase_step(pp, fac);
         for (int iw = 0; iw < nw; iw++) {
-            const T2 x = cube[(long long)iw * npix + pix];
+            const T2 x = cube[(long long)iw * npix + cell];
             const double p = (double)x.x, q = (double)x.y;
             sr = fma(p, z.x, fma(-q, z.y, sr));
             si = fma(p, z.y, fma(q, z.x, si));
@@ -43,7 +51,7 @@ __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::ty
         }
     } else
     for (int iw = 0; iw < nw; iw++) {
-        const T2 x = cube[(long long)iw * npix + pix];
+        const T2 x = cube[(long long)iw * npix + cell];
         const double p = (double)x.x, q = (double)x.y;
         if (pp.phase_on) {
             const double wterm = pp.wmin + iw * pp.dw;
@@ -124,7 +132,7 @@ static PhaseParams make_pp(int nw, int xtot, int ytot, double resolution, double
 
 hipError_t phase_sum(int precision, const void* cube, double* re, double* im, int xaxis, int yaxis,
                      int nw, int xtot, int ytot, double resolution, double wmin, double wmax,
-                     int accumulate, hipStream_t st)
+                     int accumulate, hipStream_t st, int sm_log)
 {
     const PhaseParams pp = make_pp(nw, xtot, ytot, resolution, wmin, wmax);
     const long long npix = (long long)xaxis * yaxis;
@@ -132,10 +140,11 @@ hipError_t phase_sum(int precision, const void* cube, double* re, double* im, in
     if (npix == 0) return hipSuccess;
     if (precision == LOFAR_FP64)
         hipLaunchKernelGGL(k_phase_sum<double>, dim3(blocks), dim3(256), 0, st,
-                           (const double2*)cube, re, im, xaxis, yaxis, nw, pp, accumulate);
+                           (const double2*)cube, re, im, xaxis, yaxis, nw, pp, accumulate,
+                           sm_log);
     else
         hipLaunchKernelGGL(k_phase_sum<float>, dim3(blocks), dim3(256), 0, st, (const float2*)cube,
-                           re, im, xaxis, yaxis, nw, pp, accumulate);
+                           re, im, xaxis, yaxis, nw, pp, accumulate, sm_log);
     return hipGetLastError();
 }
 
