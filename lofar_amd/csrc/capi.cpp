@@ -470,8 +470,9 @@ bool pow2_ok(int n) { return n >= 2 && n <= 8192 && (n & (n - 1)) == 0; }
 // (with `col_scale`), then rows (with `row_scale`); out may alias in.
 int fft_generic_planes(DeviceCtx& c, Arena* ar, int precision, int sign, const void* in,
                        void* out, int nx, int ny, int nw, double row_scale, hipStream_t st,
-                       bool rows_first = false)
+                       bool rows_first = false, int sm_log = -1)
 {
+    const long long plane = (long long)nx * ny, L = sm_log >= 0 ? 1LL << sm_log : nx;
     void *twx, *twy;
     int r = twiddles_for(c, ar, nx, precision, 0, st, &twx);
     if (r) return r;
@@ -479,20 +480,20 @@ int fft_generic_planes(DeviceCtx& c, Arena* ar, int precision, int sign, const v
     if (r) return r;
     auto cols = [&](const void* src) {
         return precision == LOFAR_FP64
-                   ? fft_generic<double>(sign, src, out, twy, ny, (long long)nw * nx, nx,
-                                         (long long)nx * ny, 1, nx, rows_first ? row_scale : 1.0,
-                                         st)
-                   : fft_generic<float>(sign, src, out, twy, ny, (long long)nw * nx, nx,
-                                        (long long)nx * ny, 1, nx, rows_first ? row_scale : 1.0,
-                                        st);
+                   ? fft_generic<double>(sign, src, out, twy, ny, (long long)nw * nx, L, L * ny, 1,
+                                         L, rows_first ? row_scale : 1.0, st)
+                   : fft_generic<float>(sign, src, out, twy, ny, (long long)nw * nx, L, L * ny, 1,
+                                        L, rows_first ? row_scale : 1.0, st);
     };
     auto rows = [&](const void* src) {
         const long long lines = (long long)nw * ny;
+        const int sm = sm_log >= 0 ? sm_log : 30;
+        const long long strip = sm_log >= 0 ? L * ny : 0;
         return precision == LOFAR_FP64
-                   ? fft_generic<double>(sign, src, out, twx, nx, lines, lines, 0, nx, 1,
-                                         rows_first ? 1.0 : row_scale, st)
-                   : fft_generic<float>(sign, src, out, twx, nx, lines, lines, 0, nx, 1,
-                                        rows_first ? 1.0 : row_scale, st);
+                   ? fft_generic<double>(sign, src, out, twx, nx, lines, ny, plane, L, 1,
+                                         rows_first ? 1.0 : row_scale, st, sm, strip)
+                   : fft_generic<float>(sign, src, out, twx, nx, lines, ny, plane, L, 1,
+                                        rows_first ? 1.0 : row_scale, st, sm, strip);
     };
     if (rows_first) {
         HIPCHK(stage(c, kStRows, st, [&] { return rows(in); }));
@@ -988,7 +989,11 @@ int sm_log_cfg(int precision, bool split)
 // rows and interpolation together: row-major 4.80 ms, strips of 16 4.75, of 64 4.83).
 int strip_log(int precision, int nx, int ny)
 {
-    if (!pow2_ok(nx) || !pow2_ok(ny)) return -1;
+    if (!pow2_ok(nx) || !pow2_ok(ny)) {
+        // mixed-radix sides, row-major where nx leaves a remainder
+        const int m = precision == LOFAR_FP64 ? 2 : 3;
+        return nx % (1 << m) == 0 ? m : -1;
+    }
     const int sm = sm_log_cfg(precision, nx >= 8192);
     if (sm < 0 || (1 << sm) > kTile || nx % (1 << sm) != 0 ||
         (1 << sm) % (precision == LOFAR_FP64 ? 4 : 8) != 0)
@@ -1149,19 +1154,20 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
     }
     const bool split = grid_size_x >= 8192;
     const int sm_log =
-        direct || generic ? -1 : strip_log(precision, grid_size_x, grid_size_y);
+        direct ? -1 : strip_log(precision, grid_size_x, grid_size_y);
     r = grid_impl(c, precision, 0, num_w_planes, num_points, freq_per_chan, polarizations, uu, vv,
                   ww, vis_real, vis_img, weight, dx, dw, w_support, grid_size_x, grid_size_y, cube,
                   st, occ, sm_log, ar, plan, nocc, vis64);
     if (r) return r;
     if (generic) {
         r = fft_generic_planes(c, ar, precision, 1, cube, cube, grid_size_x, grid_size_y,
-                               num_w_planes, 1.0 / ((double)grid_size_x * grid_size_y), st);
+                               num_w_planes, 1.0 / ((double)grid_size_x * grid_size_y), st, false,
+                               sm_log);
         if (r) return r;
         HIPCHK(stage(c, kStPhase, st, [&] {
             return phase_sum(precision, cube, image_real, image_imag, grid_size_x, grid_size_y,
                              num_w_planes, grid_size_x, grid_size_y, resolution, wmin, wmax,
-                             accumulate, st);
+                             accumulate, st, sm_log);
         }));
         return LOFAR_OK;
     }

@@ -600,7 +600,7 @@ bool fft_size_ok(int n);
 template <typename Real>
 hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int n, long long lines,
                        long long per, long long plane, long long lstride, long long estride,
-                       double scale, hipStream_t st);
+                       double scale, hipStream_t st, int sm = 30, long long strip = 0);
 
 // host dispatch (fft.hip); all return hipErrorInvalidValue for unsupported sizes.  tw: the
 // line length's table with rx 16 (fft_rows, fft_cols) or 8 (rows_phase, rows_phase_adj).

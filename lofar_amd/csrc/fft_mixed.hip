@@ -212,11 +212,12 @@ constexpr int kMixElems = 128 / (2 * (int)sizeof(Real)) * 2;
 // butterflies of radix p per thread, at most
 __host__ __device__ constexpr int mix_nb(int elems, int p) { return elems / p > 1 ? elems / p : 1; }
 
-// Lines of a launch: line l starts at (l / per) * plane + (l % per) * lstride and its
-// elements are estride apart.
+// Lines of a launch: line l starts at (l / per) * plane + (l % per) * lstride.  Element e is at
+// e * estride of a column and at (e >> sm) * strip + e % 2^sm of a row: strips of 2^sm columns,
+// strip cells apart (one strip for row-major planes: sm = 30, strip 0).
 struct MixLines {
     long long count, per, plane, lstride;
-    int estride;
+    int estride, sm, strip;
     int llog;     // 2^llog lines per workgroup
     int swap;     // inverse sign: parts swapped on the way in and out
 };
@@ -232,12 +233,16 @@ struct MixThread {
     T2* out;
     T2* buf;
     const T2* tw;
-    int n, r0, l, j0, tpl, llog, estride;
+    int n, r0, l, j0, tpl, llog, estride, sm, strip;
     bool active, swap;
     Real scale;
     __device__ __forceinline__ int slot(int e) const
     {
         return mix_pad(ROWS ? l * n + e : (e << llog) + l);
+    }
+    __device__ __forceinline__ long long at(int e) const
+    {
+        return ROWS ? (e >> sm) * strip + (e & ((1 << sm) - 1)) : (long long)e * estride;
     }
 };
 
@@ -248,7 +253,7 @@ __device__ __forceinline__ void mix_read(const MixThread<Real, ROWS>& m, int j, 
 #pragma unroll
     for (int q = 0; q < P; q++) {
         if constexpr (FIRST) {
-            const T2 x = m.in[(long long)(j + q * nb) * m.estride];
+            const T2 x = m.in[m.at(j + q * nb)];
             a[q] = m.swap ? T2{x.y, x.x} : x;
         } else {
             a[q] = m.buf[m.slot(j + q * nb)];
@@ -277,7 +282,7 @@ __device__ __forceinline__ void mix_butterfly(const MixThread<Real, ROWS>& m, co
             T2 x = a[r];
             x.x *= m.scale;
             x.y *= m.scale;
-            m.out[(long long)(base + r * ns) * m.estride] = m.swap ? T2{x.y, x.x} : x;
+            m.out[m.at(base + r * ns)] = m.swap ? T2{x.y, x.x} : x;
         } else {
             m.buf[m.slot(base + r * ns)] = a[r];
         }
@@ -374,6 +379,8 @@ __global__ __launch_bounds__(kMixMaxT) void k_fft_mixed(const typename cplx<Real
     m.buf = (T2*)mix_lds;
     m.tw = tw;
     m.estride = ln.estride;
+    m.sm = ln.sm;
+    m.strip = ln.strip;
     m.swap = ln.swap != 0;
     m.scale = scale;
     const int last = plan.nstages - 1;
@@ -500,7 +507,7 @@ bool fft_size_ok(int n)
 template <typename Real>
 hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int n, long long lines,
                        long long per, long long plane, long long lstride, long long estride,
-                       double scale, hipStream_t st)
+                       double scale, hipStream_t st, int sm, long long strip)
 {
     using T2 = typename cplx<Real>::type;
     MixPlan p;
@@ -537,6 +544,8 @@ hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int 
     ln.plane = plane;
     ln.lstride = lstride;
     ln.estride = (int)estride;
+    ln.sm = sm;
+    ln.strip = (int)strip;
     ln.llog = llog;
     ln.swap = sign < 0;
     const long long blocks = (lines + (1LL << llog) - 1) >> llog;
@@ -550,9 +559,9 @@ hipError_t fft_generic(int sign, const void* in, void* out, const void* tw, int 
 
 template hipError_t fft_generic<double>(int, const void*, void*, const void*, int, long long,
                                         long long, long long, long long, long long, double,
-                                        hipStream_t);
+                                        hipStream_t, int, long long);
 template hipError_t fft_generic<float>(int, const void*, void*, const void*, int, long long,
                                        long long, long long, long long, long long, double,
-                                       hipStream_t);
+                                       hipStream_t, int, long long);
 
 }  // namespace lofar

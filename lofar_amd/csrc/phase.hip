@@ -20,17 +20,25 @@ __global__ __launch_bounds__(256) void k_phase_sum(const typename cplx<Real>::ty
 {
     using T2 = typename cplx<Real>::type;
     const long long npix = (long long)xaxis * yaxis;
-    // consecutive threads on consecutive cells of a plane: row-major, or strip-major
-    // ([xaxis/L][yaxis][L], L = 2^sm_log)
-    const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= npix) return;
-    int iu = (int)(cell % xaxis), iv = (int)(cell / xaxis);
-    if (sm_log >= 0) {
-        const long long s = cell >> sm_log;
-        iv = (int)(s % yaxis);
-        iu = (int)(s / yaxis << sm_log) | (int)(cell & ((1 << sm_log) - 1));
+    int iu, iv;
+    long long pix, cell;
+    if (sm_log < 0) {
+        pix = cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+        if (pix >= npix) return;
+        iu = (int)(pix % xaxis);
+        iv = (int)(pix / xaxis);
+    } else {
+        // strip-major planes ([xaxis/L][yaxis][L], L = 2^sm_log up to 64): a workgroup takes 4
+        // rows of 64 columns, so that it reads runs of 4 L cells (of 4 complex doubles: 16
+        // planes of 3000 x 3000 take 572 us in cell order, which stores 32-byte runs)
+        const int nrow = (yaxis + 3) / 4, t = threadIdx.x;
+        iv = (int)(blockIdx.x % nrow) * 4 + ((t >> sm_log) & 3);
+        iu = (int)(blockIdx.x / nrow) * 64 + ((t >> (sm_log + 2)) << sm_log) +
+             (t & ((1 << sm_log) - 1));
+        if (iu >= xaxis || iv >= yaxis) return;
+        pix = (long long)iv * xaxis + iu;
+        cell = (((long long)(iu >> sm_log) * yaxis + iv) << sm_log) | (iu & ((1 << sm_log) - 1));
     }
-    const long long pix = (long long)iv * xaxis + iu;
     double fac = 1.0;
     if (pp.phase_on) {
         const double xcoord = pp.coord(iu, pp.xtot);
@@ -136,8 +144,10 @@ hipError_t phase_sum(int precision, const void* cube, double* re, double* im, in
 {
     const PhaseParams pp = make_pp(nw, xtot, ytot, resolution, wmin, wmax);
     const long long npix = (long long)xaxis * yaxis;
-    const unsigned blocks = (unsigned)((npix + 255) / 256);
     if (npix == 0) return hipSuccess;
+    if (sm_log > 6 || (sm_log >= 0 && xaxis % (1 << sm_log))) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)(sm_log < 0 ? (npix + 255) / 256
+                                                  : (long long)((yaxis + 3) / 4) * ((xaxis + 63) / 64));
     if (precision == LOFAR_FP64)
         hipLaunchKernelGGL(k_phase_sum<double>, dim3(blocks), dim3(256), 0, st,
                            (const double2*)cube, re, im, xaxis, yaxis, nw, pp, accumulate,

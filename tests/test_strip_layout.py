@@ -1,7 +1,7 @@
 """Images go through strip-major scratch cubes; the separate passes keep row-major ones.  The
 image against grid, fft and phase of the same samples, at one strip, less than one (row-major),
-strips shorter and longer than a row pass's loads, rows of 8192 (two passes), few rows and row
-counts that no XCD share divides.  Both sides are the same sums: FP64 agrees to rounding
+strips shorter and longer than a row pass's loads, rows of 8192 (two passes), few rows, row
+counts that no XCD share divides, and mixed-radix sides with and without strips.  Both sides are the same sums: FP64 agrees to rounding
 (1e-12), FP32C to two FP32 transforms' (2e-6); a misplaced cell is an error of order one."""
 import numpy as np
 import pytest
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nx,ny,nw", [(8, 64, 3), (16, 16, 2), (32, 8, 5), (64, 512, 4),
                                       (128, 2, 3), (512, 64, 3), (1024, 4, 6), (2048, 128, 2),
                                       (4096, 64, 3), (16, 8192, 2), (8192, 2, 3),
-                                      (8192, 64, 2)])
+                                      (8192, 64, 2), (12, 25, 3), (100, 7, 2), (300, 480, 3),
+                                      (1250, 60, 2), (64, 90, 3), (1000, 2, 2), (3000, 66, 2)])
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32c", 2e-6)])
 def test_image_equals_the_separate_passes(cuda, nx, ny, nw, precision, tol):
     import torch
