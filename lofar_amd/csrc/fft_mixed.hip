@@ -187,21 +187,55 @@ __device__ __forceinline__ void dft_pair(T2* v)
     }
 }
 
+// DFT over A*B, A and B coprime (Good's mapping): x[B*n1 + A*n2 mod AB] as an A x B array has
+// no factors between its two DFTs, and output k is element (k mod A, k mod B).  Against
+// dft_pair it rounds less: transforms of 3000 x 3000 complex floats 1.97e-7 -> 1.84e-7 from 64
+// bits, of 1000 x 1000 1.85e-7 -> 1.63e-7.
+template <int A, int B, typename T2>
+__device__ __forceinline__ void dft_coprime(T2* v)
+{
+    T2 m[A * B];
+#pragma unroll
+    for (int n2 = 0; n2 < B; n2++) {
+        T2 a[A];
+#pragma unroll
+        for (int n1 = 0; n1 < A; n1++) a[n1] = v[(B * n1 + A * n2) % (A * B)];
+        dft_mixed<A>(a);
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) m[k1 * B + n2] = a[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; k1++) dft_mixed<B>(&m[k1 * B]);
+#pragma unroll
+    for (int k = 0; k < A * B; k++) v[k] = m[(k % A) * B + k % B];
+}
+
+// complex doubles keep dft_pair: with dft_coprime the column kernel's 1024-thread register
+// allocation comes out worse (16 planes of 3000 columns of 3000, 1.43 -> 1.56 ms)
+template <int A, int B, typename T2>
+__device__ __forceinline__ void dft_product(T2* v)
+{
+    if constexpr (sizeof(T2) == 16)
+        dft_pair<A, B>(v);
+    else
+        dft_coprime<A, B>(v);
+}
+
 template <int P, typename T2>
 __device__ __forceinline__ void dft_mixed(T2* v)
 {
     if constexpr (P == 2 || P == 4 || P == 8 || P == 16)
         dft<P, 1>(v);
     else if constexpr (P == 6)
-        dft_pair<2, 3>(v);
+        dft_product<2, 3>(v);
     else if constexpr (P == 9)
         dft_pair<3, 3>(v);
     else if constexpr (P == 10)
-        dft_pair<2, 5>(v);
+        dft_product<2, 5>(v);
     else if constexpr (P == 12)
-        dft_pair<4, 3>(v);
+        dft_product<4, 3>(v);
     else if constexpr (P == 15)
-        dft_pair<3, 5>(v);
+        dft_product<3, 5>(v);
     else
         dft_odd<P>(v);
 }
