@@ -983,14 +983,16 @@ int sm_log_cfg(int precision, bool split)
     return precision == LOFAR_FP64 || split ? 6 : 4;
 }
 
-// the strips of a power-of-two grid's cube.  The column kernels take whole strips of 4 (FP64)
+// The strips of an image's cube.  The power-of-two column kernels take whole strips of 4 (FP64)
 // or 8 columns.  Adjoints keep row-major cubes: the row pass's stores and the degridder's
 // loads lose what the columns gain (FP32C 32 planes of 4096 x 4096, 16M samples, columns,
 // rows and interpolation together: row-major 4.80 ms, strips of 16 4.75, of 64 4.83).
 int strip_log(int precision, int nx, int ny)
 {
     if (!pow2_ok(nx) || !pow2_ok(ny)) {
-        // mixed-radix sides, row-major where nx leaves a remainder
+        // mixed-radix sides: strips of 64 bytes, row-major where nx leaves a remainder (3000 x
+        // 3000 x 16, columns, rows and plane sum together: FP64 3.55 -> 3.28 ms, FP32C 1.90 ->
+        // 1.82)
         const int m = precision == LOFAR_FP64 ? 2 : 3;
         return nx % (1 << m) == 0 ? m : -1;
     }
@@ -1141,7 +1143,7 @@ static int image_impl(DeviceCtx& c, hipStream_t st, Arena* ar, int precision, in
     // row-major cube
     const bool direct = w_support >= 1 && 2 * ((w_support - 1) / 2) + 1 > kMaxTileWin;
     // sides that are not powers of two: the mixed-radix transforms and the standalone
-    // phase sum over a whole row-major cube
+    // phase sum over a whole cube
     const bool generic = !pow2_ok(grid_size_x) || !pow2_ok(grid_size_y);
     if (plane_bytes < (1LL << 31) && !direct && !generic) {
         const long long ntv = (grid_size_y + kTile - 1) / kTile;

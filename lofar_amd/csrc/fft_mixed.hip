@@ -18,9 +18,11 @@
 //
 // Bound: the load - stages - store sequence of the one or two workgroups a CU holds; rows
 // are near the copy rate, columns longer than 2048 complex doubles get runs of only 32
-// bytes (a strip of 64-byte runs does not fit LDS).  16 planes of 3000 x 3000 complex
-// doubles: columns 1.98 ms, rows 1.18 ms (2.3 and 3.9 TB/s); one line per 256-thread
-// workgroup with 128 KiB of LDS and radices 8, 3, 5, 5, 5 took 12.5 ms for both.
+// bytes (64-byte runs do not fit LDS).  16 planes of 3000 x 3000 complex doubles, row-major:
+// columns 1.92 ms, rows 1.15 ms (2.4 and 4.0 TB/s); in strips of 4 columns ([nx/4][ny][4], the
+// images' cubes: strip_log in capi.cpp) 1.42 and 1.36, of 2 1.20 and 1.77, of 8 1.77 and 1.24.
+// One line per 256-thread workgroup with 128 KiB of LDS and radices 8, 3, 5, 5, 5 took 12.5 ms
+// for both.
 #include <algorithm>
 
 #include "fft_kernels.h"
