@@ -235,7 +235,9 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
         clear_heavy<1024>(h, hslot, hn);
         return;
     }
-    // block descriptors, one thread each: its segment is the last that starts at or before it
+    // block descriptors, one thread each: its segment is the last that starts at or before it.
+    // off1[nk1] is not read: no barrier stands between its store above and here, and every
+    // thread holds the total (crec).
     for (long long j = tid; j < cblk; j += 1024) {
         long long lo = 0, hi = nk1;  // boff[lo] <= j < boff[hi]
         while (hi - lo > 1) {
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(1024) void k_l1_scan(long long nk1, const unsigned*
         L2Block d;
         d.k1 = lo;
         d.beg = off1[lo] + (j - boff[lo]) * bs;
-        d.end = min(off1[lo + 1], d.beg + bs);
+        d.end = min(lo + 1 < nk1 ? off1[lo + 1] : crec, d.beg + bs);
         d.pad = 0;
         blk[j] = d;
     }
