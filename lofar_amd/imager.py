@@ -329,8 +329,9 @@ class Plan:
                 image_real=None, image_imag=None, accumulate=False):
         """``image`` of float64 visibilities (FP64 plans): weight*vis is formed in float64."""
         need = self.n * self.F * self.P
-        if vis_real.numel() < need or vis_img.numel() < need:
-            raise ValueError("visibility arrays too short")
+        if (vis_real.numel() < need or vis_img.numel() < need or
+                weight.numel() < self.n * self.P):
+            raise ValueError("visibility or weight arrays too short")
         return self._image("lofar_plan_image64", _torch().float64, vis_real, vis_img, weight,
                            resolution, wmin, wmax, cube, image_real, image_imag, accumulate)
 
