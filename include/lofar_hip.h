@@ -191,8 +191,8 @@ int lofar_plan_image(lofar_plan plan, const float* vis_real, const float* vis_im
                      void* cube, double* image_real, double* image_imag, int accumulate,
                      void* stream);
 /* lofar_plan_image of double visibilities (FP64 plans, LOFAR_EARG for others): the product
- * weight*vis is formed in double.  The adjoint of lofar_plan_degrid's double model in one
- * pass. */
+ * weight*vis is formed in double, and a visibility whose product's real part is NaN is
+ * skipped.  The adjoint of lofar_plan_degrid's double model in one pass. */
 int lofar_plan_image64(lofar_plan plan, const double* vis_real, const double* vis_img,
                        const float* weight, double resolution, double wmin, double wmax,
                        void* cube, double* image_real, double* image_imag, int accumulate,

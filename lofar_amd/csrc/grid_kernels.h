@@ -47,7 +47,9 @@ __device__ __forceinline__ bool sample_window(double u, double v, double w, cons
 
 // Channel/polarisation sum of one sample with the reference's weighting:
 // product weight*vis in the visibilities' type (float; double for a plan's 64-bit ones),
-// promoted to double, NaN real parts skipped (w-stacking_omp.c:116-133).
+// promoted to double, NaN real parts skipped (w-stacking_omp.c:116-133).  Of 64-bit ones NaN
+// products are (0 times infinity and NaN weights too): they are the products that an adjoint
+// without a plan forms and splits into float visibilities.
 template <typename V>
 __device__ __forceinline__ void sample_vis(long long i, long long F, long long P, const V* vr,
                                            const V* vi, const float* wt, double& sr,
@@ -60,9 +62,9 @@ __device__ __forceinline__ void sample_vis(long long i, long long F, long long P
         for (long long p = 0; p < P; p++) {
             const long long ifine = vbase + f * P + p;
             const V x = vr[ifine];
-            if (!isnan(x)) {
-                const V w = (V)wt[i * P + p];
-                const V a = w * x;
+            const V w = (V)wt[i * P + p];
+            const V a = w * x;
+            if (!isnan(sizeof(V) == 8 ? a : x)) {
                 const V b = w * vi[ifine];
                 sr += (double)a;
                 si += (double)b;

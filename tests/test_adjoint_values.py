@@ -1,0 +1,36 @@
+"""FP64 adjoints of unusual float64 cotangents: the planned call (one pass over doubles) against
+the unplanned one (two passes over float parts) where products are NaN, in tiles summed by one
+workgroup and by several."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def samples(cuda, n, seed):
+    import torch
+    rng = np.random.default_rng(seed)
+    return [torch.from_numpy(a).to(cuda) for a in (
+        rng.uniform(0.2, 0.8, n), rng.uniform(0.2, 0.8, n), rng.uniform(0, 0.999, n),
+        rng.standard_normal(n), rng.standard_normal(n))]
+
+
+@pytest.mark.parametrize("support", [7, 21])
+@pytest.mark.parametrize("n", [300, 20000])
+def test_nan_products_are_skipped(cuda, n, support):
+    """A visibility whose weighted real part is NaN (NaN weight, or 0 times infinity) adds
+    nothing, with a plan and without: both sum 53-bit products, 1e-12 relative L2."""
+    import torch
+    from lofar_amd import autograd
+    u, v, w, vr, vi = samples(cuda, n, n)
+    wt = 0.5 + torch.rand(n, device=cuda)
+    wt[::7] = float("nan")
+    wt[1::7] = 0.0
+    vr[1::14] = float("inf")
+    out = []
+    for plan in (False, True):
+        op = autograd.ImagingOperator(u, v, w, wt, 2, support, 64, 64, 1.0 / 128, -40.0, 60.0,
+                                      plan=plan)
+        out.append(torch.complex(*op.adjoint(vr, vi)))
+    assert torch.isfinite(torch.view_as_real(out[0])).all()
+    assert torch.linalg.norm(out[1] - out[0]) <= 1e-12 * torch.linalg.norm(out[0])
