@@ -1025,6 +1025,10 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_pk(Geometry g, TileMap tm, co
 // Gaussian factors come from gauss_row (two exponentials per axis).
 constexpr int kFixedBits64 = 62;
 
+// Tiles whose largest component is below 2^-960 (double visibilities can be) are summed in
+// floating point: from there on 2^S and its inverse leave the normal doubles (S reaches 1023).
+__device__ __forceinline__ bool below_fixed64(double m) { return m > 0.0 && m < 0x1p-960; }
+
 // round(a*b) (nearest, ties to even, of the exact product) as a two's-complement
 // 64-bit value, |a*b| < 2^62, in three full-rate double operations and one 64-bit
 // shift-add:
@@ -1239,7 +1243,7 @@ __global__ __launch_bounds__(NT) void k_grid_tiles_fx64(Geometry g, TileMap tm,
         all_finite = all_finite && wfin[i] != 0;
     }
     // a bright outlier (largest |vis| far above the tile's mean): floating-point path
-    if (!all_finite || m > kHdrRatio * (sa - m) / (double)(2 * n - 1)) {
+    if (!all_finite || m > kHdrRatio * (sa - m) / (double)(2 * n - 1) || below_fixed64(m)) {
         double* dacc = (double*)acc;
         if (j0 >= 0) accumulate_f64<WIN>(dacc, g, u0, v0, norm, en0);
         for (long long q0 = NT; q0 < n; q0 += NT) {
@@ -1295,7 +1299,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy64(Geometry g, TileMap tm, con
     for (int c = tid; c < kPlane; c += NT)  // 2*kPlane words, 16 bytes a store
         ((ulonglong2*)acc)[c] = ulonglong2{0ull, 0ull};
     __syncthreads();
-    const bool flt = heavy_float(st, n);
+    const bool flt = heavy_float(st, n) || below_fixed64(m);
     int S = 0;
     if (flt) {
         for (long long e = p.beg + tid; e < p.end; e += NT)
