@@ -90,3 +90,49 @@ def test_image_and_plan(cuda, n, support, precision):
     a = imager.degrid(sky, sky, *t[:3], t[5], nw, support, *args, precision=precision)
     b = plan.degrid(sky, sky, *args)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("kind", ["spread", "point", "outlier", "inf"])
+@pytest.mark.parametrize("nx,ny,nw", [(1100, 1000, 2), (1024, 1024, 3)])
+def test_two_level_sort(cuda, nx, ny, nw, kind):
+    """More than 512 tiles, so two levels sort them: the dense tile among sparse ones, its
+    super-tile's records in more level-2 blocks than one read of the scan takes (70000 in
+    blocks of 1024).  Grid, degridding, image and plan as above, with the same tolerances."""
+    import torch
+    from lofar_amd import imager
+    n, sparse = 70000, 5000
+    rng = np.random.default_rng(nx)
+    back = (rng.uniform(0, 0.999, sparse), rng.uniform(0, 0.999, sparse) * ny / nx,
+            rng.uniform(0, 0.999, sparse), rng.standard_normal(sparse).astype(np.float32),
+            rng.standard_normal(sparse).astype(np.float32),
+            rng.uniform(0.5, 1.5, sparse).astype(np.float32))
+    d = [np.concatenate(x) for x in zip(case(n, nx, ny, nw, kind), back)]
+    st, want = O.wstack(nw, *d, 1 / nx, 1 / nw, 7, nx, ny)
+    assert st == O.OK
+    cube = rng.standard_normal((nw, ny, nx)) + 0j
+    st, ref = O.degrid(cube, *d[:3], d[5], 1 / nx, 1 / nw, 7)
+    assert st == O.OK
+    t = [torch.from_numpy(a).to(cuda) for a in d]
+    perm = torch.from_numpy(np.random.default_rng(1).permutation(len(d[0]))).to(cuda)
+    mr, mi = imager.degrid_cube(torch.from_numpy(cube).to(cuda), *t[:3], t[5], 7)
+    close(mr.cpu().numpy() + 1j * mi.cpu().numpy(), ref, 1e-12)
+    args = (1.0 / 2200, -40.0, 60.0)
+    sky = torch.randn((ny, nx), dtype=torch.float64, device=cuda)
+    for precision, tol in (("fp64", 1e-12), ("fp32c", 1e-6)):
+        got = imager.grid(*t, nw, 7, nx, ny, precision=precision)
+        close(got.cpu().numpy(), want, tol)
+        plan = imager.Plan(*t[:3], t[5], nw, 7, nx, ny, precision=precision)
+        a = imager.degrid(sky, sky, *t[:3], t[5], nw, 7, *args, precision=precision)
+        b = plan.degrid(sky, sky, *args)
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+        if kind in ("outlier", "inf"):
+            continue  # floating sums: no fixed order, and no finite image of an infinity
+        again = imager.grid(*[x[perm].contiguous() for x in t], nw, 7, nx, ny,
+                            precision=precision)
+        assert torch.equal(torch.view_as_real(got), torch.view_as_real(again))
+        re, im = imager.image(*t, nw, 7, nx, ny, *args, precision=precision)
+        pre, pim = plan.image(*t[3:], *args)
+        assert torch.equal(re, pre) and torch.equal(im, pim)
+        img = O.image(nw, *d, 7, nx, ny, *args)
+        close(re.cpu().numpy() + 1j * im.cpu().numpy(), img,
+              1e-10 if precision == "fp64" else 1e-6)
