@@ -36,6 +36,13 @@ def test_grid_and_degrid(cuda, n, nx, ny, nw):
     assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("n", [1, 511, 513, 1025, 262144, 262145, 524289])
+def test_grid_and_degrid_two_levels(cuda, n):
+    """576 tiles, more than one level sorts: the level-2 blocks' rule as well (1024 records up
+    to 524288 samples, more beyond), with the tolerances above."""
+    test_grid_and_degrid(cuda, n, 1500, 1500, 1)
+
+
 CHILD = r"""
 import hashlib, sys
 import numpy as np, torch
