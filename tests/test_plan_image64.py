@@ -53,3 +53,11 @@ def test_refuses_other_plans_and_types(cuda):
         plan.image64(v64.float(), v64.float(), wt, *args)
     with pytest.raises(ValueError):
         plan.image64(v64[:50].contiguous(), v64, wt, *args)
+
+
+@pytest.mark.parametrize("n,nx,ny,nw,support,F,P", [(60000, 128, 256, 4, 9, 1, 1),
+                                                    (20000, 64, 64, 1, 7, 2, 2)])
+def test_dense_tiles_match_the_float_parts(cuda, n, nx, ny, nw, support, F, P):
+    """The same with more than 4096 entries in several tiles, or in the only one: tiles that
+    several workgroups sum."""
+    test_matches_the_float_parts(cuda, n, nx, ny, nw, support, F, P)
