@@ -131,13 +131,14 @@ def cpu_baseline(work, names):
 LDS_ATOMIC_PEAK_G = 16 * 256 * 2.4
 
 
-def lds_atomics(n, support, prof):
-    """Secondary bound of the gridder: 64-bit LDS atomic adds it needs (re and im of every
-    cell a sample's window covers, 2*S^2 per sample) per second of grid_tiles time."""
+def lds_atomics(n, support, prof, per_cell=2):
+    """Secondary bound of the gridder: 64-bit LDS atomic adds it needs (per_cell for every cell
+    a sample's window covers: re and im in FP64 mode, one word of both in FP32C mode) per
+    second of grid_tiles time."""
     if "grid_tiles" not in prof:
         return None
     ms = prof["grid_tiles"][0] / max(prof["grid_tiles"][1], 1)
-    ops = 2 * support * support * n
+    ops = per_cell * support * support * n
     g = ops / (ms * 1e-3) / 1e9
     return {"kernel": "grid_tiles", "algorithmic_atomics": ops, "avg_launch_ms": ms,
             "achieved": g, "peak": LDS_ATOMIC_PEAK_G, "unit": "G 64-bit LDS atomics/s",
@@ -177,7 +178,7 @@ def bench_fp32c(dev, a, fp64_value, work, names, nx=4096, nw=32, support=7):
            "speedup_vs_fp64_mode": (mvis32 / fp64_value) if fp64_value else None,
            "end_to_end_algorithmic_GBs": kb["total"] / (ms32 * 1e-3) / 1e9,
            "stages_ms": {k: round(v[0], 4) for k, v in prof32.items()},
-           "gridder_lds_atomics": lds_atomics(n3, support, prof32)}
+           "gridder_lds_atomics": lds_atomics(n3, support, prof32, per_cell=1)}
     print("bench: fp32c %.3f ms/step %.1f Mvis/s" % (ms32, mvis32), file=sys.stderr, flush=True)
     if work is not None:
         save_workload(work, "fp32c", d3, nx, nw, support, re32, im32)
