@@ -1,8 +1,9 @@
 // C-ABI layer of liblofar_hip: per-device context, workspace, twiddle tables,
 // the reference drop-ins (wstack, phase_correction, test) and the device entry
 // points.  Host pointers only cross PCIe in the drop-ins; the lofar_*_dev entry
-// points enqueue on the caller's stream and never synchronise except to read
-// back the sample-validation flag and the bucket total (16 bytes) per gridding.
+// points enqueue on the caller's stream and never wait for it except for the
+// sample-validation flag and the bucket total, which the sort writes to pinned
+// host memory, once per unplanned gridding or degridding.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -169,7 +170,7 @@ struct DeviceCtx {
     char* stage_buf[kStage] = {};
     hipEvent_t stage_done[kStage] = {};
     Buffer occ;                     // per-tile occupancy of the fused imaging path
-    volatile long long* status_host = nullptr;  // pinned: [total, err, call number]
+    volatile long long* status_host = nullptr;  // pinned: [total, err, call number, largest]
     long long status_seq = 0;       // call number of the last bucket count
     char* scratch = nullptr;        // this device's copy of `scratch` (allocation-free calls)
     hipError_t scratch_err = hipSuccess;

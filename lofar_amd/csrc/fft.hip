@@ -263,8 +263,10 @@ __device__ __forceinline__ void prefetch_row(const T2* psrc, T2* pbuf, int t, in
 }
 
 // The fused row passes of complex floats from 2048 on are compiled for two workgroups of
-// 4096 a CU (128 VGPRs, 72 KiB of LDS), which overlap each other's loads, exchanges and
-// arithmetic: the last stage's twiddles in registers, the others' in LDS.  Shorter rows have
+// 4096 a CU (capped at 128 VGPRs, 72 KiB of LDS), which overlap each other's loads, exchanges
+// and arithmetic: the last stage's twiddles in registers, the others' in LDS.  The cap costs
+// spilled registers, 8 at 4096, 14 at 2048 and 20 in the adjoint, and is a gain with them
+// (32 planes of 4096 x 4096: 1.50 -> 1.17 ms).  Shorter rows have
 // several workgroups a CU either way, and complex doubles (172-256 VGPRs) one: theirs are
 // all in registers, since LDS is what bounds them (1024 rows of 1024 complex doubles and 8
 // planes: 48 us, 73 with the early stages' twiddles in LDS).

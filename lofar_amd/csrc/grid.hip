@@ -7,8 +7,9 @@
 // values and for accumulate mode), then writes the tile to HBM once with plain
 // coalesced stores.
 // A sample whose window straddles tiles is listed in each of them with the
-// window clipped to that tile, so no two workgroups write the same cell and no
-// global atomics or zero-fill pass are needed.  The (w-plane, tile) buckets
+// window clipped to that tile, so no two tiles share a cell and no zero-fill pass
+// is needed; only the workgroups that share a dense tile (Heavy) meet in global
+// atomics, on sum words beside the cube.  The (w-plane, tile) buckets
 // come from the two-level counting sort in bucket.hip; a bucket index that
 // names a tile beyond the grid (a partial super-tile) ends its workgroup at once.
 #include <algorithm>
@@ -516,7 +517,8 @@ __device__ __forceinline__ void add_block_bound(unsigned long long* bsum, const 
 
 // Windows up to this side take all their columns in accumulate_pk32 (the others mask the
 // clipped ones: at 17 cells a quarter of the adds would be of zeros), and the words past a
-// tile that they reach.
+// tile that they reach.  The masked kernels (13 and 17 cells) index their row of factors at run
+// time and keep it in scratch, 96 bytes a lane.
 constexpr int kPkWhole = 9;
 constexpr int kPkPad = kPkWhole - 1;
 
@@ -650,7 +652,9 @@ __device__ __forceinline__ void grid_halves(unsigned long long* acc, const Geome
 // dense tiles (Heavy): their pieces' workgroups first collect the tile's largest component,
 // sum and finiteness (in the tile kernels' launch), then accumulate with the scale that
 // follows from them; the pieces' integer sums meet in the tile's sum words with global
-// atomics, and the last piece stores the tile.  The sums are those of one workgroup bit for
+// atomics, and the last piece stores the tile.  Tiles summed in floating point (heavy_float)
+// are split as well, and their pieces' doubles meet the same way, in no fixed order.  The
+// integer sums are those of one workgroup bit for
 // bit in FP32C mode; in FP64 mode the scale follows the entries touching the densest 4x4
 // block instead of all of the tile's, so the quantum is finer.  A core-dominated array's
 // 1.05M x 8 visibilities on 2048x2048x16: the FP64 gridder 1.45 -> 0.3 ms, the image 2.79
@@ -735,7 +739,9 @@ __device__ __forceinline__ void heavy_stats(const Geometry& g, const TileMap& tm
 }
 
 // Whether the tile is summed in floating point (a non-finite value, or a bright outlier), as
-// the tile kernels decide it.
+// the tile kernels decide it.  Here as there sa is a double sum in the entries' order, which
+// the sort's atomics make: a tile whose outlier is within that sum's rounding of the limit may
+// be summed either way.
 __device__ __forceinline__ bool heavy_float(const HeavyState& st, long long n)
 {
     const double m = __longlong_as_double((long long)st.m);

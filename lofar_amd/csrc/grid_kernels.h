@@ -264,7 +264,8 @@ struct Buckets {
     int* err;              // validation flag (device)
     void* zero;            // err, count1, count1e: nzero words to clear before the count
     long long nzero;
-    volatile long long* status;  // host memory: entry total, validation flag, call number
+    volatile long long* status;  // host memory: entry total, validation flag, call number,
+                                 // entries of the fullest tile (one level)
     Heavy heavy;                 // dense tiles, listed by the sort
     // level 2
     long long l2_block;       // records per level-2 block
