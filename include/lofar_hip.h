@@ -176,7 +176,9 @@ int lofar_degrid_dev(int precision, int num_w_planes, long num_points, long freq
  * arrays may change or be freed afterwards.  lofar_plan_image and
  * lofar_plan_degrid then run lofar_image_dev and lofar_degrid_dev on the planned
  * samples without sorting and without host synchronisation: the same results, bit
- * for bit.  The degridding weights are those given to lofar_plan_create; the
+ * for bit (images to rounding where tiles hold non-finite values or bright outliers,
+ * or windows are wider than 17 cells: those sum doubles in no fixed order).  The
+ * degridding weights are those given to lofar_plan_create; the
  * imaging weights come with each call.  Windows wider than 17 cells keep copies of
  * uu, vv, ww and take the unsorted paths.  A plan belongs to the device current at
  * its creation (LOFAR_EARG elsewhere).  FP32C plans keep sample indices in 32 bits:
